@@ -152,7 +152,7 @@ int build_lists(gn_batch_s *b)
         gn_plan_s *p = b->m[i];
         const Geometry &g = p->geo;
         const SpreadArgs sa = make_spread_args(p, nullptr, 0);
-        const int ncg = p->nc >= 8 ? 8 : p->nc >= 4 ? 4 : p->nc >= 2 ? 2 : 1;
+        const int ncg = spread_coil_group(p->nc);
         int waves = 0, nbg = 0;
         spread_shape(sa, g.dim, &waves, &nbg);
         const bool mfma = spread_uses_mfma(sa, g.dim);

@@ -2374,14 +2374,12 @@ hipError_t spread_dispatch(const SpreadArgs &a, int nitems, int nritems, const i
                            hipStream_t st)
 {
     hipError_t e;
-    if (nc >= 8)
-        e = spread_launch<D, 8>(a, nitems, nc, st);
-    else if (nc >= 4)
-        e = spread_launch<D, 4>(a, nitems, nc, st);
-    else if (nc >= 2)
-        e = spread_launch<D, 2>(a, nitems, nc, st);
-    else
-        e = spread_launch<D, 1>(a, nitems, nc, st);
+    switch (spread_coil_group(nc)) {
+    case 8: e = spread_launch<D, 8>(a, nitems, nc, st); break;
+    case 4: e = spread_launch<D, 4>(a, nitems, nc, st); break;
+    case 2: e = spread_launch<D, 2>(a, nitems, nc, st); break;
+    default: e = spread_launch<D, 1>(a, nitems, nc, st); break;
+    }
     if (e == hipSuccess && nritems > 0) {
         hipLaunchKernelGGL(k_spread_reduce<D>, dim3((unsigned)nritems), dim3(kReduceThreads), 0, st, a, ritems);
         e = hipGetLastError();
