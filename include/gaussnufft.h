@@ -204,12 +204,15 @@ int gn_plan_destroy(gn_plan *plan);
  * backward = ifftshift(IFFT(fftshift(ksp))), shifts over the transformed axes).
  * mask: null or float32 of prod(shape) entries (broadcast over the batch, mask_batch
  * = 1) or prod(shape) * batch entries (mask_batch = batch); it multiplies the output.
- * in and out may be the same buffer.  Host-synchronous on `stream` (the shifted copy
- * uses one workspace per device): calls from several threads are serialized. */
+ * in and out may be the same buffer.  Host-synchronous on `stream`; with GN_FFT_ASYNC the
+ * call returns once its kernels are queued on `stream`, except for lengths the library's
+ * own passes do not cover (see gn_fft.hip: fft_length_supported), whose workspace is
+ * shared by the calls on a device.  Calls from several threads are serialized. */
 #define GN_FFT_FORWARD 1
 #define GN_FFT_INVERSE -1
 #define GN_FFT_SHIFT_IN 1  /* fftshift the input over the transformed axes  */
 #define GN_FFT_SHIFT_OUT 2 /* ifftshift the output over the transformed axes */
+#define GN_FFT_ASYNC 4     /* do not wait for the queued kernels */
 int gn_fft_c2c(int rank, const int64_t *shape, int64_t batch, int direction, int flags, const float *mask,
                int64_t mask_batch, const void *in, void *out, void *stream);
 

@@ -21,7 +21,7 @@ GN_TYPE1, GN_TYPE2, GN_ADJOINT, GN_TYPE21 = 1, 2, 3, 21
 GN_SENSE_TYPE2, GN_SENSE_TYPE1, GN_SENSE_ADJOINT, GN_SENSE_TYPE21 = 32, 31, 33, 321
 GN_GRID_SPREAD, GN_GRID_GATHER = 41, 42
 GN_FFT_AUTO, GN_FFT_ROCFFT = 0, 1
-GN_FFT_FORWARD, GN_FFT_INVERSE, GN_FFT_SHIFT_IN, GN_FFT_SHIFT_OUT = 1, -1, 1, 2
+GN_FFT_FORWARD, GN_FFT_INVERSE, GN_FFT_SHIFT_IN, GN_FFT_SHIFT_OUT, GN_FFT_ASYNC = 1, -1, 1, 2, 4
 STAGES = ("pad", "fft2", "gather", "spread", "fft1", "crop")
 GN_F32, GN_C64, GN_C128 = 1, 2, 3
 GN_TV_AMP_SQUARE, GN_TV_AMP_MODULUS = 0, 1

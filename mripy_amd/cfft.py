@@ -8,7 +8,7 @@
   (pics/operators_cuda_class.py:7-58): forward = ifftshift(FFT(fftshift(im))) * mask,
   backward = ifftshift(IFFT(fftshift(ksp))), shifts over ``axes``.  When the shift
   axes are the transformed axes (the default) the shifts and the mask run inside
-  ``gn_fft_c2c``'s passes before and after rocFFT; otherwise the shifts are separate
+  ``gn_fft_c2c``'s passes; otherwise the shifts are separate
   device rolls.
 
 numpy inputs give numpy outputs (complex64, host-synchronous like the reference);
@@ -22,7 +22,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import GN_FFT_FORWARD, GN_FFT_INVERSE, GN_FFT_SHIFT_IN, GN_FFT_SHIFT_OUT, check
+from ._lib import GN_FFT_ASYNC, GN_FFT_FORWARD, GN_FFT_INVERSE, GN_FFT_SHIFT_IN, GN_FFT_SHIFT_OUT, check
 
 
 def _dev(x):
@@ -47,9 +47,14 @@ def _c2c(x, rank, direction, flags=0, mask=None):
     shp = (ctypes.c_int64 * 3)(*(list(lead) + [1] * (3 - rank)))
     if t.numel():
         with torch.cuda.device(dev):
-            stream = torch.cuda.current_stream(dev).cuda_stream
-            check(_lib.load().gn_fft_c2c(rank, shp, batch, direction, flags, m.data_ptr() if m is not None else None,
-                                         mb, t.data_ptr(), out.data_ptr(), ctypes.c_void_p(stream)))
+            stream = torch.cuda.current_stream(dev)
+            # the call only queues its kernels: inputs allocated on another stream stay
+            # reserved until this one has read them
+            for r in (t,) if m is None else (t, m):
+                r.record_stream(stream)
+            check(_lib.load().gn_fft_c2c(rank, shp, batch, direction, flags | GN_FFT_ASYNC,
+                                         m.data_ptr() if m is not None else None, mb, t.data_ptr(), out.data_ptr(),
+                                         ctypes.c_void_p(stream.cuda_stream)))
     return out.cpu().numpy() if is_np else out
 
 

@@ -1,8 +1,13 @@
 // Cartesian complex-to-complex FFTs over the leading axes of a C-order array whose
 // trailing dimensions are a batch (coils), interleaved element by element -- the
 // layout of the reference's cuFFT wrappers -- with the centring shifts and the
-// k-space mask of the masked Cartesian operators fused into one pass before and one
-// pass after rocFFT.
+// k-space mask of the masked Cartesian operators fused.
+//
+// Lengths the in-LDS transform covers take one kernel pass per axis (k_fft_axis): the
+// shifts are index offsets of its loads and stores, the mask and the scale multiply the
+// last pass's stores, and the passes run from the input into the output and then in
+// place, with no workspace.  Other lengths, and an output that partly overlaps the
+// input, use rocFFT between a pass before and a pass after it.
 //
 //   forward: out = [ifftshift] ( FFT( [fftshift] in ) ) * mask       (unnormalized)
 //   inverse: out = [ifftshift] ( IFFT( [fftshift] in ) ) / prod(shape)
@@ -17,6 +22,7 @@
 #include <tuple>
 #include <vector>
 
+#include "gn_fft_device.h"
 #include "gn_internal.h"
 
 namespace gn {
@@ -76,6 +82,211 @@ __global__ __launch_bounds__(256) void k_shift_copy(ShiftArgs a, const float2 *_
         }
         dst[e] = v;
     }
+}
+
+// ---------------------------------------------------------------------------
+// One axis of the transform.  The array is (slabs, L, ncols) with ncols contiguous
+// (the trailing axes and the batch); a block takes S slabs x C columns (C = ncols when
+// S > 1, so that its elements are one contiguous run) as S * C lines in LDS.  Input row
+// n enters at FFT position n + in_off, output row n is FFT index n + out_off (mod L).
+// Bound by memory: each pass reads and writes the array once.  512-thread blocks of 16
+// lines (128-byte row segments), fewer lines while the launch has fewer than two blocks
+// per CU.  Measured at 256 x 256 x 32 (16.8 MB), masked forward then inverse through the
+// operator: 47 us, against 147 us for shift pass, rocFFT, shift pass and a wait per call.
+// ---------------------------------------------------------------------------
+constexpr int kAxisThreads = 512;
+constexpr int kAxisLines = 16;
+constexpr int kAxisUnroll = 4;                // global loads in flight per thread
+constexpr int64_t kAxisBlocks = 512;          // two blocks per CU
+constexpr size_t kAxisLdsMax = 64 * 1024;
+
+struct AxisArgs {
+    const float2 *src;
+    float2 *dst;       // src, or an array that does not overlap it
+    int L;
+    int C, S;
+    int64_t ncols, nslabs;
+    int64_t ncb;       // column blocks
+    int in_off, out_off;
+    int vec;           // 1: two columns per lane (16-byte accesses)
+    float sign, scale;
+    const float *mask; // last pass only, or null
+    int64_t mask_div;  // elements per mask entry: 1 or the batch
+    Stages st;
+    const float2 *tw;
+    const int *pinv;
+};
+
+inline size_t axis_lds(int L, int lines)
+{
+    return (size_t)L * sizeof(float2) + (size_t)L * (lines + 1) * sizeof(float2) + (size_t)L * sizeof(int);
+}
+
+__global__ __launch_bounds__(kAxisThreads) void k_fft_axis(AxisArgs a)
+{
+    extern __shared__ float2 lds_axis[];
+    const int lines = a.C * a.S, estride = lines + 1;
+    float2 *tw = lds_axis, *buf = tw + a.L;
+    int *spinv = (int *)(buf + a.L * estride);
+    const int64_t sb = blockIdx.x / a.ncb, slab0 = sb * a.S, col0 = (blockIdx.x - sb * a.ncb) * a.C;
+    const int ns = (int)min((int64_t)a.S, a.nslabs - slab0), nc = (int)min((int64_t)a.C, a.ncols - col0);
+    const int64_t base = slab0 * a.L * a.ncols + col0;
+    const int ws = a.vec, cw = nc >> ws; // vec: nc is even
+    const int total = ns * a.L * cw;
+    const float rcw = 1.0f / (float)cw, rL = 1.0f / (float)a.L;
+    // element e of the block: lane columns j, j + ws; row n; slab s (line s * C + j)
+    auto place = [&](int e, int &line, int &n) -> int64_t {
+        const int r = fdiv(e, cw, rcw), j = (e - r * cw) << ws;
+        const int s = fdiv(r, a.L, rL);
+        n = r - s * a.L;
+        line = s * a.C + j;
+        return base + (int64_t)r * a.ncols + j; // (s * L + n) * ncols + j
+    };
+    load_tables(tw, spinv, a.tw, a.pinv, a.L, a.sign);
+    __syncthreads();
+    for (int e0 = threadIdx.x; e0 < total; e0 += kAxisUnroll * kAxisThreads) {
+        float4 v[kAxisUnroll];
+        int at[kAxisUnroll];
+#pragma unroll
+        for (int u = 0; u < kAxisUnroll; ++u) {
+            const int e = e0 + u * kAxisThreads;
+            v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (e < total) {
+                int line, n;
+                const float2 *p = a.src + place(e, line, n);
+                if (ws) {
+                    v[u] = *reinterpret_cast<const float4 *>(p);
+                } else {
+                    const float2 t = *p;
+                    v[u].x = t.x;
+                    v[u].y = t.y;
+                }
+                int q = n + a.in_off;
+                if (q >= a.L) q -= a.L;
+                at[u] = spinv[q] * estride + line;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kAxisUnroll; ++u)
+            if (e0 + u * kAxisThreads < total) {
+                buf[at[u]] = make_float2(v[u].x, v[u].y);
+                if (ws) buf[at[u] + 1] = make_float2(v[u].z, v[u].w);
+            }
+    }
+    __syncthreads();
+    if ((lines & 1) == 0)
+        fft_lines<2>(buf, lines, 1, estride, a.L, a.st, tw, a.sign);
+    else
+        fft_lines<1>(buf, lines, 1, estride, a.L, a.st, tw, a.sign);
+    for (int e = threadIdx.x; e < total; e += kAxisThreads) {
+        int line, n;
+        const int64_t g = place(e, line, n);
+        int q = n + a.out_off;
+        if (q >= a.L) q -= a.L;
+        const float2 lo = buf[q * estride + line];
+        float f0 = a.scale, f1 = a.scale;
+        if (a.mask) {
+            // mask_div is 1 or the batch, which divides ncols
+            f0 *= a.mask_div == 1 ? a.mask[g] : a.mask[g / a.mask_div];
+            if (ws) f1 *= a.mask_div == 1 ? a.mask[g + 1] : a.mask[(g + 1) / a.mask_div];
+        }
+        if (ws) {
+            const float2 hi = buf[q * estride + line + 1];
+            *reinterpret_cast<float4 *>(a.dst + g) = make_float4(lo.x * f0, lo.y * f0, hi.x * f1, hi.y * f1);
+        } else {
+            a.dst[g] = make_float2(lo.x * f0, lo.y * f0);
+        }
+    }
+}
+
+// Tables per (device, length), kept until the process ends: lengths are at most 2048,
+// 12 bytes per point.  Under g_cfft_mu.
+std::map<std::pair<int, int>, FFTAxis> g_axis_tables;
+
+int axis_table(int dev, int L, FFTAxis **ax)
+{
+    auto it = g_axis_tables.find({dev, L});
+    if (it == g_axis_tables.end()) {
+        FFTAxis t;
+        const int rc = fft_axis_init(&t, L);
+        if (rc) {
+            fft_axis_free(&t);
+            return rc;
+        }
+        it = g_axis_tables.emplace(std::make_pair(dev, L), t).first;
+    }
+    *ax = &it->second;
+    return GN_OK;
+}
+
+// The axis passes apply: every length is 1 or covered, and the output is the input or
+// does not overlap it.
+bool axis_passes_ok(int rank, const int64_t *n, int64_t total, const void *in, const void *out)
+{
+    bool any = false;
+    for (int a = 0; a < rank; ++a) {
+        if (n[a] == 1) continue;
+        if (!fft_length_supported(n[a])) return false;
+        any = true;
+    }
+    const uintptr_t i = (uintptr_t)in, o = (uintptr_t)out, bytes = (uintptr_t)total * sizeof(float2);
+    const bool overlap = i != o && i < o + bytes && o < i + bytes;
+    return any && !overlap && total < ((int64_t)1 << 40);
+}
+
+int axis_passes(const ShiftArgs &sh, bool fwd, const float2 *in, float2 *out, hipStream_t st)
+{
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    int last = sh.rank - 1;
+    while (sh.n[last] == 1) --last;
+    const float2 *src = in;
+    int64_t slabs = 1;
+    for (int ax = 0; ax <= last; ++ax) {
+        const int64_t n = sh.n[ax];
+        if (n == 1) continue;
+        FFTAxis *t = nullptr;
+        const int rc = axis_table(dev, (int)n, &t);
+        if (rc) return rc;
+        AxisArgs a;
+        a.src = src;
+        a.dst = out;
+        a.L = (int)n;
+        a.nslabs = slabs;
+        a.ncols = sh.total / (slabs * n);
+        const bool even = (a.ncols & 1) == 0;
+        int lines = kAxisLines;
+        while (lines > 1 && axis_lds(a.L, lines) > kAxisLdsMax) lines /= 2;
+        if (a.ncols >= lines) {
+            a.C = lines;
+            a.S = 1;
+            while (a.C > 4 && (a.ncols + a.C - 1) / a.C * slabs < kAxisBlocks) a.C /= 2;
+        } else {
+            a.C = (int)a.ncols;
+            a.S = (int)std::min<int64_t>(lines / a.C, slabs);
+            while (a.S > 1 && (slabs + a.S - 1) / a.S < kAxisBlocks) a.S = (a.S + 1) / 2;
+        }
+        a.ncb = (a.ncols + a.C - 1) / a.C;
+        a.vec = even && a.C % 2 == 0 && (((uintptr_t)a.src | (uintptr_t)a.dst) & 15) == 0 ? 1 : 0;
+        // fftshift: input row n sits at position n + L/2; ifftshift: output row n is index n + L/2
+        a.in_off = sh.pre ? a.L / 2 : 0;
+        a.out_off = sh.post ? a.L / 2 : 0;
+        a.sign = fwd ? -1.0f : 1.0f;
+        a.scale = ax == last ? sh.scale : 1.0f;
+        a.mask = ax == last ? sh.mask : nullptr;
+        a.mask_div = sh.mask_batch > 1 ? 1 : sh.batch;
+        a.st = make_stages(*t);
+        a.tw = t->tw;
+        a.pinv = t->pinv;
+        const int64_t nblk = (slabs + a.S - 1) / a.S * a.ncb;
+        if (nblk >= ((int64_t)1 << 31)) return fail(GN_EINVAL, "gn_fft_c2c: array too large");
+        hipLaunchKernelGGL(k_fft_axis, dim3((unsigned)nblk), dim3(kAxisThreads), axis_lds(a.L, a.C * a.S), st, a);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return hip_fail(e, "FFT axis pass");
+        src = out;
+        slabs *= n;
+    }
+    return GN_OK;
 }
 
 int cfft_plan(int rank, const int64_t *n, int64_t batch, bool forward, CPlan **out)
@@ -153,6 +364,12 @@ int gn_fft_c2c(int rank, const int64_t *shape, int64_t batch, int direction, int
     a.mask_batch = mask_batch;
     hipStream_t st = (hipStream_t)stream;
     std::lock_guard<std::mutex> g(g_cfft_mu);
+    if (axis_passes_ok(rank, a.n, a.total, in, out)) {
+        const int r = axis_passes(a, fwd, (const float2 *)in, (float2 *)out, st);
+        if (r || (flags & GN_FFT_ASYNC)) return r;
+        hipError_t e = hipStreamSynchronize(st);
+        return e == hipSuccess ? GN_OK : hip_fail(e, "FFT synchronize");
+    }
     CPlan *cp = nullptr;
     int rc = cfft_plan(rank, a.n, batch, fwd, &cp);
     if (rc) return rc;

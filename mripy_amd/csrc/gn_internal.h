@@ -303,6 +303,7 @@ void default_tiles(int dim, int ns, const int64_t *nf, int *tile, int *gtile);
 bool fft_length_supported(int64_t L);
 int fft_axis_init(FFTAxis *ax, int L);
 void fft_axis_free(FFTAxis *ax);
+Stages make_stages(const FFTAxis &ax);
 int pruned_type2_rows(gn_plan_s *p, const float2 *image, float scale, float sign);
 int pruned_type2_cols(gn_plan_s *p, float sign);
 int pruned_type1_cols(gn_plan_s *p, float sign);

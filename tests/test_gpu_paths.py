@@ -34,3 +34,40 @@ def test_spread_coil_groups(modes, nc):
     p = O.Params(modes, rat=2, nspread=3)
     ref = O.type1([c.astype(np.float64) for c in coords], y.astype(np.complex128), p)
     assert rel(P.type1(y), ref) <= TOL
+
+
+# (shape, rank): one long line, odd and even batches, unit axes, ragged column blocks,
+# several slabs per block, the longest covered length, and lengths left to rocFFT
+@pytest.mark.parametrize("shape,rank", [((2048,), 1), ((2, 3), 2), ((1, 30, 1), 3), ((45, 1, 2), 2), ((27, 50, 3), 2),
+                                        ((20, 25, 21), 2), ((9, 8, 15, 2), 3), ((160, 6, 33), 2), ((4, 2048, 1), 2),
+                                        ((17, 31), 2), ((2049,), 1), ((12, 2050), 2)])
+@pytest.mark.parametrize("batch_mask", [False, True])
+def test_cartesian_axis_passes(shape, rank, batch_mask):
+    """gn_fft_c2c with shifts and mask, both directions, out of place, in place and from a
+    base that is only 8-byte aligned."""
+    import torch
+    from mripy_amd import _lib
+    from mripy_amd.cfft import _c2c
+    print("case: c2c", shape, rank, batch_mask, flush=True)
+    rng = np.random.default_rng(sum(shape))
+    x = _cnormal(rng, shape)
+    ax = tuple(range(rank))
+    mask = rng.random(shape if batch_mask else shape[:rank]).astype(np.float32)
+    mb = mask if batch_mask else mask.reshape(shape[:rank] + (1,) * (len(shape) - rank))
+    xs = np.fft.fftshift(x.astype(np.complex128), ax)
+    fwd = np.fft.ifftshift(np.fft.fftn(xs, axes=ax), ax) * mb
+    inv = np.fft.ifftshift(np.fft.ifftn(xs, axes=ax), ax)
+    flags = _lib.GN_FFT_SHIFT_IN | _lib.GN_FFT_SHIFT_OUT
+    buf = torch.empty(x.size + 1, dtype=torch.complex64, device="cuda")
+    for t in (torch.as_tensor(x).cuda(), buf[1:].view(shape)):
+        t.copy_(torch.as_tensor(x))
+        assert rel(_c2c(t, rank, _lib.GN_FFT_FORWARD, flags, torch.as_tensor(mask).cuda()).cpu(), fwd) <= 2e-6
+        assert rel(_c2c(t, rank, _lib.GN_FFT_INVERSE, flags).cpu(), inv) <= 2e-6
+        assert rel(t.cpu(), x) == 0
+    import ctypes
+    shp = (ctypes.c_int64 * 3)(*(shape[:rank] + (1,) * (3 - rank)))
+    batch = int(np.prod(shape[rank:])) if len(shape) > rank else 1
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(_lib.load().gn_fft_c2c(rank, shp, batch, _lib.GN_FFT_INVERSE, flags, None, 1, t.data_ptr(), t.data_ptr(),
+                                      st))
+    assert rel(t.cpu(), inv) <= 2e-6
