@@ -569,7 +569,9 @@ int gn_execute_type21_noalloc(gn_plan *p, const void *in, void *out)
     if ((size_t)(p->M * p->nc) * sizeof(float2) > kNoAllocScratchBytes)
         return fail(GN_EINVAL, "gn_execute_type21_noalloc: M * ncoils exceeds the 4,194,304 complex samples of the "
                                "static scratch");
-    if (!(p->fft_custom && p->fft_engine == GN_FFT_AUTO))
+    bool smooth = p->fft_custom && p->fft_engine == GN_FFT_AUTO;
+    for (int a = 0; a < p->geo.dim; ++a) smooth &= fft_length_smooth(p->geo.nf[a]);
+    if (!smooth)
         return fail(GN_ESTATE, "gn_execute_type21_noalloc needs the pruned FFT passes (grid lengths with prime "
                                "factors 2, 3, 5 and the default engine): rocFFT plans allocate");
     if (p->timing) return fail(GN_ESTATE, "gn_execute_type21_noalloc: stage timers create events; disable them");

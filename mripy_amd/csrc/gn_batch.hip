@@ -55,6 +55,7 @@ struct LaunchList {
 // length; the LDS size is the largest any of them needs
 struct FFTLaunch {
     size_t lds = 0;
+    bool gen = false; // prime radices (of the length, so of every item)
     std::vector<int4> items;
     int4 *d = nullptr;
 };
@@ -307,7 +308,8 @@ int build_fft_lists(gn_batch_s *b)
             b->frows.push_back(FFTLaunch());
         }
         FFTLaunch &rl = b->frows[rkey[ra.L]];
-        rl.lds = std::max(rl.lds, row_lds(ra.L, ra.CL)); // coils per block vary with the instance
+        rl.gen = ra.st.gen;
+        rl.lds = std::max(rl.lds, row_lds(ra.L, ra.CL, ra.st.dbl)); // coils per block vary with the instance
         const int64_t nch = (p->nc + ra.CL - 1) / ra.CL;
         for (int64_t line = 0; line < ra.nlines; ++line)
             for (int64_t c = 0; c < nch; ++c) rl.items.push_back(make_int4(i, (int)line, (int)c, 0));
@@ -318,7 +320,8 @@ int build_fft_lists(gn_batch_s *b)
                 if (!ckey[t][k].count(a.L)) {
                     ckey[t][k][a.L] = b->fcols[t][k].size();
                     FFTLaunch l;
-                    l.lds = col_lds(a.L, a.CB);
+                    l.lds = col_lds(a.L, a.CB, a.st.dbl);
+                    l.gen = a.st.gen;
                     b->fcols[t][k].push_back(l);
                 }
                 FFTLaunch &cl = b->fcols[t][k][ckey[t][k][a.L]];
@@ -349,7 +352,7 @@ int launch_fft_cols(gn_batch_s *b, int t, hipStream_t st)
 {
     for (int k = 0; k < 2; ++k)
         for (auto &l : b->fcols[t][k]) {
-            hipError_t e = launch_fft_cols_batch(b->d_cols[t], l.d, (int)l.items.size(), l.lds, st);
+            hipError_t e = launch_fft_cols_batch(l.gen, b->d_cols[t], l.d, (int)l.items.size(), l.lds, st);
             if (e != hipSuccess) return hip_fail(e, "batch FFT column pass");
         }
     return GN_OK;
@@ -358,7 +361,7 @@ int launch_fft_cols(gn_batch_s *b, int t, hipStream_t st)
 int launch_fft_rows(gn_batch_s *b, bool pad, const RowArgs *args, hipStream_t st)
 {
     for (auto &l : b->frows) {
-        hipError_t e = launch_fft_rows_batch(pad, args, l.d, (int)l.items.size(), l.lds, st);
+        hipError_t e = launch_fft_rows_batch(pad, l.gen, args, l.d, (int)l.items.size(), l.lds, st);
         if (e != hipSuccess) return hip_fail(e, pad ? "batch FFT pass A" : "batch FFT pass A'");
     }
     return GN_OK;

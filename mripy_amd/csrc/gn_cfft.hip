@@ -117,17 +117,14 @@ struct AxisArgs {
     const int *pinv;
 };
 
-inline size_t axis_lds(int L, int lines)
-{
-    return (size_t)L * sizeof(float2) + (size_t)L * (lines + 1) * sizeof(float2) + (size_t)L * sizeof(int);
-}
-
-__global__ __launch_bounds__(kAxisThreads) void k_fft_axis(AxisArgs a)
+template <bool GEN>
+__global__ __launch_bounds__(kAxisThreads, GEN ? 6 : 1) void k_fft_axis(AxisArgs a)
 {
     extern __shared__ float2 lds_axis[];
     const int lines = a.C * a.S, estride = lines + 1;
     float2 *tw = lds_axis, *buf = tw + a.L;
-    int *spinv = (int *)(buf + a.L * estride);
+    float2 *alt = buf + a.L * estride;
+    int *spinv = (int *)(GEN && a.st.dbl ? alt + a.L * estride : alt);
     const int64_t sb = blockIdx.x / a.ncb, slab0 = sb * a.S, col0 = (blockIdx.x - sb * a.ncb) * a.C;
     const int ns = (int)min((int64_t)a.S, a.nslabs - slab0), nc = (int)min((int64_t)a.C, a.ncols - col0);
     const int64_t base = slab0 * a.L * a.ncols + col0;
@@ -174,16 +171,14 @@ __global__ __launch_bounds__(kAxisThreads) void k_fft_axis(AxisArgs a)
             }
     }
     __syncthreads();
-    if ((lines & 1) == 0)
-        fft_lines<2>(buf, lines, 1, estride, a.L, a.st, tw, a.sign);
-    else
-        fft_lines<1>(buf, lines, 1, estride, a.L, a.st, tw, a.sign);
+    const float2 *res = (lines & 1) == 0 ? fft_lines<2, GEN>(buf, alt, lines, 1, estride, a.L, a.st, tw, a.sign)
+                                         : fft_lines<1, GEN>(buf, alt, lines, 1, estride, a.L, a.st, tw, a.sign);
     for (int e = threadIdx.x; e < total; e += kAxisThreads) {
         int line, n;
         const int64_t g = place(e, line, n);
         int q = n + a.out_off;
         if (q >= a.L) q -= a.L;
-        const float2 lo = buf[q * estride + line];
+        const float2 lo = res[q * estride + line];
         float f0 = a.scale, f1 = a.scale;
         if (a.mask) {
             // mask_div is 1 or the batch, which divides ncols
@@ -191,7 +186,7 @@ __global__ __launch_bounds__(kAxisThreads) void k_fft_axis(AxisArgs a)
             if (ws) f1 *= a.mask_div == 1 ? a.mask[g + 1] : a.mask[(g + 1) / a.mask_div];
         }
         if (ws) {
-            const float2 hi = buf[q * estride + line + 1];
+            const float2 hi = res[q * estride + line + 1];
             *reinterpret_cast<float4 *>(a.dst + g) = make_float4(lo.x * f0, lo.y * f0, hi.x * f1, hi.y * f1);
         } else {
             a.dst[g] = make_float2(lo.x * f0, lo.y * f0);
@@ -255,8 +250,9 @@ int axis_passes(const ShiftArgs &sh, bool fwd, const float2 *in, float2 *out, hi
         a.nslabs = slabs;
         a.ncols = sh.total / (slabs * n);
         const bool even = (a.ncols & 1) == 0;
+        a.st = make_stages(*t);
         int lines = kAxisLines;
-        while (lines > 1 && axis_lds(a.L, lines) > kAxisLdsMax) lines /= 2;
+        while (lines > 1 && col_lds(a.L, lines, a.st.dbl) > kAxisLdsMax) lines /= 2;
         if (a.ncols >= lines) {
             a.C = lines;
             a.S = 1;
@@ -275,13 +271,19 @@ int axis_passes(const ShiftArgs &sh, bool fwd, const float2 *in, float2 *out, hi
         a.scale = ax == last ? sh.scale : 1.0f;
         a.mask = ax == last ? sh.mask : nullptr;
         a.mask_div = sh.mask_batch > 1 ? 1 : sh.batch;
-        a.st = make_stages(*t);
         a.tw = t->tw;
         a.pinv = t->pinv;
         const int64_t nblk = (slabs + a.S - 1) / a.S * a.ncb;
         if (nblk >= ((int64_t)1 << 31)) return fail(GN_EINVAL, "gn_fft_c2c: array too large");
-        hipLaunchKernelGGL(k_fft_axis, dim3((unsigned)nblk), dim3(kAxisThreads), axis_lds(a.L, a.C * a.S), st, a);
-        hipError_t e = hipGetLastError();
+        auto kernel = a.st.gen ? k_fft_axis<true> : k_fft_axis<false>;
+        const size_t lds = col_lds(a.L, a.C * a.S, a.st.dbl);
+        hipError_t e = hipSuccess;
+        if (lds > kAxisLdsMax) // long lines with a second buffer
+            e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e == hipSuccess) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(kAxisThreads), lds, st, a);
+            e = hipGetLastError();
+        }
         if (e != hipSuccess) return hip_fail(e, "FFT axis pass");
         src = out;
         slabs *= n;

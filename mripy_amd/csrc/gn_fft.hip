@@ -18,7 +18,8 @@
 // leading rows of the grid itself and no scratch buffer is needed.  Deapodization
 // and scale are applied in A (type 2) and A' (type 1), which also read / write the
 // caller's coil-last or coil-major image.  Each 1-D FFT runs in LDS as an in-place
-// mixed-radix (8, 4, 2, 3, 5) decimation-in-time transform: loads scatter the input
+// mixed-radix (8, 4, 2, 3, 5) decimation-in-time transform, with primes up to 256 in
+// kernels of their own (GEN): loads scatter the input
 // to digit-reversed slots, so the stages need no reordering and the output comes
 // out in natural order.
 // Twiddles come from an FP64-computed table of e^{-2 pi i k / L}.
@@ -69,7 +70,7 @@ __device__ inline unsigned long long col_mask(const ColArgs &a, const unsigned l
 }
 
 // MASK: 0 none, 1 read mask (cells outside it enter the FFT as zeros)
-template <int MASK>
+template <int MASK, bool GEN>
 __device__ __forceinline__ void fft_cols_body(const ColArgs &a, int64_t colblk, int64_t slab)
 {
     extern __shared__ float2 lds_fft[];
@@ -103,7 +104,8 @@ __device__ __forceinline__ void fft_cols_body(const ColArgs &a, int64_t colblk, 
         mw0 = col_mask(a, a.rmask, col0 + min(j, ncb - 1));
         mw1 = col_mask(a, a.rmask, col0 + min(j + 1, ncb - 1));
     }
-    int *spinv = (int *)(buf + a.L * estride); // digit-reversal map, staged in LDS
+    float2 *alt = buf + a.L * estride; // second line buffer (direct-sum stages only)
+    int *spinv = (int *)(GEN && a.st.dbl ? alt + a.L * estride : alt); // digit-reversal map, staged in LDS
     // kColLoadUnroll independent global loads in flight per thread before the LDS stores.
     // 16- and 8-byte cells take separate loops, and the mask is applied at the LDS
     // stores: a loaded value that is copied or selected right after its load makes the
@@ -205,10 +207,8 @@ __device__ __forceinline__ void fft_cols_body(const ColArgs &a, int64_t colblk, 
     }
     __syncthreads();
     // columns in pairs: one index computation and one set of twiddle reads serve both
-    if ((CB & 1) == 0)
-        fft_lines<2>(buf, CB, lstride, estride, a.L, a.st, tw, a.sign);
-    else
-        fft_lines<1>(buf, CB, lstride, estride, a.L, a.st, tw, a.sign);
+    const float2 *res = (CB & 1) == 0 ? fft_lines<2, GEN>(buf, alt, CB, lstride, estride, a.L, a.st, tw, a.sign)
+                                      : fft_lines<1, GEN>(buf, alt, CB, lstride, estride, a.L, a.st, tw, a.sign);
     const int half_out = a.rows_out / 2;
     for (int e = threadIdx.x; e < a.rows_out * cbw; e += blockDim.x) {
         const int n = e >> cbws, j = (e & (cbw - 1)) << ws;
@@ -218,7 +218,7 @@ __device__ __forceinline__ void fft_cols_body(const ColArgs &a, int64_t colblk, 
             p = n - half_out;
             if (p < 0) p += a.L;
         }
-        const float2 *src = buf + p * estride + j;
+        const float2 *src = res + p * estride + j;
         float2 *dst = base + (int64_t)n * a.ncols + j;
         if (v2) {
             const float2 lo = src[0], hi = src[1];
@@ -229,10 +229,10 @@ __device__ __forceinline__ void fft_cols_body(const ColArgs &a, int64_t colblk, 
     }
 }
 
-template <int MASK>
-__global__ __launch_bounds__(kFFTColThreads) void k_fft_cols(ColArgs a)
+template <int MASK, bool GEN>
+__global__ __launch_bounds__(kFFTColThreads, GEN ? 6 : 1) void k_fft_cols(ColArgs a)
 {
-    fft_cols_body<MASK>(a, blockIdx.x, blockIdx.y);
+    fft_cols_body<MASK, GEN>(a, blockIdx.x, blockIdx.y);
 }
 
 // Pass C of a 3-D type 2 (m0 rows in, nf0 rows out at a stride of a whole plane):
@@ -242,16 +242,17 @@ constexpr int kFFTColThreadsWide = 2 * kFFTColThreads;
 constexpr int kWideCB = 2 * GN_FFT_CB;
 __global__ __launch_bounds__(kFFTColThreadsWide) void k_fft_cols_wide(ColArgs a)
 {
-    fft_cols_body<0>(a, blockIdx.x, blockIdx.y);
+    fft_cols_body<0, false>(a, blockIdx.x, blockIdx.y);
 }
 
 // Batched column passes: items[b] = {argument index, column block, slab, 0}.
-__global__ __launch_bounds__(kFFTColThreads) void k_fft_cols_batch(const ColArgs *__restrict__ args,
+template <bool GEN>
+__global__ __launch_bounds__(kFFTColThreads, GEN ? 6 : 1) void k_fft_cols_batch(const ColArgs *__restrict__ args,
                                                                    const int4 *__restrict__ items)
 {
     const int4 it = items[blockIdx.x];
     const ColArgs &a = args[it.x]; // read in place: uniform scalar loads
-    fft_cols_body<0>(a, it.y, it.z);
+    fft_cols_body<0, GEN>(a, it.y, it.z);
 }
 
 // ---------------------------------------------------------------------------
@@ -278,6 +279,7 @@ __device__ inline bool grid_pairs(const RowArgs &a)
     return aligned16(a.grid) && ((a.L | a.s0 | a.G) & 1) == 0;
 }
 
+template <bool GEN>
 __device__ __forceinline__ void fft_rows_pad_body(const RowArgs &a, int64_t line, int64_t chunk)
 {
     extern __shared__ float2 lds_fft[];
@@ -286,7 +288,8 @@ __device__ __forceinline__ void fft_rows_pad_body(const RowArgs &a, int64_t line
     const int64_t c0 = chunk * a.CL;
     const int ncl = (int)min((int64_t)a.CL, a.nc - c0);
     const int ls = a.L + 1;
-    int *spinv = (int *)(buf + a.CL * ls);
+    float2 *alt = buf + a.CL * ls; // second line buffer (direct-sum stages only)
+    int *spinv = (int *)(GEN && a.st.dbl ? alt + a.CL * ls : alt);
     load_tables(tw, spinv, a.tw, a.pinv, a.L, a.sign);
     for (int e = threadIdx.x; e < ncl * ls; e += blockDim.x) buf[e] = make_float2(0.f, 0.f);
     __syncthreads();
@@ -357,14 +360,15 @@ __device__ __forceinline__ void fft_rows_pad_body(const RowArgs &a, int64_t line
         }
     }
     __syncthreads();
-    fft_lines<1>(buf, ncl, ls, 1, a.L, a.st, tw, a.sign);
+    const float2 *res = fft_lines<1, GEN>(buf, alt, ncl, ls, 1, a.L, a.st, tw, a.sign);
     const int64_t off = n0 * a.s0 + n1 * a.L;
     for (int e = threadIdx.x; e < ncl * a.L; e += blockDim.x) {
         const int c = fdiv(e, a.L, rL), k = e - c * a.L;
-        a.grid[(c0 + c) * a.G + off + k] = buf[c * ls + k];
+        a.grid[(c0 + c) * a.G + off + k] = res[c * ls + k];
     }
 }
 
+template <bool GEN>
 __device__ __forceinline__ void fft_rows_crop_body(const RowArgs &a, int64_t line, int64_t chunk)
 {
     extern __shared__ float2 lds_fft[];
@@ -376,7 +380,8 @@ __device__ __forceinline__ void fft_rows_crop_body(const RowArgs &a, int64_t lin
     const int64_t n0 = (uint32_t)line / (uint32_t)a.m_b, n1 = line - n0 * a.m_b; // line < 2^31
     const int64_t off = n0 * a.s0 + n1 * a.L;
     const float rncl = 1.0f / (float)ncl, rm = 1.0f / (float)a.m, rL = 1.0f / (float)a.L;
-    int *spinv = (int *)(buf + a.CL * ls);
+    float2 *alt = buf + a.CL * ls; // second line buffer (direct-sum stages only)
+    int *spinv = (int *)(GEN && a.st.dbl ? alt + a.CL * ls : alt);
     load_tables(tw, spinv, a.tw, a.pinv, a.L, a.sign);
     __syncthreads();
     const int gw = grid_pairs(a) ? 1 : 0; // log2 of the elements per lane
@@ -408,7 +413,7 @@ __device__ __forceinline__ void fft_rows_crop_body(const RowArgs &a, int64_t lin
         }
     }
     __syncthreads();
-    fft_lines<1>(buf, ncl, ls, 1, a.L, a.st, tw, a.sign);
+    const float2 *res = fft_lines<1, GEN>(buf, alt, ncl, ls, 1, a.L, a.st, tw, a.sign);
     const float d01 = a.scale * a.deap_a[n0] * (a.deap_b ? a.deap_b[n1] : 1.0f);
     const int half = a.m / 2;
     const bool cl = a.layout == GN_COIL_LAST;
@@ -419,7 +424,7 @@ __device__ __forceinline__ void fft_rows_crop_body(const RowArgs &a, int64_t lin
             const float d = d01 * a.deap_last[n];
             float2 acc = make_float2(0.f, 0.f);
             for (int c = 0; c < ncl; ++c) {
-                const float2 v = buf[c * ls + p];
+                const float2 v = res[c * ls + p];
                 const float2 o = make_float2(v.x * d, v.y * d);
                 const float2 sc = cl ? a.sens[(line * a.m + n) * a.nc + c] : a.sens[c * a.nlines * a.m + line * a.m + n];
                 acc.x += sc.x * o.x + sc.y * o.y;
@@ -434,7 +439,7 @@ __device__ __forceinline__ void fft_rows_crop_body(const RowArgs &a, int64_t lin
         int p = n - half;
         if (p < 0) p += a.L;
         const float d = d01 * dl;
-        const float2 v = buf[c * ls + p];
+        const float2 v = res[c * ls + p];
         return make_float2(v.x * d, v.y * d);
     };
     // the deapodization factors of kCropSteps output steps are loaded together
@@ -484,35 +489,45 @@ __device__ __forceinline__ void fft_rows_crop_body(const RowArgs &a, int64_t lin
 // host side
 // ---------------------------------------------------------------------------
 
-using host::fft_radices;
-
-__global__ __launch_bounds__(kFFTThreads) void k_fft_rows_pad(RowArgs a) { fft_rows_pad_body(a, blockIdx.x, blockIdx.y); }
-__global__ __launch_bounds__(kFFTThreads) void k_fft_rows_crop(RowArgs a) { fft_rows_crop_body(a, blockIdx.x, blockIdx.y); }
+template <bool GEN>
+__global__ __launch_bounds__(kFFTThreads) void k_fft_rows_pad(RowArgs a)
+{
+    fft_rows_pad_body<GEN>(a, blockIdx.x, blockIdx.y);
+}
+template <bool GEN>
+__global__ __launch_bounds__(kFFTThreads) void k_fft_rows_crop(RowArgs a)
+{
+    fft_rows_crop_body<GEN>(a, blockIdx.x, blockIdx.y);
+}
 
 // Batched row passes: items[b] = {instance, image line, coil chunk, 0}.
+template <bool GEN>
 __global__ __launch_bounds__(kFFTThreads) void k_fft_rows_pad_batch(const RowArgs *__restrict__ args,
                                                                     const int4 *__restrict__ items)
 {
     const int4 it = items[blockIdx.x];
     const RowArgs &a = args[it.x]; // read in place: uniform scalar loads
-    fft_rows_pad_body(a, it.y, it.z);
+    fft_rows_pad_body<GEN>(a, it.y, it.z);
 }
+template <bool GEN>
 __global__ __launch_bounds__(kFFTThreads) void k_fft_rows_crop_batch(const RowArgs *__restrict__ args,
                                                                      const int4 *__restrict__ items)
 {
     const int4 it = items[blockIdx.x];
     const RowArgs &a = args[it.x]; // read in place: uniform scalar loads
-    fft_rows_crop_body(a, it.y, it.z);
+    fft_rows_crop_body<GEN>(a, it.y, it.z);
 }
 
 #ifndef GN_FFT_COL_LDS_MAX
 #define GN_FFT_COL_LDS_MAX (64 * 1024)
 #endif
 
-int pick_cb(int L)
+// Lengths with a second line buffer may take two blocks per CU (80 KiB), so that rows keep
+// segments of at least 64 bytes up to 502 points.
+int pick_cb(int L, bool dbl)
 {
     int cb = GN_FFT_CB;
-    while (cb > 1 && col_lds(L, cb) > GN_FFT_COL_LDS_MAX) cb /= 2;
+    while (cb > 1 && col_lds(L, cb, dbl) > (dbl ? 80 * 1024 : GN_FFT_COL_LDS_MAX)) cb /= 2;
     return cb;
 }
 
@@ -525,10 +540,10 @@ int pick_cb(int L)
 #define GN_FFT_ROW_LDS_MAX (24 * 1024)
 #endif
 
-int pick_cl(int L, int64_t nc)
+int pick_cl(int L, int64_t nc, bool dbl)
 {
     int cl = (int)std::min<int64_t>(nc, 16);
-    while (cl > 1 && row_lds(L, cl) > GN_FFT_ROW_LDS_MAX) --cl;
+    while (cl > 1 && row_lds(L, cl, dbl) > GN_FFT_ROW_LDS_MAX) --cl;
     return cl;
 }
 
@@ -547,9 +562,9 @@ ColArgs make_col_args(const FFTAxis &ax, float sign, float2 *data, int rows_in, 
     a.stride_outer = stride_outer;
     a.stride_inner = stride_inner;
     a.nslabs = nslabs;
-    a.CB = pick_cb(ax.L);
     a.sign = sign;
     a.st = make_stages(ax);
+    a.CB = pick_cb(ax.L, a.st.dbl);
     a.tw = ax.tw;
     a.pinv = ax.pinv;
     return a;
@@ -563,15 +578,21 @@ void allow_lds(const void *kernel, size_t lds)
 hipError_t launch_cols(const ColArgs &a, hipStream_t st)
 {
     dim3 grid((unsigned)((a.ncols + a.CB - 1) / a.CB), (unsigned)a.nslabs);
-    const size_t lds = col_lds(a.L, a.CB);
-    if (a.rmask) {
-        allow_lds((const void *)k_fft_cols<1>, lds);
-        hipLaunchKernelGGL(k_fft_cols<1>, grid, dim3(kFFTColThreads), lds, st, a);
-    } else {
-        allow_lds((const void *)k_fft_cols<0>, lds);
-        hipLaunchKernelGGL(k_fft_cols<0>, grid, dim3(kFFTColThreads), lds, st, a);
-    }
-    return hipGetLastError();
+    const size_t lds = col_lds(a.L, a.CB, a.st.dbl);
+    auto go = [&](auto kernel) {
+        allow_lds((const void *)kernel, lds);
+        hipLaunchKernelGGL(kernel, grid, dim3(kFFTColThreads), lds, st, a);
+        return hipGetLastError();
+    };
+    if (a.st.gen) return a.rmask ? go(k_fft_cols<1, true>) : go(k_fft_cols<0, true>);
+    return a.rmask ? go(k_fft_cols<1, false>) : go(k_fft_cols<0, false>);
+}
+
+void launch_rows(void (*kernel)(RowArgs), dim3 grid, const RowArgs &a, hipStream_t st)
+{
+    const size_t lds = row_lds(a.L, a.CL, a.st.dbl);
+    allow_lds((const void *)kernel, lds);
+    hipLaunchKernelGGL(kernel, grid, dim3(kFFTThreads), lds, st, a);
 }
 
 RowArgs row_args(const gn_plan_s *p, const FFTAxis &ax, float sign, float scale)
@@ -588,7 +609,8 @@ RowArgs row_args(const gn_plan_s *p, const FFTAxis &ax, float sign, float scale)
     a.m = (int)g.modes[d - 1];
     a.nlines = g.N / g.modes[d - 1];
     a.nc = p->nc;
-    a.CL = pick_cl(ax.L, p->nc);
+    a.st = make_stages(ax);
+    a.CL = pick_cl(ax.L, p->nc, a.st.dbl);
     a.layout = p->layout;
     a.scale = scale;
     a.sign = sign;
@@ -602,7 +624,6 @@ RowArgs row_args(const gn_plan_s *p, const FFTAxis &ax, float sign, float scale)
         a.deap_last = p->deap + g.modes[0];
         a.m_b = 1;
     }
-    a.st = make_stages(ax);
     a.tw = ax.tw;
     a.pinv = ax.pinv;
     return a;
@@ -610,14 +631,14 @@ RowArgs row_args(const gn_plan_s *p, const FFTAxis &ax, float sign, float scale)
 
 } // namespace
 
-// LDS: twiddles | lines | digit-reversal map
-size_t col_lds(int L, int CB)
+// LDS: twiddles | lines | second line buffer (dbl) | digit-reversal map
+size_t col_lds(int L, int CB, bool dbl)
 {
-    return (size_t)L * sizeof(float2) + (size_t)L * (CB + 1) * sizeof(float2) + (size_t)L * sizeof(int);
+    return (size_t)L * sizeof(float2) + (size_t)L * (CB + 1) * sizeof(float2) * (dbl ? 2 : 1) + (size_t)L * sizeof(int);
 }
-size_t row_lds(int L, int CL)
+size_t row_lds(int L, int CL, bool dbl)
 {
-    return (size_t)L * sizeof(float2) + (size_t)CL * (L + 1) * sizeof(float2) + (size_t)L * sizeof(int);
+    return (size_t)L * sizeof(float2) + (size_t)CL * (L + 1) * sizeof(float2) * (dbl ? 2 : 1) + (size_t)L * sizeof(int);
 }
 
 RowArgs make_row_args(const gn_plan_s *p, float sign, float scale)
@@ -656,25 +677,24 @@ int pruned_col_args(const gn_plan_s *p, bool type2, float sign, ColArgs *out)
     return k;
 }
 
-hipError_t launch_fft_cols_batch(const ColArgs *d_args, const int4 *d_items, int n, size_t lds, hipStream_t st)
-{
-    if (n <= 0) return hipSuccess;
-    allow_lds((const void *)k_fft_cols_batch, lds);
-    hipLaunchKernelGGL(k_fft_cols_batch, dim3((unsigned)n), dim3(kFFTColThreads), lds, st, d_args, d_items);
-    return hipGetLastError();
-}
-
-hipError_t launch_fft_rows_batch(bool pad, const RowArgs *d_args, const int4 *d_items, int n, size_t lds,
+hipError_t launch_fft_cols_batch(bool gen, const ColArgs *d_args, const int4 *d_items, int n, size_t lds,
                                  hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
-    if (pad) {
-        allow_lds((const void *)k_fft_rows_pad_batch, lds);
-        hipLaunchKernelGGL(k_fft_rows_pad_batch, dim3((unsigned)n), dim3(kFFTThreads), lds, st, d_args, d_items);
-    } else {
-        allow_lds((const void *)k_fft_rows_crop_batch, lds);
-        hipLaunchKernelGGL(k_fft_rows_crop_batch, dim3((unsigned)n), dim3(kFFTThreads), lds, st, d_args, d_items);
-    }
+    auto kernel = gen ? k_fft_cols_batch<true> : k_fft_cols_batch<false>;
+    allow_lds((const void *)kernel, lds);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(kFFTColThreads), lds, st, d_args, d_items);
+    return hipGetLastError();
+}
+
+hipError_t launch_fft_rows_batch(bool pad, bool gen, const RowArgs *d_args, const int4 *d_items, int n, size_t lds,
+                                 hipStream_t st)
+{
+    if (n <= 0) return hipSuccess;
+    auto kernel = pad ? (gen ? k_fft_rows_pad_batch<true> : k_fft_rows_pad_batch<false>)
+                      : (gen ? k_fft_rows_crop_batch<true> : k_fft_rows_crop_batch<false>);
+    allow_lds((const void *)kernel, lds);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(kFFTThreads), lds, st, d_args, d_items);
     return hipGetLastError();
 }
 
@@ -682,6 +702,11 @@ Stages make_stages(const FFTAxis &ax)
 {
     Stages s;
     s.n = ax.nst;
+    s.gen = s.dbl = 0;
+    for (int i = 0; i < ax.nst; ++i) {
+        s.gen |= ax.radix[i] == 7 || ax.radix[i] > 8;
+        s.dbl |= ax.radix[i] > host::kFFTRadixMax;
+    }
     int q = 1;
     for (int i = 0; i < kFFTMaxStages; ++i) {
         s.radix[i] = i < ax.nst ? ax.radix[i] : 1;
@@ -693,15 +718,23 @@ Stages make_stages(const FFTAxis &ax)
     return s;
 }
 
+// Up to 2048 points with prime factors up to host::kFFTPrimeMax.  Against pad / rocFFT /
+// crop the pass A + columns of a type 2 took: 224^3 x 8 coils 0.49 instead of 1.89 ms,
+// 182 x 218 x 150 x 3 0.24 / 0.48, 226^3 x 4 0.69 / 1.97, 502^2 x 16 (prime 251) 0.136 /
+// 0.143, 142^2 x 1 0.022 / 0.040: primes above 256 would cost more than rocFFT's
+// Bluestein passes.
 bool fft_length_supported(int64_t L)
 {
     if (L < 2 || L > 2048) return false; // LDS: one line of 2048 + twiddles fits in 64 KiB
-    return !fft_radices((int)L).empty() && (int)fft_radices((int)L).size() <= kFFTMaxStages;
+    const size_t n = host::fft_radices_prime((int)L).size();
+    return n > 0 && n <= (size_t)kFFTMaxStages;
 }
+
+bool fft_length_smooth(int64_t L) { return L >= 1 && L <= 2048 && !host::fft_radices((int)L).empty(); }
 
 int fft_axis_init(FFTAxis *ax, int L)
 {
-    std::vector<int> r = fft_radices(L);
+    std::vector<int> r = host::fft_radices_prime(L);
     if (r.empty() || (int)r.size() > kFFTMaxStages) return fail(GN_EINVAL, "FFT length not supported");
     ax->L = L;
     ax->nst = (int)r.size();
@@ -736,7 +769,7 @@ int pruned_type2_rows_sense(gn_plan_s *p, const float2 *image, float scale, floa
     ra.img_in = image;
     ra.sens = p->sens;
     dim3 ga((unsigned)ra.nlines, (unsigned)((p->nc + ra.CL - 1) / ra.CL));
-    hipLaunchKernelGGL(k_fft_rows_pad, ga, dim3(kFFTThreads), row_lds(az.L, ra.CL), p->stream, ra);
+    launch_rows(ra.st.gen ? k_fft_rows_pad<true> : k_fft_rows_pad<false>, ga, ra, p->stream);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GN_OK : hip_fail(e, "FFT pass A (SENSE)");
 }
@@ -749,20 +782,20 @@ int pruned_type1_rows_sense(gn_plan_s *p, float2 *image, float scale, float sign
     const Geometry &g = p->geo;
     const FFTAxis &az = p->fft_ax[g.dim - 1];
     RowArgs ra = row_args(p, az, sign, scale);
-    const size_t lds = row_lds(az.L, (int)p->nc);
+    const size_t lds = row_lds(az.L, (int)p->nc, ra.st.dbl);
     if (p->nc > 1024 || lds > 160 * 1024) return fail(GN_EINVAL, "SENSE combine: coils do not fit one block");
     ra.CL = (int)p->nc;
     ra.img_out = image;
     ra.sens = p->sens;
-    allow_lds((const void *)k_fft_rows_crop, lds);
-    hipLaunchKernelGGL(k_fft_rows_crop, dim3((unsigned)ra.nlines, 1), dim3(kFFTThreads), lds, p->stream, ra);
+    launch_rows(ra.st.gen ? k_fft_rows_crop<true> : k_fft_rows_crop<false>, dim3((unsigned)ra.nlines, 1), ra, p->stream);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GN_OK : hip_fail(e, "FFT pass A' (SENSE)");
 }
 
 bool sense_rows_fit(const gn_plan_s *p)
 {
-    return p->nc <= 1024 && row_lds(p->fft_ax[p->geo.dim - 1].L, (int)p->nc) <= 160 * 1024;
+    const FFTAxis &az = p->fft_ax[p->geo.dim - 1];
+    return p->nc <= 1024 && row_lds(az.L, (int)p->nc, make_stages(az).dbl) <= 160 * 1024;
 }
 
 // Type 2, pass A: image -> leading grid rows (pad, deapodize, scale, FFT along the last axis).
@@ -773,7 +806,7 @@ int pruned_type2_rows(gn_plan_s *p, const float2 *image, float scale, float sign
     RowArgs ra = row_args(p, az, sign, scale);
     ra.img_in = image;
     dim3 ga((unsigned)ra.nlines, (unsigned)((p->nc + ra.CL - 1) / ra.CL));
-    hipLaunchKernelGGL(k_fft_rows_pad, ga, dim3(kFFTThreads), row_lds(az.L, ra.CL), p->stream, ra);
+    launch_rows(ra.st.gen ? k_fft_rows_pad<true> : k_fft_rows_pad<false>, ga, ra, p->stream);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GN_OK : hip_fail(e, "FFT pass A");
 }
@@ -798,8 +831,8 @@ int pruned_type2_cols(gn_plan_s *p, float sign)
     for (int k = 0; k < n; ++k) {
         hipError_t e;
         ColArgs &c = a[k];
-        const size_t wide_lds = col_lds(c.L, kWideCB);
-        if (k == n - 1 && p->geo.dim == 3 && c.CB == GN_FFT_CB && wide_lds <= 80 * 1024) {
+        const size_t wide_lds = col_lds(c.L, kWideCB, false);
+        if (k == n - 1 && p->geo.dim == 3 && !c.st.gen && c.CB == GN_FFT_CB && wide_lds <= 80 * 1024) {
             c.CB = kWideCB; // two blocks per CU
             dim3 grid((unsigned)((c.ncols + c.CB - 1) / c.CB), (unsigned)c.nslabs);
             allow_lds((const void *)k_fft_cols_wide, wide_lds);
@@ -839,7 +872,7 @@ int pruned_type1_rows(gn_plan_s *p, float2 *image, float scale, float sign)
     RowArgs ra = row_args(p, az, sign, scale);
     ra.img_out = image;
     dim3 ga((unsigned)ra.nlines, (unsigned)((p->nc + ra.CL - 1) / ra.CL));
-    hipLaunchKernelGGL(k_fft_rows_crop, ga, dim3(kFFTThreads), row_lds(az.L, ra.CL), p->stream, ra);
+    launch_rows(ra.st.gen ? k_fft_rows_crop<true> : k_fft_rows_crop<false>, ga, ra, p->stream);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GN_OK : hip_fail(e, "FFT pass A'");
 }

@@ -84,6 +84,32 @@ inline std::vector<int> fft_radices(int L)
     return r;
 }
 
+// The same with primes from 7 up to kFFTPrimeMax, which come first (the first stage
+// needs no twiddles); empty when L has a larger prime factor.  Primes up to
+// kFFTRadixMax are register butterflies, larger ones the direct-sum stage.
+constexpr int kFFTRadixMax = 13;
+constexpr int kFFTPrimeMax = 256;
+inline std::vector<int> fft_radices_prime(int L)
+{
+    std::vector<int> big;
+    int n = L;
+    if (L < 1) return {};
+    while (n % 2 == 0) n /= 2;
+    for (int p : {3, 5})
+        while (n % p == 0) n /= p;
+    int smooth = L / n;
+    for (int p = 7; p <= kFFTPrimeMax && n > 1; p += 2)
+        while (n % p == 0) {
+            big.push_back(p);
+            n /= p;
+        }
+    if (n != 1) return {};
+    std::reverse(big.begin(), big.end());
+    const std::vector<int> r = fft_radices(smooth);
+    big.insert(big.end(), r.begin(), r.end());
+    return big;
+}
+
 // Digit-reversal map (pinv[position] = LDS slot) and twiddles e^{-2 pi i k/L}
 // (tw[2k], tw[2k+1]) of a length-L transform with radices r.
 inline void fft_tables(int L, const std::vector<int> &r, std::vector<int> &pinv, std::vector<float> &tw)

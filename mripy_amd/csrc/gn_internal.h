@@ -55,6 +55,8 @@ struct FFTAxis {
 // line L / r.
 struct Stages {
     int n;
+    int gen; // has a radix above 8 or 7: kernels with GEN
+    int dbl; // has a direct-sum stage: the lines need a second LDS buffer
     int radix[kFFTMaxStages];
     int q[kFFTMaxStages];
     int tws[kFFTMaxStages];
@@ -258,8 +260,8 @@ struct gn_plan_s {
     float *deap = nullptr;    // concatenated per-axis exp(tau k^2) tables
     int *err_flag = nullptr;  // device flag set by set_points on bad coordinates
 
-    // FFT engine: the pruned in-place passes (gn_fft.hip) when every nf is a product
-    // of 2, 3, 5 (fft_custom), else rocFFT; GN_FFT_ROCFFT forces rocFFT
+    // FFT engine: the pruned in-place passes (gn_fft.hip) when they cover every nf
+    // (fft_custom), else rocFFT; GN_FFT_ROCFFT forces rocFFT
     bool fft_custom = false;
     int fft_engine = GN_FFT_AUTO;
     gn::FFTAxis fft_ax[3];
@@ -313,12 +315,14 @@ int pruned_type2_rows_sense(gn_plan_s *p, const float2 *image, float scale, floa
 int pruned_type1_rows_sense(gn_plan_s *p, float2 *image, float scale, float sign);
 bool sense_rows_fit(const gn_plan_s *p);
 // pieces of the pruned passes for the batched launch (batch.hip)
-size_t col_lds(int L, int CB);
-size_t row_lds(int L, int CL);
+size_t col_lds(int L, int CB, bool dbl);
+size_t row_lds(int L, int CL, bool dbl);
+bool fft_length_smooth(int64_t L); // prime factors 2, 3, 5 only
 RowArgs make_row_args(const gn_plan_s *p, float sign, float scale);
 int pruned_col_args(const gn_plan_s *p, bool type2, float sign, ColArgs *out);
-hipError_t launch_fft_cols_batch(const ColArgs *d_args, const int4 *d_items, int n, size_t lds, hipStream_t st);
-hipError_t launch_fft_rows_batch(bool pad, const RowArgs *d_args, const int4 *d_items, int n, size_t lds,
+hipError_t launch_fft_cols_batch(bool gen, const ColArgs *d_args, const int4 *d_items, int n, size_t lds,
+                                 hipStream_t st);
+hipError_t launch_fft_rows_batch(bool pad, bool gen, const RowArgs *d_args, const int4 *d_items, int n, size_t lds,
                                  hipStream_t st);
 
 // api.hip

@@ -40,7 +40,8 @@ def test_spread_coil_groups(modes, nc):
 # several slabs per block, the longest covered length, and lengths left to rocFFT
 @pytest.mark.parametrize("shape,rank", [((2048,), 1), ((2, 3), 2), ((1, 30, 1), 3), ((45, 1, 2), 2), ((27, 50, 3), 2),
                                         ((20, 25, 21), 2), ((9, 8, 15, 2), 3), ((160, 6, 33), 2), ((4, 2048, 1), 2),
-                                        ((17, 31), 2), ((2049,), 1), ((12, 2050), 2)])
+                                        ((17, 31), 2), ((1001, 3), 2), ((2021, 1), 2), ((251, 8, 3), 2), ((2049,), 1),
+                                        ((12, 2050), 2), ((257, 4), 2)])
 @pytest.mark.parametrize("batch_mask", [False, True])
 def test_cartesian_axis_passes(shape, rank, batch_mask):
     """gn_fft_c2c with shifts and mask, both directions, out of place, in place and from a
@@ -71,3 +72,32 @@ def test_cartesian_axis_passes(shape, rank, batch_mask):
     _lib.check(_lib.load().gn_fft_c2c(rank, shp, batch, _lib.GN_FFT_INVERSE, flags, None, 1, t.data_ptr(), t.data_ptr(),
                                       st))
     assert rel(t.cpu(), inv) <= 2e-6
+
+
+@pytest.mark.parametrize("modes,nc", [((7, 11), 3), ((13, 49), 2), ((17, 33), 17), ((251, 20), 2), ((24, 254), 40),
+                                      ((43, 34), 1), ((9, 17, 22), 3), ((17, 10, 29), 9), ((257, 12), 2)])
+def test_prime_grid_lengths(modes, nc):
+    """Grid lengths with primes 7 .. 251 (register butterflies, direct-sum stages, both on one
+    axis, two direct sums) and 257 (rocFFT): both directions, SENSE, and the batched launch
+    equal to the plain plan."""
+    import torch
+    from mripy_amd.batch import BatchPlan
+    from mripy_amd.plan import Plan
+    print("case: prime lengths", modes, nc, flush=True)
+    rng = np.random.default_rng(sum(modes))
+    M = 900
+    coords = [(np.pi * (2 * rng.random(M) - 1)).astype(np.float32) for _ in modes]
+    c64 = [c.astype(np.float64) for c in coords]
+    F, y, x = _cnormal(rng, modes + (nc,)), _cnormal(rng, (M, nc)), _cnormal(rng, modes)
+    P = Plan(modes, ncoils=nc, rat=2, nspread=3).set_points(coords)
+    p = O.Params(modes, rat=2, nspread=3)
+    assert rel(P.type2(F), O.type2(c64, F.astype(np.complex128), p)) <= TOL
+    want = O.type1(c64, y.astype(np.complex128), p)
+    assert rel(P.type1(y), want) <= TOL
+    P.set_sense(F)
+    assert rel(P.sense_type2(x), O.type2(c64, x[..., None] * F.astype(np.complex128), p)) <= TOL
+    assert rel(P.sense_type1(y), (np.conj(F) * want).sum(-1)) <= TOL
+    B = BatchPlan([dict(modes=modes, coords=[torch.as_tensor(c).cuda() for c in coords], ncoils=nc)] * 2)
+    yt, Ft = torch.as_tensor(y).cuda(), torch.as_tensor(F).cuda()
+    assert all(rel(o.cpu(), P.type2(Ft).cpu()) <= 1e-6 for o in B.type2([Ft, Ft]))
+    assert all(rel(o.cpu(), P.type1(yt).cpu()) <= 1e-6 for o in B.type1([yt, yt]))
