@@ -14,7 +14,7 @@ names, arguments and iteration logic.
 Vectors live on the GPU as torch tensors (complex64 images and k-space, as the NUFFT
 computes in).  Every inner product and norm the iteration logic branches on is a
 deterministic FP64 reduction on the device (``gn_dot_f64`` / ``gn_sqdist_f64``), and
-the TV prox runs in FP64 in two HIP kernels per Chambolle step (``gn_tv_prox``).
+the TV prox runs in FP64, several Chambolle steps per kernel (``gn_tv_prox``).
 Operator callables receive and return device tensors (the operator classes in
 ``mripy_amd.operators`` do); a numpy ``b`` is moved to the device and the result is
 returned as numpy.

@@ -101,3 +101,52 @@ def test_prime_grid_lengths(modes, nc):
     yt, Ft = torch.as_tensor(y).cuda(), torch.as_tensor(F).cuda()
     assert all(rel(o.cpu(), P.type2(Ft).cpu()) <= 1e-6 for o in B.type2([Ft, Ft]))
     assert all(rel(o.cpu(), P.type1(yt).cpu()) <= 1e-6 for o in B.type1([yt, yt]))
+
+
+def _tv_ref(x, ndim, niter, amp):
+    from oracle import solvers_oracle as R
+    tv = R.TV2d_r() if ndim == 2 else R.TV3d()
+    G = np.zeros(x.shape + (ndim,))
+    for _ in range(niter):
+        G = G - 0.1 * tv.grad(tv.Div(G) - x / 0.3)
+        a = tv.amp(G) if amp == "reference" else np.sqrt((np.abs(G) ** 2).sum(-1, keepdims=True))
+        G = G / np.maximum(a, np.ones(a.shape))
+    return x - 0.3 * tv.Div(G)
+
+
+@pytest.mark.parametrize("shape,ndim", [((2, 2), 2), ((18, 19), 2), ((33, 17, 3), 2), ((70, 2), 2), ((2, 2, 2), 3),
+                                        ((8, 9, 17), 3), ((11, 3, 8, 2), 3)])
+@pytest.mark.parametrize("niter", [0, 1, 7, 8, 15])
+def test_tv_steps_per_launch(shape, ndim, niter):
+    """Chambolle steps split over launches, at the edges of tiles and regions: against the
+    FP64 oracle per trailing element, both amplitudes."""
+    import torch
+    from mripy_amd import solvers as S
+    print("case: tv", shape, ndim, niter, flush=True)
+    rng = np.random.default_rng(niter + sum(shape))
+    x = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    prox = S.prox_tv2d_r if ndim == 2 else S.prox_tv3d
+    for amp in ("reference", "modulus"):
+        got = prox(torch.as_tensor(x).cuda(), 0.3, niter=niter, amp=amp).cpu().numpy()
+        cols = x.reshape(shape[:ndim] + (-1,))
+        want = np.stack([_tv_ref(cols[..., k], ndim, niter, amp) for k in range(cols.shape[-1])], -1)
+        assert rel(got, want.reshape(shape)) <= 1e-10
+        g32 = prox(torch.as_tensor(x.astype(np.complex64)).cuda(), 0.3, niter=niter, amp=amp)
+        assert g32.dtype == torch.complex64 and rel(g32.cpu(), want.reshape(shape)) <= 1e-5
+
+
+def test_tv_extreme_values():
+    """Fields beyond the range of a^2 + b^2 follow the rule; infinities and NaN stay local."""
+    import torch
+    from mripy_amd import solvers as S
+    rng = np.random.default_rng(3)
+    for scale in (1e100, 1e-200):
+        x = scale * (rng.standard_normal((12, 9)) + 1j * rng.standard_normal((12, 9)))
+        want = _tv_ref(x, 2, 3, "reference")
+        got = S.prox_tv2d_r(torch.as_tensor(x).cuda(), 0.3, niter=3).cpu().numpy()
+        assert np.isfinite(want).all() and np.abs(got - want).max() <= 1e-10 * scale
+    for bad in (np.nan, np.inf):
+        x = rng.standard_normal((20, 40)) + 0j
+        x[3, 4] = bad
+        got = S.prox_tv2d_r(torch.as_tensor(x).cuda(), 0.3, niter=2).cpu().numpy()
+        assert np.isfinite(got[10:, 12:]).all() and not np.isfinite(got[3, 4])
