@@ -43,9 +43,8 @@ struct FFTGroup {
 // one batched kernel launch: work items {instance, item, coil group, 0} of the
 // instances that share its launch shape
 struct LaunchList {
-    int ncg = 0, waves = 0, nbg = 0; // spread
-    bool mfma = false;               // spread on the matrix cores
-    bool wrap = false;               // gather
+    SpreadShape spread;
+    bool wrap = false; // gather
     size_t lds = 0;
     std::vector<int4> items;
     int4 *d = nullptr;
@@ -147,30 +146,22 @@ int upload_list(std::vector<int4> &h, int4 **d)
 int build_lists(gn_batch_s *b)
 {
     free_lists(b);
-    std::map<std::tuple<int, bool, int, int, size_t>, size_t> skey;
+    std::map<std::tuple<int, int, int, int, size_t>, size_t> skey;
     std::map<std::tuple<int, size_t>, size_t> gkey;
     for (int i = 0; i < b->n; ++i) {
         gn_plan_s *p = b->m[i];
         const Geometry &g = p->geo;
         const SpreadArgs sa = make_spread_args(p, nullptr, 0);
-        const int ncg = spread_coil_group(p->nc);
-        int waves = 0, nbg = 0;
-        spread_shape(sa, g.dim, &waves, &nbg);
-        const bool mfma = spread_uses_mfma(sa, g.dim);
-        const size_t slds = spread_lds(sa, ncg, mfma, waves);
-        auto sk = std::make_tuple(ncg, mfma, waves, nbg, slds);
+        const SpreadShape sh = spread_shape(sa, g.dim);
+        auto sk = std::make_tuple(sh.kind, sh.width, sh.waves, sh.nbg, sh.lds);
         if (!skey.count(sk)) {
             skey[sk] = b->spread_lists.size();
             LaunchList l;
-            l.ncg = ncg;
-            l.mfma = mfma;
-            l.waves = waves;
-            l.nbg = nbg;
-            l.lds = slds;
+            l.spread = sh;
             b->spread_lists.push_back(l);
         }
         LaunchList &sl = b->spread_lists[skey[sk]];
-        const int scg = (int)((p->nc + ncg - 1) / ncg);
+        const int scg = (int)((p->nc + sh.coils - 1) / sh.coils);
         for (int k = 0; k < p->rec.n_spread_items; ++k)
             for (int c = 0; c < scg; ++c) sl.items.push_back(make_int4(i, k, c, 0));
         for (int r = 0; r < p->rec.n_reduce_items; ++r) b->reduce_items.push_back(make_int4(i, r, 0, 0));
@@ -455,8 +446,7 @@ int enqueue(gn_batch_s *b, int kind, hipStream_t st)
     };
     auto type1 = [&]() -> int {
         for (auto &l : b->spread_lists)
-            if ((e = launch_spread_batch(b->dim, l.ncg, l.mfma, t.spread, l.d, (int)l.items.size(), l.waves, l.nbg, l.lds,
-                                         st)) != hipSuccess)
+            if ((e = launch_spread_batch(b->dim, l.spread, t.spread, l.d, (int)l.items.size(), st)) != hipSuccess)
                 return hip_fail(e, "batch spread");
         if ((e = launch_spread_reduce_batch(b->dim, t.spread, b->d_reduce, (int)b->reduce_items.size(), st)) !=
             hipSuccess)

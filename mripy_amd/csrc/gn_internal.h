@@ -25,7 +25,7 @@ constexpr int kCoilGroup = 8;       // coils accumulated together per pass
 // 8.  Every group stages the pairs, fills the weight tables and issues the same matrix
 // products whatever its width (a product has columns for 8 coils), so a second group
 // for the remaining coils costs as much as the first: 91 x 109 x 75, 3 coils, nspread 5
-// took 0.80 ms as two groups of 2 and 0.43 ms as one of 4.
+// took 0.80 ms as two groups of 2 and 0.43 ms as one (k_spread_mfma).
 inline int spread_coil_group(int64_t nc) { return nc > 4 ? kCoilGroup : nc > 2 ? 4 : nc > 1 ? 2 : 1; }
 // coils per gather work-group: a coil pair, staged together as 16-byte cells so
 // that one LDS read serves both coils of a tap
@@ -194,6 +194,13 @@ struct SpreadArgs {
     int occ_k = 1;
 };
 
+// Launch shape of a spread: kernel, coils (or reals) per wave it is compiled for, waves
+// and coils per workgroup, workgroups per tile and coil set, dynamic LDS.
+struct SpreadShape {
+    int kind = 0, width = 0, waves = 1, coils = 1, nbg = 1;
+    size_t lds = 0;
+};
+
 struct GatherArgs {
     int64_t nf[3];
     int tile[3];
@@ -333,11 +340,9 @@ int plan_create_impl(int dim, const int64_t *modes, int rat, int nspread, int if
 SpreadArgs make_spread_args(const gn_plan_s *p, const float2 *samples, int use_dcf);
 GatherArgs make_gather_args(const gn_plan_s *p, float2 *samples);
 PrepostArgs make_prepost(const gn_plan_s *p, float scale);
-void spread_shape(const SpreadArgs &a, int dim, int *waves, int *nbg);
-bool spread_uses_mfma(const SpreadArgs &a, int dim);
-size_t spread_lds(const SpreadArgs &a, int ncg, bool mfma, int waves);
-hipError_t launch_spread_batch(int dim, int ncg, bool mfma, const SpreadArgs *d_args, const int4 *d_items, int n,
-                               int waves, int nbg, size_t lds, hipStream_t st);
+SpreadShape spread_shape(const SpreadArgs &a, int dim);
+hipError_t launch_spread_batch(int dim, const SpreadShape &sh, const SpreadArgs *d_args, const int4 *d_items, int n,
+                               hipStream_t st);
 hipError_t launch_spread_reduce_batch(int dim, const SpreadArgs *d_args, const int4 *d_items, int n, hipStream_t st);
 hipError_t launch_gather_batch(int dim, int ns, bool wrap, const GatherArgs *d_args, const int4 *d_items, int n,
                                size_t lds, hipStream_t st);

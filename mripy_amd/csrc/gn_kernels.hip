@@ -1198,9 +1198,453 @@ __global__ __launch_bounds__(64 * kSpreadWavesMax) void k_spread_mfma_batch(cons
     spread_mfma_body<D, NCG>(a, a.items[bi.y], bi.z, (int)(w / gridDim.x));
 }
 
-// Kahan-compensated sum of the partial tiles of each split tile, in slice order;
-// one thread per (coil, cell) of a tile (kReduceThreads covers 8 coils of 128 cells).
-constexpr int kReduceThreads = 1024;
+// ---------------------------------------------------------------------------
+// Adjoint spread of few coils, one wave per tile (v_mfma_f32_16x16x4_f32).
+//
+// For the default tiles (4 x 4 x 8 cells in 3-D, 8 x 16 in 2-D), whose 128 cells are 16
+// "row" cells (the x-y cells, or the 16 y cells) times 8 "slices" (the z planes, or the x
+// rows).  A pair's weight is w_row(i) w_slice(s) and its value v[real], so with
+//     A[i][k] = w_row of pair k,     B[k][(s, real)] = w_slice(s) v[real] of pair k
+// one product accumulates 16 / R slices of R reals (R / 2 coils) for 4 pairs, and M = R / 2
+// products per 4 pairs cover the tile (slice (j / R) M + m in column j of product m):
+// where k_spread_mfma leaves 16 - R columns empty, these are full.  Every pair of a tile
+// reaches it, so there are no lists or masks, and a one-wave workgroup has no barriers to
+// wait at.  Batches of 64 pairs are folded with a Kahan step, as in k_spread_mfma.
+// Bound by the batches' table fills and load latency.  128^3, 1,048,576 samples, 1 coil:
+// nspread 3 486 -> 231 us, nspread 5 1172 -> 491 us; 4 coils, nspread 3 499 -> 459 us.
+// LDS per batch: row weights [B][8 (x, y) or 16], slice weights [B][8], values [B][R]; the
+// 4 pairs of a product fall on distinct banks.
+// ---------------------------------------------------------------------------
+inline size_t spread_tile_lds(int dim, int R)
+{
+    return (size_t)kSpreadBatch * ((dim == 3 ? 8 : 16) + 8 + R) * sizeof(float);
+}
+
+template <int D, int R>
+__device__ __forceinline__ void spread_tile_body(const SpreadArgs &a, const int4 item, const int cgi)
+{
+    constexpr int B = kSpreadBatch, M = R / 2, NC = R / 2; // products per step, coils per wave
+    constexpr int RW = D == 3 ? 8 : 16;                    // row-weight stride
+    constexpr int T0 = D == 3 ? 4 : 8, T1 = D == 3 ? 4 : 16, T2 = D == 3 ? 8 : 1, TC = 128;
+    constexpr int QP = D == 3 ? 4 : 6;                     // table quads per pair
+    extern __shared__ float lds_sp[];
+    if (tile_skippable(a, item)) return; // uniform over the workgroup
+    const int lane = threadIdx.x;
+    float *s_row = lds_sp, *s_sl = s_row + B * RW, *s_v = s_sl + B * 8;
+    const int cg0 = cgi * NC;
+    const int ncg = (int)min((int64_t)NC, a.nc - cg0);
+    const int ri = lane & 15, kg = lane >> 4;
+    const float *pa0 = s_row + (D == 3 ? (ri >> 2) : ri) + kg * RW, *pa1 = s_row + 4 + (ri & 3) + kg * RW;
+    const float *ps = s_sl + (ri / R) * M + kg * 8, *pv = s_v + (ri % R) + kg * R;
+    // coil-last with an even coil count: a pair's coils are 16-byte pairs
+    const bool v4 = NC >= 2 && a.layout == GN_COIL_LAST && ((a.nc | cg0) & 1) == 0 &&
+                    (reinterpret_cast<uintptr_t>(a.in) & 15) == 0;
+    float S[M][4], K[M][4];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) S[m][v] = K[m][v] = 0.f;
+    for (int base = item.y; base < item.z; base += B) {
+        const int n = min(B, item.z - base), np = (n + 3) & ~3;
+        if (base != item.y) __syncthreads(); // previous batch fully consumed (uniform)
+        // values, one pair per lane (pairs n .. np - 1 are zeros)
+        if (lane < np) {
+            float2 v[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) v[c] = make_float2(0.f, 0.f);
+            float scale = 1.0f;
+            if (lane < n) {
+                const int orig = a.pair_a[base + lane].x;
+                if (a.use_dcf) scale = __int_as_float(a.pair_b[base + lane].w);
+                if (v4) {
+                    const float4 *src = reinterpret_cast<const float4 *>(a.in + (int64_t)orig * a.nc + cg0);
+#pragma unroll
+                    for (int c2 = 0; c2 < NC / 2; ++c2)
+                        if (2 * c2 < ncg) {
+                            const float4 t = src[c2];
+                            v[2 * c2] = make_float2(t.x, t.y);
+                            v[2 * c2 + 1] = make_float2(t.z, t.w);
+                        }
+                } else {
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        if (c < ncg)
+                            v[c] = a.layout == GN_COIL_LAST ? a.in[(int64_t)orig * a.nc + cg0 + c]
+                                                            : a.in[(int64_t)(cg0 + c) * a.M + orig];
+                }
+            }
+            if constexpr (NC == 1) {
+                *(float2 *)(s_v + lane * R) = make_float2(v[0].x * scale, v[0].y * scale);
+            } else {
+#pragma unroll
+                for (int c2 = 0; c2 < NC / 2; ++c2)
+                    *(float4 *)(s_v + lane * R + 4 * c2) =
+                        make_float4(v[2 * c2].x * scale, v[2 * c2].y * scale, v[2 * c2 + 1].x * scale,
+                                    v[2 * c2 + 1].y * scale);
+            }
+        }
+        // weight tables: 4 consecutive tile-local cells of one axis per step
+        for (int q = lane; q < np * QP; q += 64) {
+            const int k = q / QP, e = q - k * QP;
+            const int ax = D == 3 ? min(e, 2) : (e < 2 ? 0 : 1);
+            const int L0 = D == 3 ? (e == 3 ? 4 : 0) : (e < 2 ? 4 * e : 4 * (e - 2));
+            const int T = D == 3 ? (ax == 2 ? T2 : T0) : (ax == 0 ? T0 : T1);
+            float w[4] = {0.f, 0.f, 0.f, 0.f};
+            if (k < n) {
+                const int4 pa = a.pair_a[base + k], pb = a.pair_b[base + k];
+                const int l = (pa.w >> (10 * ax)) & 0x3ff, c = (pa.z >> (8 * ax)) & 0xff;
+                const int j = a.ns - ((pa.y >> (8 * ax)) & 0xff);
+                const float t = __int_as_float(ax == 0 ? pb.x : ax == 1 ? pb.y : pb.z);
+                const float coef = ax == 0 ? a.coef[0] : ax == 1 ? a.coef[1] : a.coef[2];
+                int rel0 = L0 - l; // (L - l) mod T of the quad's first cell
+                if (rel0 < 0) rel0 += T;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    int rel = rel0 + i;
+                    if (i > 0 && rel >= T) rel -= T;
+                    const float u = t + (float)(j - rel);
+                    const float g = __builtin_amdgcn_exp2f(-coef * u * u);
+                    w[i] = rel < c ? g : 0.f;
+                }
+            }
+            float *dst = D == 3 ? (e < 2 ? s_row + k * RW + 4 * e : s_sl + k * 8 + L0)
+                                : (e < 2 ? s_sl + k * 8 + L0 : s_row + k * RW + L0);
+            *(float4 *)dst = make_float4(w[0], w[1], w[2], w[3]);
+        }
+        __syncthreads();
+        f32x4 acc[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int t = 0; t < np; t += 4) {
+            float w = pa0[t * RW];
+            if (D == 3) w *= pa1[t * RW];
+            const float v = pv[t * R];
+            float b[M];
+            if constexpr (M == 4) {
+                const float4 x = *(const float4 *)(ps + t * 8);
+                b[0] = x.x * v;
+                b[1] = x.y * v;
+                b[2] = x.z * v;
+                b[3] = x.w * v;
+            } else if constexpr (M == 2) {
+                const float2 x = *(const float2 *)(ps + t * 8);
+                b[0] = x.x * v;
+                b[1] = x.y * v;
+            } else {
+                b[0] = ps[t * 8] * v;
+            }
+#pragma unroll
+            for (int m = 0; m < M; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, b[m], acc[m], 0, 0, 0);
+        }
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float y = acc[m][v] - K[m][v];
+                const float ts = S[m][v] + y;
+                K[m][v] = (ts - S[m][v]) - y;
+                S[m][v] = ts;
+            }
+    }
+    // Write-out.  Lane (ri, kg) holds re (ri even) or im (ri odd) of coil (ri % R) / 2 for
+    // slices (ri / R) M + m and row cells 4 kg + v.  Neighbouring lanes swap halves (DPP):
+    // the even lane gets row cells v = 0, 1 and the odd lane v = 2, 3 as (re, im) pairs.
+    const int c = (ri % R) >> 1;
+    const bool odd = (ri & 1) != 0;
+    const bool slot = item.w >= 0;
+    float2 o[M][2];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        float x[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[v] = S[m][v] - K[m][v];
+        // quad_perm [1, 0, 3, 2]: the value of lane ^ 1
+        const float r0 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(odd ? x[0] : x[2]), 0xb1, 0xf, 0xf, false));
+        const float r1 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(odd ? x[1] : x[3]), 0xb1, 0xf, 0xf, false));
+        o[m][0] = odd ? make_float2(r0, x[2]) : make_float2(x[0], r0);
+        o[m][1] = odd ? make_float2(r1, x[3]) : make_float2(x[1], r1);
+    }
+    if (c >= ncg) return;
+    int org[3] = {0, 0, 0}, te[3] = {T0, T1, T2};
+    if (!slot) {
+        uint32_t r = (uint32_t)item.x;
+#pragma unroll
+        for (int ax = D - 1; ax >= 0; --ax) {
+            const uint32_t nt = (uint32_t)a.ntiles[ax], qq = r % nt;
+            r /= nt;
+            org[ax] = (int)qq * (ax == 0 ? T0 : ax == 1 ? T1 : T2);
+            te[ax] = (int)min((int64_t)te[ax], a.nf[ax] - org[ax]);
+        }
+    }
+    float2 *dst = slot ? a.partial + ((int64_t)item.w * a.nc + cg0 + c) * TC : a.grid + (int64_t)(cg0 + c) * a.G;
+    const bool wide = slot || ((a.G | a.nf[D - 1]) & 1) == 0; // 16-byte pairs along the last axis
+    const int s0 = (ri / R) * M;
+    if (D == 3) {
+        // x = kg, y = 2 odd + i, z = s0 + m
+        const int64_t n1 = slot ? T1 : a.nf[1], n2 = slot ? T2 : a.nf[2];
+        if (kg >= te[0]) return;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int y = (odd ? 2 : 0) + i;
+            if (y >= te[1]) continue;
+            float2 *p = dst + ((org[0] + kg) * n1 + (org[1] + y)) * n2 + org[2] + s0;
+            if constexpr (M == 1) {
+                if (s0 < te[2]) p[0] = o[0][i];
+            } else {
+#pragma unroll
+                for (int m = 0; m < M; m += 2) {
+                    if (wide && s0 + m + 1 < te[2]) {
+                        *(float4 *)(p + m) = make_float4(o[m][i].x, o[m][i].y, o[m + 1][i].x, o[m + 1][i].y);
+                    } else {
+                        if (s0 + m < te[2]) p[m] = o[m][i];
+                        if (s0 + m + 1 < te[2]) p[m + 1] = o[m + 1][i];
+                    }
+                }
+            }
+        }
+    } else {
+        // x = s0 + m, y = 4 kg + 2 odd + i
+        const int64_t n1 = slot ? T1 : a.nf[1];
+        const int y = 4 * kg + (odd ? 2 : 0);
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            if (s0 + m >= te[0]) continue;
+            float2 *p = dst + (org[0] + s0 + m) * n1 + org[1] + y;
+            if (wide && y + 1 < te[1]) {
+                *(float4 *)p = make_float4(o[m][0].x, o[m][0].y, o[m][1].x, o[m][1].y);
+            } else {
+                if (y < te[1]) p[0] = o[m][0];
+                if (y + 1 < te[1]) p[1] = o[m][1];
+            }
+        }
+    }
+}
+
+template <int D, int R>
+__global__ __launch_bounds__(64) void k_spread_tile(SpreadArgs a)
+{
+    const uint32_t n = gridDim.x * gridDim.y;
+    const uint32_t w = xcd_swizzle(blockIdx.x + gridDim.x * blockIdx.y, n);
+    spread_tile_body<D, R>(a, a.items[w % gridDim.x], (int)(w / gridDim.x));
+}
+
+template <int D, int R>
+__global__ __launch_bounds__(64) void k_spread_tile_batch(const SpreadArgs *__restrict__ args,
+                                                                            const int4 *__restrict__ bitems)
+{
+    const int4 bi = bitems[xcd_swizzle(blockIdx.x, gridDim.x)];
+    const SpreadArgs &a = args[bi.x]; // read in place: uniform scalar loads
+    spread_tile_body<D, R>(a, a.items[bi.y], bi.z);
+}
+
+// ---------------------------------------------------------------------------
+// Adjoint spread in 2-D on 4 x 4 sub-blocks (v_mfma_f32_16x16x4_f32).
+//
+// Default 8 x 16 tiles, four waves: wave q takes y cells 4 q .. 4 q + 3, as two 4 x 4
+// sub-blocks, and 8 NG coils.  Per batch of 64 pairs a wave lists the pairs whose windows
+// reach each sub-block; 4 listed pairs take one weight product wx wy per lane (row = cell)
+// and NG matrix products whose columns are the reals of 8 coils.  A window of 6 cells
+// fills 0.44 of a 4 x 4 block it reaches, against 0.22 of an 8 x 8 block, so the products
+// are half of k_spread_mfma's; the tables and records serve up to 32 coils.
+// Bound by the matrix cores and, at few coils, by the latency of the batches: 256^2, 98304
+// spiral samples, nspread 3, with equal work items: 32 coils 107 -> 82 us, 8 coils
+// 43 -> 36 us.
+// LDS rows, one per pair: weights x[8] y[16] | reals [16 NG]; row B is zero (list padding).
+// ---------------------------------------------------------------------------
+constexpr int kSpreadSubWaves = 4;
+constexpr int spread_sub_row(int NG) { return 24 + 16 * NG; }
+
+inline size_t spread_sub_lds(int NG)
+{
+    return (size_t)(kSpreadBatch + 1) * spread_sub_row(NG) * 4 + (size_t)kSpreadBatch * 4 +
+           (size_t)kSpreadSubWaves * 2 * kSpreadBatch * 4;
+}
+
+template <int NG>
+__device__ __forceinline__ void spread_sub_body(const SpreadArgs &a, const int4 item, const int cgi)
+{
+    constexpr int B = kSpreadBatch, ROW = spread_sub_row(NG), NC = 8 * NG, NT = 64 * kSpreadSubWaves;
+    constexpr int T0 = 8, T1 = 16, TC = 128;
+    extern __shared__ float lds_sp[];
+    if (tile_skippable(a, item)) return; // uniform over the workgroup
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int *s_msk = (int *)(lds_sp + (B + 1) * ROW);
+    int *s_list = s_msk + B + wave * 2 * B;
+    const int cg0 = cgi * NC;
+    const int ncg = (int)min((int64_t)NC, a.nc - cg0);
+    const int ri = lane & 15, kg = lane >> 4;
+    // coil-last with an even coil count: a pair's coils are 16-byte pairs
+    const bool v4 = a.layout == GN_COIL_LAST && ((a.nc | cg0) & 1) == 0 && (reinterpret_cast<uintptr_t>(a.in) & 15) == 0;
+    const char *qx = (const char *)(lds_sp + (ri >> 2)), *qy = (const char *)(lds_sp + 8 + 4 * wave + (ri & 3));
+    const char *qv = (const char *)(lds_sp + 24 + ri);
+    for (int i = tid; i < ROW; i += NT) lds_sp[B * ROW + i] = 0.f;
+    float S[2][NG][4], K[2][NG][4];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) S[s][g][v] = K[s][g][v] = 0.f;
+    for (int base = item.y; base < item.z; base += B) {
+        const int n = min(B, item.z - base);
+        if (base != item.y) __syncthreads(); // previous batch fully consumed (uniform)
+        // values: one 16-byte coil pair per step
+        for (int q = tid; q < n * (NC / 2); q += NT) {
+            const int k = q / (NC / 2), c = 2 * (q - k * (NC / 2));
+            const int orig = a.pair_a[base + k].x;
+            const float scale = a.use_dcf ? __int_as_float(a.pair_b[base + k].w) : 1.0f;
+            float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (v4) {
+                if (c < ncg) t = *reinterpret_cast<const float4 *>(a.in + (int64_t)orig * a.nc + cg0 + c);
+            } else {
+                float2 x = make_float2(0.f, 0.f), y = x;
+                if (c < ncg) x = a.layout == GN_COIL_LAST ? a.in[(int64_t)orig * a.nc + cg0 + c] : a.in[(int64_t)(cg0 + c) * a.M + orig];
+                if (c + 1 < ncg) y = a.layout == GN_COIL_LAST ? a.in[(int64_t)orig * a.nc + cg0 + c + 1] : a.in[(int64_t)(cg0 + c + 1) * a.M + orig];
+                t = make_float4(x.x, x.y, y.x, y.y);
+            }
+            *(float4 *)(lds_sp + k * ROW + 24 + 2 * c) = make_float4(t.x * scale, t.y * scale, t.z * scale, t.w * scale);
+        }
+        // weight tables: 4 consecutive tile-local cells of one axis per step; the first
+        // step of a pair also forms its sub-block masks (x halves | y quarters << 2)
+        for (int q = tid; q < n * 6; q += NT) {
+            const int k = q / 6, e = q - k * 6, ax = e < 2 ? 0 : 1;
+            const int L0 = 4 * (ax ? e - 2 : e), T = ax ? T1 : T0;
+            const int4 pa = a.pair_a[base + k], pb = a.pair_b[base + k];
+            const int l = (pa.w >> (10 * ax)) & 0x3ff, c = (pa.z >> (8 * ax)) & 0xff;
+            const int j = a.ns - ((pa.y >> (8 * ax)) & 0xff);
+            const float t = __int_as_float(ax ? pb.y : pb.x), coef = ax ? a.coef[1] : a.coef[0];
+            int rel0 = L0 - l; // (L - l) mod T of the quad's first cell
+            if (rel0 < 0) rel0 += T;
+            float w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                int rel = rel0 + i;
+                if (i > 0 && rel >= T) rel -= T;
+                const float u = t + (float)(j - rel);
+                const float g = __builtin_amdgcn_exp2f(-coef * u * u);
+                w[i] = rel < c ? g : 0.f;
+            }
+            *(float4 *)(lds_sp + k * ROW + 4 * e) = make_float4(w[0], w[1], w[2], w[3]);
+            if (e == 0) {
+                uint32_t h = 0;
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    const int lx = x ? (pa.w >> 10) & 0x3ff : pa.w & 0x3ff, cx = x ? (pa.z >> 8) & 0xff : pa.z & 0xff;
+                    const int Tx = x ? T1 : T0;
+                    uint64_t m = ((1ull << cx) - 1) << lx; // window cells (L - l) mod T < c
+                    m = (m | (m >> Tx)) & ((1ull << Tx) - 1);
+#pragma unroll
+                    for (int b = 0; b < (x ? 4 : 2); ++b)
+                        if ((m >> (4 * b)) & 0xf) h |= 1u << ((x ? 2 : 0) + b);
+                }
+                s_msk[k] = (int)h;
+            }
+        }
+        __syncthreads();
+        const uint32_t h = lane < n ? (uint32_t)s_msk[lane] : 0u;
+        const bool hy = (h >> (2 + wave)) & 1u;
+        int cnt[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const bool hit = hy && ((h >> s) & 1u);
+            const unsigned long long hm = __ballot(hit);
+            cnt[s] = __popcll(hm);
+            const int pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0));
+            if (hit) s_list[s * B + pos] = lane * (ROW * 4);
+            if (lane >= cnt[s] && lane < ((cnt[s] + 3) & ~3)) s_list[s * B + lane] = B * (ROW * 4);
+        }
+        // the lists were written by this wave's own lanes: order the LDS accesses
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            f32x4 acc[NG];
+#pragma unroll
+            for (int g = 0; g < NG; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const int *lst = s_list + s * B + kg;
+            for (int t = 0; t < cnt[s]; t += 4) {
+                const int off = lst[t]; // byte offset of the pair's row
+                const float w = *(const float *)(qx + 16 * s + off) * *(const float *)(qy + off);
+#pragma unroll
+                for (int g = 0; g < NG; ++g)
+                    acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, *(const float *)(qv + 64 * g + off), acc[g], 0, 0, 0);
+            }
+#pragma unroll
+            for (int g = 0; g < NG; ++g)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float y = acc[g][v] - K[s][g][v];
+                    const float ts = S[s][g][v] + y;
+                    K[s][g][v] = (ts - S[s][g][v]) - y;
+                    S[s][g][v] = ts;
+                }
+        }
+    }
+    // Write-out.  Lane (ri, kg) holds re (ri even) or im (ri odd) of coil 8 g + ri / 2 for
+    // the cells x = 4 s + kg, y = 4 wave + v.  Neighbouring lanes swap halves (DPP): the
+    // even lane gets cells v = 0, 1 and the odd lane v = 2, 3 as (re, im) pairs.
+    const bool odd = (ri & 1) != 0;
+    const bool slot = item.w >= 0;
+    int org0 = 0, org1 = 0, te0 = T0, te1 = T1;
+    if (!slot) {
+        const uint32_t t1 = (uint32_t)item.x % (uint32_t)a.ntiles[1], t0 = (uint32_t)item.x / (uint32_t)a.ntiles[1];
+        org0 = (int)t0 * T0;
+        org1 = (int)t1 * T1;
+        te0 = (int)min((int64_t)T0, a.nf[0] - org0);
+        te1 = (int)min((int64_t)T1, a.nf[1] - org1);
+    }
+    const bool wide = slot || ((a.G | a.nf[1]) & 1) == 0; // 16-byte pairs of cells
+    const int64_t n1 = slot ? T1 : a.nf[1];
+    const int y = 4 * wave + (odd ? 2 : 0);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const int x = 4 * s + kg;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            float o[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o[v] = S[s][g][v] - K[s][g][v];
+            // quad_perm [1, 0, 3, 2]: the value of lane ^ 1
+            const float r0 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(odd ? o[0] : o[2]), 0xb1, 0xf, 0xf, false));
+            const float r1 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(odd ? o[1] : o[3]), 0xb1, 0xf, 0xf, false));
+            const float4 w = odd ? make_float4(r0, o[2], r1, o[3]) : make_float4(o[0], r0, o[1], r1);
+            const int c = 8 * g + (ri >> 1);
+            if (c >= ncg || x >= te0) continue;
+            float2 *p = (slot ? a.partial + ((int64_t)item.w * a.nc + cg0 + c) * TC : a.grid + (int64_t)(cg0 + c) * a.G) +
+                        (org0 + x) * n1 + org1 + y;
+            if (wide && y + 1 < te1) {
+                *(float4 *)p = w;
+            } else {
+                if (y < te1) p[0] = make_float2(w.x, w.y);
+                if (y + 1 < te1) p[1] = make_float2(w.z, w.w);
+            }
+        }
+    }
+}
+
+template <int NG>
+__global__ __launch_bounds__(64 * kSpreadSubWaves) void k_spread_sub(SpreadArgs a)
+{
+    const uint32_t n = gridDim.x * gridDim.y;
+    const uint32_t w = xcd_swizzle(blockIdx.x + gridDim.x * blockIdx.y, n);
+    spread_sub_body<NG>(a, a.items[w % gridDim.x], (int)(w / gridDim.x));
+}
+
+template <int NG>
+__global__ __launch_bounds__(64 * kSpreadSubWaves) void k_spread_sub_batch(const SpreadArgs *__restrict__ args,
+                                                                           const int4 *__restrict__ bitems)
+{
+    const int4 bi = bitems[xcd_swizzle(blockIdx.x, gridDim.x)];
+    const SpreadArgs &a = args[bi.x]; // read in place: uniform scalar loads
+    spread_sub_body<NG>(a, a.items[bi.y], bi.z);
+}
+
+// Kahan-compensated sum of the partial tiles of each split tile, in slice order; one
+// thread per (coil, cell) of a tile, blockIdx.y over its cells of every coil (as one block
+// of 1024 threads per tile: 27 instead of 11 us at 32 coils and 256^2).
+constexpr int kReduceThreads = 256;
+constexpr int kReduceBlocks = 16; // blocks per tile at most
 template <int D>
 __device__ __forceinline__ void spread_reduce_body(const SpreadArgs &a, const int4 it)
 {
@@ -1218,7 +1662,7 @@ __device__ __forceinline__ void spread_reduce_body(const SpreadArgs &a, const in
     const int TC = a.TC;
     const int T1 = a.tile[1], T2 = (D == 3) ? a.tile[2] : 1;
     const int ne = (int)(TC * a.nc); // a tile's cells of every coil (< 2^31)
-    for (int e = threadIdx.x; e < ne; e += blockDim.x) {
+    for (int e = blockIdx.y * blockDim.x + threadIdx.x; e < ne; e += blockDim.x * gridDim.y) {
         const int64_t coil = e / TC;
         const int cidx = e - (int)coil * TC;
         int x0, x1, x2 = 0;
@@ -2131,6 +2575,18 @@ __global__ __launch_bounds__(kGatherThreads) void k_bank_order(GatherArgs a, int
         if (e_ != hipSuccess) return hip_fail(e_, #call);                                                              \
     } while (0)
 
+// Pairs per spread work item, at most kSpreadChunk.  A launch lasts as long as its longest
+// item, eight batches of 64 at kSpreadChunk, so smaller spreads take shorter items; the
+// partial tiles cost more than that saves once the items fill the chip many times over.
+// Items of 512 / 192 / 128 pairs: 43 k pairs (192^2, 8 coils) 36 / 24 / 22 us, 209 k pairs
+// (256^2 spiral, 8 coils) 50 / 36 / 38 us, 1.1 M pairs (64^3, 4 coils) 107 / 83 / 82 us,
+// 2.9 M pairs (64^3, 8 coils) 202 / 225 / 268 us.
+int spread_chunk(int64_t pairs)
+{
+    static_assert(kSpreadChunk >= 192, "shorter items than the longest");
+    return pairs >= (1 << 21) ? kSpreadChunk : pairs >= (1 << 17) ? 192 : 128;
+}
+
 int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const void *z, int coord_f64, double df,
                  const float *dcf)
 {
@@ -2238,7 +2694,8 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
     // their counts come back with the gather bin offsets in one synchronisation
     {
         const int64_t P = R.npairs;
-        const int64_t cap_items = K + P / kSpreadChunk + 1, cap_red = std::min<int64_t>(K, P / kSpreadChunk + 1);
+        const int chunk = spread_chunk(P);
+        const int64_t cap_items = K + P / chunk + 1, cap_red = std::min<int64_t>(K, P / chunk + 1);
         const int64_t ncolt = (int64_t)g.ntiles[1] * g.ntiles[2];
         if ((rc = grow_alloc(&R.spread_items, &R.spread_items_cap, (size_t)cap_items, "work items")) ||
             (rc = grow_alloc(&R.reduce_items, &R.reduce_items_cap, (size_t)cap_red, "work items")) ||
@@ -2253,13 +2710,13 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
             (rc = sc.alloc(&bs, (size_t)nbk + 1, "work items")) || (rc = sc.alloc(&br, (size_t)nbk + 1, "work items")))
             return rc;
         const dim3 gk(grid_blocks(K, 256, INT32_MAX));
-        hipLaunchKernelGGL(k_item_counts, gk, dim3(256), 0, st, K, tile_pairs, kSpreadChunk, ni, ne, ns, nr);
+        hipLaunchKernelGGL(k_item_counts, gk, dim3(256), 0, st, K, tile_pairs, chunk, ni, ne, ns, nr);
         GN_HIP(hipGetLastError());
         GN_HIP(device_scan(ni, K, bi, st));
         GN_HIP(device_scan(ne, K, be, st));
         GN_HIP(device_scan(ns, K, bs, st));
         GN_HIP(device_scan(nr, K, br, st));
-        hipLaunchKernelGGL(k_item_write, gk, dim3(256), 0, st, K, tile_pairs, kSpreadChunk, ni, ne, bi + nbk, ns, nr,
+        hipLaunchKernelGGL(k_item_write, gk, dim3(256), 0, st, K, tile_pairs, chunk, ni, ne, bi + nbk, ns, nr,
                            R.spread_items, R.reduce_items);
         GN_HIP(hipGetLastError());
         R.mask_k = (g.ntiles[0] + 63) / 64;
@@ -2347,25 +2804,50 @@ inline size_t spread_lds_bytes(const SpreadArgs &a, int ncg)
 // the dispatch-order arithmetic of the spread and gather kernels is 32-bit
 inline bool grid_ok(dim3 g) { return (uint64_t)g.x * g.y * g.z < (1ull << 31); }
 
-template <int D, int NCG>
-hipError_t spread_launch(const SpreadArgs &a, int nitems, int64_t nc, hipStream_t st)
+enum { kSpreadValu = 0, kSpreadMfma = 1, kSpreadTile = 2, kSpreadSub = 3 };
+
+} // namespace
+
+// Kernel and launch shape of a spread.  Default tiles: k_spread_tile for up to 2 coils in
+// 2-D and 4 in 3-D, k_spread_sub for more in 2-D.  3-D with 5 and more coils, and other
+// block-aligned tiles, take k_spread_mfma (128^3, 1,048,576 samples, nspread 3: 4 coils
+// 499 -> 459 us with k_spread_tile, but 8 coils 571 -> 763 us: its products fill the
+// matrix cores without skipping half tiles).  Any other tile takes k_spread.
+SpreadShape spread_shape(const SpreadArgs &a, int dim)
 {
-    const int ng = (int)((nc + NCG - 1) / NCG);
-    const int nb = a.nblk[0] * a.nblk[1] * (D == 3 ? a.nblk[2] : 1);
-    const int waves = std::min(nb, kSpreadWavesMax);
-    const int nbg = (nb + waves - 1) / waves;
-    if (nitems == 0) return hipSuccess;
-    const dim3 grid((unsigned)nitems, (unsigned)ng, (unsigned)nbg);
-    if (!grid_ok(grid)) return hipErrorInvalidConfiguration;
-    if (mfma_tiles_ok(a, D)) {
-        const size_t lds = spread_mfma_lds_bytes(a, waves);
-        lds_limit(k_spread_mfma<D, NCG>, lds);
-        hipLaunchKernelGGL((k_spread_mfma<D, NCG>), grid, dim3(64 * waves), lds, st, a);
-    } else {
-        const size_t lds = spread_lds_bytes(a, NCG);
-        lds_limit(k_spread<D, NCG>, lds);
-        hipLaunchKernelGGL((k_spread<D, NCG>), grid, dim3(64 * waves), lds, st, a);
+    SpreadShape s;
+    const bool tile = dim == 3 ? a.tile[0] == 4 && a.tile[1] == 4 && a.tile[2] == 8 : a.tile[0] == 8 && a.tile[1] == 16;
+    if (tile && dim == 2 && a.nc > 2 && mfma_tiles_ok(a, dim)) {
+        s.kind = kSpreadSub;
+        s.width = a.nc <= 8 ? 1 : 2; // 16 coils per workgroup; 32 took 132 registers: 96 -> 82 us at 32 coils
+        s.waves = kSpreadSubWaves;
+        s.coils = 8 * s.width;
+        s.lds = spread_sub_lds(s.width);
+        return s;
     }
+    if (tile && a.nc <= 4 && mfma_tiles_ok(a, dim)) {
+        s.kind = kSpreadTile;
+        s.width = a.nc == 1 ? 2 : a.nc == 2 ? 4 : 8;
+        s.coils = s.width / 2;
+        s.lds = spread_tile_lds(dim, s.width);
+        return s;
+    }
+    s.coils = s.width = spread_coil_group(a.nc);
+    const int nb = a.nblk[0] * a.nblk[1] * (dim == 3 ? a.nblk[2] : 1);
+    s.waves = std::min(nb, kSpreadWavesMax);
+    s.nbg = (nb + s.waves - 1) / s.waves;
+    s.kind = mfma_tiles_ok(a, dim) ? kSpreadMfma : kSpreadValu;
+    s.lds = s.kind == kSpreadMfma ? spread_mfma_lds_bytes(a, s.waves) : spread_lds_bytes(a, s.width);
+    return s;
+}
+
+namespace {
+
+template <typename K>
+hipError_t spread_go(K kernel, dim3 grid, const SpreadShape &sh, const SpreadArgs &a, hipStream_t st)
+{
+    lds_limit(kernel, sh.lds);
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * sh.waves), sh.lds, st, a);
     return hipGetLastError();
 }
 
@@ -2373,15 +2855,32 @@ template <int D>
 hipError_t spread_dispatch(const SpreadArgs &a, int nitems, int nritems, const int4 *ritems, int64_t nc,
                            hipStream_t st)
 {
-    hipError_t e;
-    switch (spread_coil_group(nc)) {
-    case 8: e = spread_launch<D, 8>(a, nitems, nc, st); break;
-    case 4: e = spread_launch<D, 4>(a, nitems, nc, st); break;
-    case 2: e = spread_launch<D, 2>(a, nitems, nc, st); break;
-    default: e = spread_launch<D, 1>(a, nitems, nc, st); break;
+    const SpreadShape sh = spread_shape(a, D);
+    const dim3 grid((unsigned)nitems, (unsigned)((nc + sh.coils - 1) / sh.coils), (unsigned)sh.nbg);
+    if (!grid_ok(grid)) return hipErrorInvalidConfiguration;
+    hipError_t e = hipSuccess;
+    if (nitems > 0) {
+        switch (sh.kind * 16 + sh.width) {
+        case kSpreadSub * 16 + 1: e = spread_go(k_spread_sub<1>, grid, sh, a, st); break;
+        case kSpreadSub * 16 + 2: e = spread_go(k_spread_sub<2>, grid, sh, a, st); break;
+        case kSpreadTile * 16 + 8: e = spread_go(k_spread_tile<3, 8>, grid, sh, a, st); break; // 3-D only
+        case kSpreadTile * 16 + 4: e = spread_go(k_spread_tile<D, 4>, grid, sh, a, st); break;
+        case kSpreadTile * 16 + 2: e = spread_go(k_spread_tile<D, 2>, grid, sh, a, st); break;
+        case kSpreadMfma * 16 + 8: e = spread_go(k_spread_mfma<D, 8>, grid, sh, a, st); break;
+        case kSpreadMfma * 16 + 4: e = spread_go(k_spread_mfma<D, 4>, grid, sh, a, st); break;
+        case kSpreadMfma * 16 + 2: e = spread_go(k_spread_mfma<D, 2>, grid, sh, a, st); break;
+        case kSpreadMfma * 16 + 1: e = spread_go(k_spread_mfma<D, 1>, grid, sh, a, st); break;
+        case kSpreadValu * 16 + 8: e = spread_go(k_spread<D, 8>, grid, sh, a, st); break;
+        case kSpreadValu * 16 + 4: e = spread_go(k_spread<D, 4>, grid, sh, a, st); break;
+        case kSpreadValu * 16 + 2: e = spread_go(k_spread<D, 2>, grid, sh, a, st); break;
+        case kSpreadValu * 16 + 1: e = spread_go(k_spread<D, 1>, grid, sh, a, st); break;
+        default: return hipErrorInvalidValue;
+        }
     }
     if (e == hipSuccess && nritems > 0) {
-        hipLaunchKernelGGL(k_spread_reduce<D>, dim3((unsigned)nritems), dim3(kReduceThreads), 0, st, a, ritems);
+        const int64_t nb = std::min<int64_t>(kReduceBlocks, (a.TC * nc + kReduceThreads - 1) / kReduceThreads);
+        hipLaunchKernelGGL(k_spread_reduce<D>, dim3((unsigned)nritems, (unsigned)nb), dim3(kReduceThreads), 0, st, a,
+                           ritems);
         e = hipGetLastError();
     }
     return e;
@@ -2682,36 +3181,36 @@ int launch_sense_combine(gn_plan_s *p, const float2 *coil_images, float2 *image)
 // Batched launchers: one launch per stage over the work of many plans.
 // ---------------------------------------------------------------------------
 
-void spread_shape(const SpreadArgs &a, int dim, int *waves, int *nbg)
-{
-    const int nb = a.nblk[0] * a.nblk[1] * (dim == 3 ? a.nblk[2] : 1);
-    *waves = std::min(nb, kSpreadWavesMax);
-    *nbg = (nb + *waves - 1) / *waves;
-}
-
-bool spread_uses_mfma(const SpreadArgs &a, int dim) { return mfma_tiles_ok(a, dim); }
-
-size_t spread_lds(const SpreadArgs &a, int ncg, bool mfma, int waves)
-{
-    return mfma ? spread_mfma_lds_bytes(a, waves) : spread_lds_bytes(a, ncg);
-}
-
 namespace {
-template <int D, int NCG>
-hipError_t spread_batch_launch(bool mfma, const SpreadArgs *d_args, const int4 *d_items, int n, int waves, int nbg,
-                               size_t lds, hipStream_t st)
+template <typename K>
+hipError_t spread_batch_go(K kernel, const SpreadShape &sh, const SpreadArgs *d_args, const int4 *d_items, int n,
+                           hipStream_t st)
 {
-    if (!grid_ok(dim3((unsigned)n, (unsigned)nbg))) return hipErrorInvalidConfiguration;
-    if (mfma) {
-        lds_limit(k_spread_mfma_batch<D, NCG>, lds);
-        hipLaunchKernelGGL((k_spread_mfma_batch<D, NCG>), dim3((unsigned)n, (unsigned)nbg), dim3(64 * waves), lds, st,
-                           d_args, d_items);
-    } else {
-        lds_limit(k_spread_batch<D, NCG>, lds);
-        hipLaunchKernelGGL((k_spread_batch<D, NCG>), dim3((unsigned)n, (unsigned)nbg), dim3(64 * waves), lds, st,
-                           d_args, d_items);
-    }
+    lds_limit(kernel, sh.lds);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)n, (unsigned)sh.nbg), dim3(64 * sh.waves), sh.lds, st, d_args, d_items);
     return hipGetLastError();
+}
+
+template <int D>
+hipError_t spread_batch_dispatch(const SpreadShape &sh, const SpreadArgs *d_args, const int4 *d_items, int n,
+                                 hipStream_t st)
+{
+    switch (sh.kind * 16 + sh.width) {
+    case kSpreadSub * 16 + 1: return spread_batch_go(k_spread_sub_batch<1>, sh, d_args, d_items, n, st);
+    case kSpreadSub * 16 + 2: return spread_batch_go(k_spread_sub_batch<2>, sh, d_args, d_items, n, st);
+    case kSpreadTile * 16 + 8: return spread_batch_go(k_spread_tile_batch<3, 8>, sh, d_args, d_items, n, st); // 3-D only
+    case kSpreadTile * 16 + 4: return spread_batch_go(k_spread_tile_batch<D, 4>, sh, d_args, d_items, n, st);
+    case kSpreadTile * 16 + 2: return spread_batch_go(k_spread_tile_batch<D, 2>, sh, d_args, d_items, n, st);
+    case kSpreadMfma * 16 + 8: return spread_batch_go(k_spread_mfma_batch<D, 8>, sh, d_args, d_items, n, st);
+    case kSpreadMfma * 16 + 4: return spread_batch_go(k_spread_mfma_batch<D, 4>, sh, d_args, d_items, n, st);
+    case kSpreadMfma * 16 + 2: return spread_batch_go(k_spread_mfma_batch<D, 2>, sh, d_args, d_items, n, st);
+    case kSpreadMfma * 16 + 1: return spread_batch_go(k_spread_mfma_batch<D, 1>, sh, d_args, d_items, n, st);
+    case kSpreadValu * 16 + 8: return spread_batch_go(k_spread_batch<D, 8>, sh, d_args, d_items, n, st);
+    case kSpreadValu * 16 + 4: return spread_batch_go(k_spread_batch<D, 4>, sh, d_args, d_items, n, st);
+    case kSpreadValu * 16 + 2: return spread_batch_go(k_spread_batch<D, 2>, sh, d_args, d_items, n, st);
+    case kSpreadValu * 16 + 1: return spread_batch_go(k_spread_batch<D, 1>, sh, d_args, d_items, n, st);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 template <int D, int NS>
@@ -2731,35 +3230,22 @@ hipError_t gather_batch_dispatch(bool wrap, const GatherArgs *d_args, const int4
 }
 } // namespace
 
-hipError_t launch_spread_batch(int dim, int ncg, bool mfma, const SpreadArgs *d_args, const int4 *d_items, int n,
-                               int waves, int nbg, size_t lds, hipStream_t st)
+hipError_t launch_spread_batch(int dim, const SpreadShape &sh, const SpreadArgs *d_args, const int4 *d_items, int n,
+                               hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
-    if (dim == 3) {
-        switch (ncg) {
-        case 8: return spread_batch_launch<3, 8>(mfma, d_args, d_items, n, waves, nbg, lds, st);
-        case 4: return spread_batch_launch<3, 4>(mfma, d_args, d_items, n, waves, nbg, lds, st);
-        case 2: return spread_batch_launch<3, 2>(mfma, d_args, d_items, n, waves, nbg, lds, st);
-        case 1: return spread_batch_launch<3, 1>(mfma, d_args, d_items, n, waves, nbg, lds, st);
-        }
-    } else {
-        switch (ncg) {
-        case 8: return spread_batch_launch<2, 8>(mfma, d_args, d_items, n, waves, nbg, lds, st);
-        case 4: return spread_batch_launch<2, 4>(mfma, d_args, d_items, n, waves, nbg, lds, st);
-        case 2: return spread_batch_launch<2, 2>(mfma, d_args, d_items, n, waves, nbg, lds, st);
-        case 1: return spread_batch_launch<2, 1>(mfma, d_args, d_items, n, waves, nbg, lds, st);
-        }
-    }
-    return hipErrorInvalidValue;
+    if (!grid_ok(dim3((unsigned)n, (unsigned)sh.nbg))) return hipErrorInvalidConfiguration;
+    return dim == 3 ? spread_batch_dispatch<3>(sh, d_args, d_items, n, st)
+                    : spread_batch_dispatch<2>(sh, d_args, d_items, n, st);
 }
 
 hipError_t launch_spread_reduce_batch(int dim, const SpreadArgs *d_args, const int4 *d_items, int n, hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
     if (dim == 3)
-        hipLaunchKernelGGL(k_spread_reduce_batch<3>, dim3((unsigned)n), dim3(kReduceThreads), 0, st, d_args, d_items);
+        hipLaunchKernelGGL(k_spread_reduce_batch<3>, dim3((unsigned)n, 4), dim3(kReduceThreads), 0, st, d_args, d_items);
     else
-        hipLaunchKernelGGL(k_spread_reduce_batch<2>, dim3((unsigned)n), dim3(kReduceThreads), 0, st, d_args, d_items);
+        hipLaunchKernelGGL(k_spread_reduce_batch<2>, dim3((unsigned)n, 4), dim3(kReduceThreads), 0, st, d_args, d_items);
     return hipGetLastError();
 }
 

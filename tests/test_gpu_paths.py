@@ -150,3 +150,30 @@ def test_tv_extreme_values():
         x[3, 4] = bad
         got = S.prox_tv2d_r(torch.as_tensor(x).cuda(), 0.3, niter=2).cpu().numpy()
         assert np.isfinite(got[10:, 12:]).all() and not np.isfinite(got[3, 4])
+
+
+@pytest.mark.parametrize("modes,ns", [((4, 8), 3), ((21, 9), 3), ((30, 25), 5), ((4, 4, 4), 2), ((5, 9, 7), 3),
+                                      ((10, 6, 13), 4)])
+@pytest.mark.parametrize("nc,layout", [(1, "coil_last"), (2, "coil_major"), (4, "coil_last"), (3, "coil_major"),
+                                       (17, "coil_last")])
+def test_spread_tiles(modes, ns, nc, layout):
+    """Axes of one tile, ragged last tiles and rows of odd length, both layouts, samples in a
+    cluster (tiles of several work items) and spread out, with density weights: type 1 and
+    the spread alone (every tile written)."""
+    from mripy_amd.plan import Plan
+    print("case: spread tiles", modes, ns, nc, layout, flush=True)
+    rng = np.random.default_rng(nc + sum(modes))
+    M = 700
+    coords = [np.concatenate([0.02 * rng.standard_normal(400) + 0.4, np.pi * (2 * rng.random(300) - 1)]).astype(np.float32)
+              for _ in modes]
+    y, dcf = _cnormal(rng, (M, nc)), rng.random(M).astype(np.float32)
+    P = Plan(modes, ncoils=nc, rat=2, nspread=ns, layout=layout).set_points(coords, dcf=dcf)
+    p = O.Params(modes, rat=2, nspread=ns)
+    c64 = [c.astype(np.float64) for c in coords]
+    yl = y if layout == "coil_last" else np.ascontiguousarray(y.T)
+    want = O.type1(c64, dcf[:, None].astype(np.float64) * y, p)
+    got = P.type1(yl)
+    assert rel(got if layout == "coil_last" else np.moveaxis(got, 0, -1), want) <= TOL
+    grid = P.grid_spread(yl)
+    ref = np.moveaxis(O.spread(c64, y.astype(np.complex128), p.nf, p.ns, p.tau), -1, 0)
+    assert rel(grid, ref) <= TOL
