@@ -289,9 +289,11 @@ int plan_create_impl(int dim, const int64_t *modes, int rat, int nspread, int if
         return fail(GN_ENOMEM, "hipMalloc failed for the oversampled grid");
     }
     hipError_t e = hipMemcpy(p->deap, deap.data(), deap.size() * sizeof(float), hipMemcpyHostToDevice);
+    const int none = 0;
+    if (e == hipSuccess) e = hipMemcpy(p->err_flag, &none, sizeof(int), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         gn_plan_destroy(p);
-        return hip_fail(e, "deapodization upload");
+        return hip_fail(e, "plan tables upload");
     }
     if (with_grid) {
         p->fft_custom = true;

@@ -265,7 +265,8 @@ struct gn_plan_s {
     float2 *sbuf = nullptr;   // N * nc coil images of a SENSE combine that does not fit one block
     int64_t ybuf_cap = 0;
     float *deap = nullptr;    // concatenated per-axis exp(tau k^2) tables
-    int *err_flag = nullptr;  // device flag set by set_points on bad coordinates
+    int *err_flag = nullptr;  // device: number of the last set_points that met bad coordinates
+    int points_seq = 0;       // number of set_points calls
 
     // FFT engine: the pruned in-place passes (gn_fft.hip) when they cover every nf
     // (fft_custom), else rocFFT; GN_FFT_ROCFFT forces rocFFT

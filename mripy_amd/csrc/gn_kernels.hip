@@ -140,7 +140,8 @@ struct PrepArgs {
     int ntiles[3];
     int4 *cell;
     float4 *frac;
-    int *err;
+    int *err; // set to seq, this call's number, on a non-finite coordinate
+    int seq;
 };
 
 __global__ __launch_bounds__(256) void k_prep(PrepArgs a)
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a)
         double x = a.coord_f64 ? ((const double *)a.x[ax])[i] : (double)((const float *)a.x[ax])[i];
         x = x * a.df;
         if (!isfinite(x)) {
-            atomicOr(a.err, 1);
+            *a.err = a.seq; // every such thread stores the same value
             x = 0.0;
         }
         double xi, dummy;
@@ -173,91 +174,152 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Device exclusive scan of ints (local scans, one block over the block sums, add)
+// Device exclusive scans in one launch: every block scans its tile in place and publishes
+// its total; the block that takes the last ticket scans the totals (bsum[nb] = the grand
+// total) and may return values to the host through mapped pinned memory.  Consumers add
+// the block's offset themselves: offset of i = data[i] + bsum[i / kScanTile].  No block
+// waits for another.  A scan was three launches (local, totals, add) and each returned
+// value a copy: 13056 samples in 2-D took 41 launches and 8 copies, 294 us; now 17 launches,
+// 140 us (1,048,576 samples in 3-D at nspread 3: 950 -> 641 us).
 // ---------------------------------------------------------------------------
 
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
+constexpr int kItemTile = kScanThreads * 4; // tiles per block of the work-item scan
 
-// exclusive scan of v over the 256 threads of the block; returns the block total
-__device__ inline int block_exclusive_scan(int v, int *lds, int *total)
+// Exclusive scan of N ints per thread over the 256 threads of the block (all threads call
+// it); total is the block's.
+template <int N>
+__device__ inline void block_exclusive_scan(int (&x)[N], int (&total)[N])
 {
-    const int tid = threadIdx.x;
-    lds[tid] = v;
-    __syncthreads();
-    for (int off = 1; off < kScanThreads; off <<= 1) {
-        int add = tid >= off ? lds[tid - off] : 0;
-        __syncthreads();
-        lds[tid] += add;
-        __syncthreads();
-    }
-    int incl = lds[tid];
-    *total = lds[kScanThreads - 1];
-    __syncthreads();
-    return incl - v;
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_scan_local(int *__restrict__ data, int64_t n, int *__restrict__ bsum)
-{
-    __shared__ int lds[kScanThreads];
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-    int v[kScanItems];
-    int sum = 0;
+    __shared__ int s_wave[N][kScanThreads / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int inc[N];
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        v[k] = (base + k < n) ? data[base + k] : 0;
-        sum += v[k];
-    }
-    int total;
-    int run = block_exclusive_scan(sum, lds, &total);
+    for (int c = 0; c < N; ++c) {
+        int v = x[c];
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-        if (base + k < n) data[base + k] = run;
-        run += v[k];
-    }
-    if (threadIdx.x == 0) bsum[blockIdx.x] = total;
-}
-
-// single block: exclusive scan of the block sums; bsum[nb] receives the grand total
-__global__ __launch_bounds__(kScanThreads) void k_scan_bsums(int *__restrict__ bsum, int64_t nb)
-{
-    __shared__ int lds[kScanThreads];
-    int carry = 0;
-    for (int64_t b0 = 0; b0 < nb; b0 += kScanTile) {
-        const int64_t base = b0 + (int64_t)threadIdx.x * kScanItems;
-        int v[kScanItems];
-        int sum = 0;
-#pragma unroll
-        for (int k = 0; k < kScanItems; ++k) {
-            v[k] = (base + k < nb) ? bsum[base + k] : 0;
-            sum += v[k];
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(v, o, 64);
+            if (lane >= o) v += u;
         }
-        int total;
-        int run = block_exclusive_scan(sum, lds, &total) + carry;
-#pragma unroll
-        for (int k = 0; k < kScanItems; ++k) {
-            if (base + k < nb) bsum[base + k] = run;
-            run += v[k];
-        }
-        carry += total;
+        inc[c] = v;
+        if (lane == 63) s_wave[c][wave] = v;
     }
-    if (threadIdx.x == 0) bsum[nb] = carry;
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+        int before = 0, all = 0;
+        for (int w = 0; w < kScanThreads / 64; ++w) {
+            const int t = s_wave[c][w];
+            before += w < wave ? t : 0;
+            all += t;
+        }
+        x[c] = inc[c] - x[c] + before;
+        total[c] = all;
+    }
+    __syncthreads(); // s_wave may be written again
 }
 
-__global__ __launch_bounds__(kScanThreads) void k_scan_add(int *__restrict__ data, int64_t n,
-                                                            const int *__restrict__ bsum)
+// Publish this block's totals and, in the block that finishes last, turn all of them into
+// exclusive offsets; bsum holds (gridDim.x + 1) * N ints.  True in the last block, with the
+// grand totals in total (thread 0).  The ticket is left at zero for the next scan.
+template <int N>
+__device__ inline bool scan_block_totals(int *bsum, int *ticket, int (&total)[N])
 {
-    const int add = bsum[blockIdx.x];
+    __shared__ int s_last;
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int c = 0; c < N; ++c)
+            __hip_atomic_store(bsum + (int64_t)blockIdx.x * N + c, total[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int t = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = t == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!s_last) return false;
+    int carry[N] = {};
+    const int64_t nb = gridDim.x;
+    for (int64_t b0 = 0; b0 < nb; b0 += kScanThreads) {
+        const int64_t i = b0 + threadIdx.x;
+        int x[N], all[N];
+#pragma unroll
+        for (int c = 0; c < N; ++c)
+            x[c] = i < nb ? __hip_atomic_load(bsum + i * N + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+        block_exclusive_scan<N>(x, all);
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            if (i < nb) bsum[i * N + c] = x[c] + carry[c];
+            carry[c] += all[c];
+        }
+    }
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            bsum[nb * N + c] = carry[c];
+            total[c] = carry[c];
+        }
+        *ticket = 0;
+    }
+    return true;
+}
+
+// data[i] = exclusive scan within the tile of load(i), i < n.  ret (null: none): ret[0] =
+// the grand total, ret[1] = *err.
+template <typename F>
+__device__ inline void scan_tile(F load, int *__restrict__ data, int64_t n, int *bsum, int *ticket, int *ret, int *err)
+{
+    // values pass through LDS, so that a wave reads and writes consecutive entries while
+    // each thread sums kScanItems consecutive ones
+    __shared__ int4 s_v[kScanTile / 4];
+    int *sv = (int *)s_v;
     const int64_t base = (int64_t)blockIdx.x * kScanTile;
-    for (int k = threadIdx.x; k < kScanTile; k += kScanThreads)
-        if (base + k < n) data[base + k] += add;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        const int i = k * kScanThreads + threadIdx.x;
+        sv[i] = base + i < n ? load(base + i) : 0;
+    }
+    __syncthreads();
+    int v[kScanItems];
+    int sum[1] = {0}, total[1];
+#pragma unroll
+    for (int k = 0; k < kScanItems; k += 4) {
+        const int4 t = s_v[(threadIdx.x * kScanItems + k) / 4];
+        v[k] = t.x;
+        v[k + 1] = t.y;
+        v[k + 2] = t.z;
+        v[k + 3] = t.w;
+        sum[0] += t.x + t.y + t.z + t.w;
+    }
+    block_exclusive_scan<1>(sum, total);
+    int run = sum[0];
+#pragma unroll
+    for (int k = 0; k < kScanItems; k += 4) {
+        const int4 t = make_int4(run, run + v[k], run + v[k] + v[k + 1], run + v[k] + v[k + 1] + v[k + 2]);
+        run = t.w + v[k + 3];
+        s_v[(threadIdx.x * kScanItems + k) / 4] = t;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        const int i = k * kScanThreads + threadIdx.x;
+        if (base + i < n) data[base + i] = sv[i];
+    }
+    if (scan_block_totals<1>(bsum, ticket, total) && ret && threadIdx.x == 0) {
+        ret[0] = total[0];
+        ret[1] = *err;
+    }
+}
+
+__global__ __launch_bounds__(kScanThreads) void k_scan(int *__restrict__ data, int64_t n, int *bsum, int *ticket)
+{
+    scan_tile([&](int64_t i) { return data[i]; }, data, n, bsum, ticket, nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------
 // Digit passes of the stable counting sort.  A key in [0, K) is sorted by
-// ceil(log2 K / kRadixBits) stable counting sorts on successive kRadixBits-wide
-// digits, least significant first.  Each wave owns one chunk of consecutive items:
+// ceil(log2 K / kRadixBits) stable counting sorts on successive digits, least significant
+// first.  Each wave owns one chunk of consecutive items:
 //   k_radix_count   : per-chunk digit histogram (LDS), written digit-major
 //                     cnt[digit * C + chunk]
 //   exclusive scan  : cnt -> global start of every (digit, chunk) run; digit-major
@@ -269,28 +331,30 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_add(int *__restrict__ dat
 // Every pass is stable, so the result is the stable order by key.
 // ---------------------------------------------------------------------------
 
-constexpr int kRadixBits = 10;
-constexpr int kRadixBins = 1 << kRadixBits;
+// Digits are of equal width, at most kRadixBits: fewer bins mean shorter count arrays to
+// scan (17-bit keys as 9 + 8 instead of 10 + 7 bits).
+constexpr int kRadixBits = 11;
 constexpr int kRadixWaves = 4;
 
 __global__ __launch_bounds__(64 * kRadixWaves) void k_radix_count(int64_t n, const int *__restrict__ keys, int stride,
                                                                   int shift, int bins, int64_t chunk_len, int C,
                                                                   int *__restrict__ cnt)
 {
-    __shared__ int hist[kRadixWaves][kRadixBins];
+    extern __shared__ int lds_radix[]; // [kRadixWaves][bins]
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int *hist = lds_radix + wave * bins;
     const int chunk = blockIdx.x * kRadixWaves + wave;
-    for (int d = lane; d < bins; d += 64) hist[wave][d] = 0;
+    for (int d = lane; d < bins; d += 64) hist[d] = 0;
     __syncthreads();
     if (chunk < C) {
         const int64_t beg = (int64_t)chunk * chunk_len;
         const int64_t end = min(n, beg + chunk_len);
         for (int64_t i = beg + lane; i < end; i += 64)
-            atomicAdd(&hist[wave][(keys[i * stride] >> shift) & (bins - 1)], 1);
+            atomicAdd(&hist[(keys[i * stride] >> shift) & (bins - 1)], 1);
     }
     __syncthreads();
     if (chunk < C)
-        for (int d = lane; d < bins; d += 64) cnt[(int64_t)d * C + chunk] = hist[wave][d];
+        for (int d = lane; d < bins; d += 64) cnt[(int64_t)d * C + chunk] = hist[d];
 }
 
 // vals_in == nullptr: the values are the item indices (first pass)
@@ -298,15 +362,20 @@ __global__ __launch_bounds__(64 * kRadixWaves) void k_radix_scatter(int64_t n, c
                                                                     int stride, const int *__restrict__ vals_in,
                                                                     int shift, int bits, int64_t chunk_len, int C,
                                                                     const int *__restrict__ offs,
+                                                                    const int *__restrict__ bsum,
                                                                     int *__restrict__ keys_out,
                                                                     int *__restrict__ vals_out)
 {
-    __shared__ int base[kRadixWaves][kRadixBins];
+    extern __shared__ int lds_radix[]; // [kRadixWaves][bins]
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int chunk = blockIdx.x * kRadixWaves + wave;
     const int bins = 1 << bits;
+    int *base = lds_radix + wave * bins;
     if (chunk < C)
-        for (int d = lane; d < bins; d += 64) base[wave][d] = offs[(int64_t)d * C + chunk];
+        for (int d = lane; d < bins; d += 64) {
+            const int64_t i = (int64_t)d * C + chunk;
+            base[d] = offs[i] + bsum[i / kScanTile];
+        }
     __syncthreads();
     if (chunk >= C) return;
     const int64_t beg = (int64_t)chunk * chunk_len;
@@ -325,9 +394,9 @@ __global__ __launch_bounds__(64 * kRadixWaves) void k_radix_scatter(int64_t n, c
             m &= on ? bb : ~bb;
         }
         const int rank = __popcll(m & lt);
-        const int b0 = base[wave][d];
+        const int b0 = base[d];
         __builtin_amdgcn_wave_barrier();
-        if (valid && rank == 0) base[wave][d] = b0 + __popcll(m);
+        if (valid && rank == 0) base[d] = b0 + __popcll(m);
         __builtin_amdgcn_wave_barrier();
         if (valid) {
             keys_out[b0 + rank] = key;
@@ -336,12 +405,11 @@ __global__ __launch_bounds__(64 * kRadixWaves) void k_radix_scatter(int64_t n, c
     }
 }
 
-// bin_start[k] = first position of key k in the sorted keys (n where none), k = 0..K
-__global__ __launch_bounds__(256) void k_bin_starts_sorted(int64_t n, const int *__restrict__ skeys, int64_t K,
-                                                           int *__restrict__ bin_start)
+// bin_start[k] = first position of key k in the sorted keys (n where none), k = 0..K;
+// thread i = 0..n
+__device__ inline void bin_starts(int64_t i, int64_t n, const int *__restrict__ skeys, int64_t K,
+                                  int *__restrict__ bin_start)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > n) return;
     const int64_t kprev = i == 0 ? -1 : skeys[i - 1];
     const int64_t knext = i == n ? K : skeys[i];
     for (int64_t k = kprev + 1; k <= knext; ++k) bin_start[k] = (int)i;
@@ -349,11 +417,14 @@ __global__ __launch_bounds__(256) void k_bin_starts_sorted(int64_t n, const int 
 
 __global__ __launch_bounds__(256) void k_make_records(int64_t M, const int *__restrict__ sorted,
                                                       const int4 *__restrict__ cell, const float4 *__restrict__ frac,
-                                                      const float *__restrict__ dcf, int4 *__restrict__ rec_cell,
-                                                      float4 *__restrict__ rec_frac)
+                                                      const float *__restrict__ dcf, const int *__restrict__ skeys,
+                                                      int64_t K, int *__restrict__ bin_start,
+                                                      int4 *__restrict__ rec_cell, float4 *__restrict__ rec_frac)
 {
     int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= M) return;
+    if (p > M) return;
+    bin_starts(p, M, skeys, K, bin_start);
+    if (p == M) return;
     const int i = sorted[p];
     const int4 c = cell[i];
     const float4 f = frac[i];
@@ -413,20 +484,25 @@ __device__ inline void tap_box(int s, int q, int T, int nf, int W, int &jlo, int
     }
 }
 
-__global__ __launch_bounds__(256) void k_pair_count(int64_t M, const int4 *__restrict__ rec_cell, TileGeom g,
-                                                    int *__restrict__ cnt)
+// offs[p] = pairs of the records before p within its scan tile; ret: the pair total and the
+// coordinate error flag
+__global__ __launch_bounds__(kScanThreads) void k_pair_scan(int64_t M, const int4 *__restrict__ rec_cell, TileGeom g,
+                                                            int *__restrict__ offs, int *bsum, int *ticket, int *ret,
+                                                            int *err)
 {
-    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= M) return;
-    const int4 rc = rec_cell[p];
-    const int s[3] = {rc.x, rc.y, rc.z};
-    int n = 1;
-    for (int ax = 0; ax < g.dim; ++ax) {
-        int q0, na;
-        axis_tile_span(s[ax], g.W, (int)g.nf[ax], g.tile[ax], q0, na);
-        n *= na;
-    }
-    cnt[p] = n;
+    scan_tile(
+        [&](int64_t p) {
+            const int4 rc = rec_cell[p];
+            const int s[3] = {rc.x, rc.y, rc.z};
+            int n = 1;
+            for (int ax = 0; ax < g.dim; ++ax) {
+                int q0, na;
+                axis_tile_span(s[ax], g.W, (int)g.nf[ax], g.tile[ax], q0, na);
+                n *= na;
+            }
+            return n;
+        },
+        offs, M, bsum, ticket, ret, err);
 }
 
 // The pairs of sample record p are offs[p] .. offs[p] + n - 1 with n = the product of
@@ -436,8 +512,8 @@ __global__ __launch_bounds__(256) void k_pair_count(int64_t M, const int4 *__res
 // after the stable sort by tile, k_pair_records rebuilds every record in sorted order
 // from its sample record, so only 8 bytes per pair are written in sample order.
 __global__ __launch_bounds__(256) void k_pair_keys(int64_t M, const int4 *__restrict__ rec_cell, TileGeom g,
-                                                   const int *__restrict__ offs, int *__restrict__ pkey,
-                                                   int *__restrict__ psamp)
+                                                   const int *__restrict__ offs, const int *__restrict__ bsum,
+                                                   int *__restrict__ pkey, int *__restrict__ psamp)
 {
     int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= M) return;
@@ -446,7 +522,7 @@ __global__ __launch_bounds__(256) void k_pair_keys(int64_t M, const int4 *__rest
     axis_tile_span(rc.x, g.W, (int)g.nf[0], g.tile[0], q0[0], n[0]);
     axis_tile_span(rc.y, g.W, (int)g.nf[1], g.tile[1], q0[1], n[1]);
     if (g.dim == 3) axis_tile_span(rc.z, g.W, (int)g.nf[2], g.tile[2], q0[2], n[2]);
-    int o = offs[p];
+    int o = offs[p] + bsum[p / kScanTile];
     int t0 = q0[0];
     for (int i = 0; i < n[0]; ++i) {
         int t1 = q0[1];
@@ -473,12 +549,16 @@ __global__ __launch_bounds__(256) void k_pair_keys(int64_t M, const int4 *__rest
 // (j = first window tap inside the tile, c = taps inside, l = tile-local cell of tap j).
 __global__ __launch_bounds__(256) void k_pair_records(int64_t P, const int *__restrict__ sorted,
                                                       const int *__restrict__ psamp, const int *__restrict__ offs,
+                                                      const int *__restrict__ bsum, const int *__restrict__ skeys,
+                                                      int64_t K, int *__restrict__ bin_start,
                                                       const int4 *__restrict__ rec_cell,
                                                       const float4 *__restrict__ rec_frac, TileGeom g,
                                                       int4 *__restrict__ pa, int4 *__restrict__ pb)
 {
     int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= P) return;
+    if (q > P) return;
+    bin_starts(q, P, skeys, K, bin_start);
+    if (q == P) return;
     const int o = sorted[q];
     const int p = psamp[o];
     const int4 rc = rec_cell[p];
@@ -487,7 +567,7 @@ __global__ __launch_bounds__(256) void k_pair_records(int64_t P, const int *__re
     axis_tile_span(rc.x, g.W, (int)g.nf[0], g.tile[0], q0[0], n[0]);
     axis_tile_span(rc.y, g.W, (int)g.nf[1], g.tile[1], q0[1], n[1]);
     if (g.dim == 3) axis_tile_span(rc.z, g.W, (int)g.nf[2], g.tile[2], q0[2], n[2]);
-    const int local = o - offs[p];
+    const int local = o - (offs[p] + bsum[p / kScanTile]);
     const int m = local % n[2], r = local / n[2];
     const int k = r % n[1], i = r / n[1];
     int t0 = q0[0] + i, t1 = q0[1] + k, t2 = q0[2] + m;
@@ -509,60 +589,82 @@ __global__ __launch_bounds__(256) void k_pair_records(int64_t P, const int *__re
 // items of tiles with pairs come first, in tile order, then one item per empty tile,
 // in tile order (a launch that need not write empty tiles takes only the first
 // part).  Items, empty-tile items, slots and reduce items are numbered by exclusive
-// scans of the per-tile counts that k_item_counts writes.
-__global__ __launch_bounds__(256) void k_item_counts(int64_t K, const int *__restrict__ pstart, int chunk,
-                                                     int *__restrict__ nitems, int *__restrict__ nempty,
-                                                     int *__restrict__ nslots, int *__restrict__ nsplit)
+// scans of the per-tile counts (k_item_scan).  The gather's items are numbered the same
+// way from the gather tiles' sample offsets.
+__global__ __launch_bounds__(kScanThreads) void k_item_scan(int64_t K, const int *__restrict__ pstart, int chunk,
+                                                            int4 *__restrict__ off, int *bsum, int *ticket, int *ret)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= K) return;
-    const int n = pstart[k + 1] - pstart[k];
-    const int nch = (n + chunk - 1) / chunk;
-    const bool split = n > chunk;
-    nitems[k] = split ? nch : n > 0 ? 1 : 0;
-    nempty[k] = n == 0 ? 1 : 0;
-    nslots[k] = split ? nch : 0;
-    nsplit[k] = split ? 1 : 0;
+    const int64_t base = (int64_t)blockIdx.x * kItemTile + (int64_t)threadIdx.x * 4;
+    int c[4][4], sum[4] = {0, 0, 0, 0}, total[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int64_t k = base + i;
+        const int n = k < K ? pstart[k + 1] - pstart[k] : 0;
+        const int nch = (n + chunk - 1) / chunk;
+        c[i][0] = nch;                             // work items
+        c[i][1] = k < K && n == 0 ? 1 : 0;         // items of empty tiles
+        c[i][2] = n > chunk ? nch : 0;             // partial slots
+        c[i][3] = n > chunk ? 1 : 0;               // reduce items
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] += c[i][j];
+    }
+    block_exclusive_scan<4>(sum, total);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (base + i < K) off[base + i] = make_int4(sum[0], sum[1], sum[2], sum[3]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[j] += c[i][j];
+    }
+    if (scan_block_totals<4>(bsum, ticket, total) && threadIdx.x == 0)
+        for (int j = 0; j < 4; ++j) ret[j] = total[j];
 }
 
-// nfull: the items of tiles with pairs (grand total of the ioff scan)
+// reduce null: gather items (none for empty tiles).  bsum: the block offsets of
+// k_item_scan, then the grand totals.
 __global__ __launch_bounds__(256) void k_item_write(int64_t K, const int *__restrict__ pstart, int chunk,
-                                                    const int *__restrict__ ioff, const int *__restrict__ eoff,
-                                                    const int *__restrict__ nfull, const int *__restrict__ soff,
-                                                    const int *__restrict__ roff, int4 *__restrict__ items,
-                                                    int4 *__restrict__ reduce)
+                                                    const int4 *__restrict__ off, const int4 *__restrict__ bsum,
+                                                    int64_t nb, int4 *__restrict__ items, int4 *__restrict__ reduce)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= K) return;
     const int b = pstart[k], e = pstart[k + 1];
+    const int4 o = off[k], s = bsum[k / kItemTile];
     if (e == b) {
-        items[*nfull + eoff[k]] = make_int4((int)k, b, e, -1);
+        if (reduce) items[bsum[nb].x + o.y + s.y] = make_int4((int)k, b, e, -1);
         return;
     }
-    const int o = ioff[k];
+    const int i0 = o.x + s.x;
+    if (!reduce) {
+        for (int c = 0, x = b; x < e; ++c, x += chunk) items[i0 + c] = make_int4((int)k, x, min(e, x + chunk), 0);
+        return;
+    }
     if (e - b <= chunk) {
-        items[o] = make_int4((int)k, b, e, -1);
+        items[i0] = make_int4((int)k, b, e, -1);
         return;
     }
-    const int nch = (e - b + chunk - 1) / chunk, s0 = soff[k];
-    reduce[roff[k]] = make_int4((int)k, s0, nch, 0);
-    for (int c = 0; c < nch; ++c) items[o + c] = make_int4((int)k, b + c * chunk, min(e, b + (c + 1) * chunk), s0 + c);
+    const int nch = (e - b + chunk - 1) / chunk, s0 = o.z + s.z;
+    reduce[o.w + s.w] = make_int4((int)k, s0, nch, 0);
+    for (int c = 0; c < nch; ++c) items[i0 + c] = make_int4((int)k, b + c * chunk, min(e, b + (c + 1) * chunk), s0 + c);
 }
 
 // Occupancy row masks: one word per column of spread tiles (ncolt = ntiles[1] *
 // ntiles[2] columns), bit b set when one of the leading-axis tiles [b mask_k,
-// (b + 1) mask_k) of the column holds pairs; one thread per column, no atomics.
+// (b + 1) mask_k) of the column holds pairs; one wave per column, a bit per lane.
 __global__ __launch_bounds__(256) void k_occ_masks(int64_t ncolt, int nt0, int mask_k, const int *__restrict__ pstart,
                                                    unsigned long long *__restrict__ occ)
 {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (c >= ncolt) return;
-    unsigned long long m = 0ull;
-    for (int t0 = 0; t0 < nt0; ++t0) {
+    const int lane = threadIdx.x & 63;
+    bool on = false;
+    for (int i = 0; i < mask_k; ++i) {
+        const int t0 = lane * mask_k + i;
+        if (t0 >= nt0) break;
         const int64_t k = t0 * ncolt + c;
-        if (pstart[k + 1] > pstart[k]) m |= 1ull << (t0 / mask_k);
+        on = on || pstart[k + 1] > pstart[k];
     }
-    occ[c] = m;
+    const unsigned long long m = __ballot(on);
+    if (lane == 0) occ[c] = m;
 }
 
 // ---------------------------------------------------------------------------
@@ -2354,7 +2456,29 @@ struct ScratchPool {
     std::mutex mu;
     std::vector<void *> ptr;
     std::vector<size_t> cap;
+    int *ticket = nullptr; // of the scans, zero between them
+    int *ret = nullptr;    // pinned: values the scans return to the host (kRet*)
+    int init()
+    {
+        if (!ticket) {
+            int *t = nullptr;
+            if (hipMalloc((void **)&t, sizeof(int)) != hipSuccess) return fail(GN_ENOMEM, "hipMalloc failed for the scans");
+            const int zero = 0;
+            hipError_t e = hipMemcpy(t, &zero, sizeof(int), hipMemcpyHostToDevice);
+            if (e != hipSuccess) {
+                (void)hipFree(t);
+                return hip_fail(e, "scan ticket");
+            }
+            ticket = t;
+        }
+        if (!ret && hipHostMalloc((void **)&ret, 16 * sizeof(int)) != hipSuccess) {
+            ret = nullptr;
+            return fail(GN_ENOMEM, "hipHostMalloc failed for the scan results");
+        }
+        return GN_OK;
+    }
 };
+enum { kRetPairs = 0, kRetErr = 1, kRetSpread = 4, kRetGather = 8 };
 
 ScratchPool &scratch_pool()
 {
@@ -2413,36 +2537,32 @@ int grow_alloc(T **p, int64_t *cap, size_t count, const char *what)
     return rc;
 }
 
-// Exclusive scan of n ints in place; writes the total to *total_dev (device int).
-hipError_t device_scan(int *data, int64_t n, int *bsum, hipStream_t st)
+// Exclusive scan of n ints (see k_scan); bsum: n / kScanTile + 2 ints.
+hipError_t device_scan(int *data, int64_t n, int *bsum, Scratch &sc)
 {
-    const int64_t nb = (n + kScanTile - 1) / kScanTile;
-    hipLaunchKernelGGL(k_scan_local, dim3((unsigned)std::max<int64_t>(nb, 1)), dim3(kScanThreads), 0, st, data, n,
-                       bsum);
-    hipLaunchKernelGGL(k_scan_bsums, dim3(1), dim3(kScanThreads), 0, st, bsum, nb);
-    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)std::max<int64_t>(nb, 1)), dim3(kScanThreads), 0, st, data, n,
-                       bsum);
+    const int64_t nb = std::max<int64_t>(1, (n + kScanTile - 1) / kScanTile);
+    hipLaunchKernelGGL(k_scan, dim3((unsigned)nb), dim3(kScanThreads), 0, sc.stream, data, n, bsum, sc.pool.ticket);
     return hipGetLastError();
 }
 
 // Stable counting sort of n items by keys[i*stride] in [0,K): writes the sorted item
-// indices and the K+1 bucket offsets.  Asynchronous on st; the temporary buffers
+// indices; *skeys: the sorted keys (scratch).  Asynchronous on st; the temporary buffers
 // belong to sc, which the caller keeps alive until the stream has consumed them.
-int stable_sort_by_key(int64_t n, const int *keys, int stride, int64_t K, int *sorted, int *bin_start,
+int stable_sort_by_key(int64_t n, const int *keys, int stride, int64_t K, int *sorted, const int **skeys,
                        hipStream_t st, Scratch &sc)
 {
     int rc;
     int kbits = 1;
     while (kbits < 31 && ((int64_t)1 << kbits) < K) ++kbits;
-    const int npass = (kbits + kRadixBits - 1) / kRadixBits;
+    const int npass = (kbits + kRadixBits - 1) / kRadixBits, pbits = (kbits + npass - 1) / npass;
     // chunks: about 4096 waves over the GPU, 256..4096 items each
     int64_t chunk_len = (n + 4095) / 4096;
     chunk_len = std::min<int64_t>(4096, std::max<int64_t>(256, ((chunk_len + 63) / 64) * 64));
     const int64_t C = std::max<int64_t>(1, (n + chunk_len - 1) / chunk_len);
-    const int64_t nKC = (int64_t)kRadixBins * C;
-    const int64_t nb = (nKC + kScanTile - 1) / kScanTile;
+    const int64_t nKC = ((int64_t)1 << pbits) * C;
     int *cnt = nullptr, *bsum = nullptr, *k0 = nullptr, *v0 = nullptr, *k1 = nullptr, *v1 = nullptr;
-    if ((rc = sc.alloc(&cnt, (size_t)nKC, "sort counts")) || (rc = sc.alloc(&bsum, (size_t)nb + 1, "sort scan")) ||
+    if ((rc = sc.alloc(&cnt, (size_t)nKC, "sort counts")) ||
+        (rc = sc.alloc(&bsum, (size_t)(nKC / kScanTile) + 2, "sort scan")) ||
         (rc = sc.alloc(&k0, (size_t)n, "sort keys")) || (rc = sc.alloc(&k1, (size_t)n, "sort keys")) ||
         (rc = sc.alloc(&v0, (size_t)n, "sort values")))
         return rc;
@@ -2457,17 +2577,17 @@ int stable_sort_by_key(int64_t n, const int *keys, int stride, int64_t K, int *s
     int shift = 0;
     hipError_t e = hipSuccess;
     for (int ps = 0; ps < npass && e == hipSuccess; ++ps) {
-        const int bits = std::min(kRadixBits, kbits - shift);
+        const int bits = std::min(pbits, kbits - shift);
         const int bins = 1 << bits;
         const int o = (npass - 1 - ps) % 2 == 0 ? 1 : 0; // the last pass writes slot 1 (sorted)
-        const int64_t nbins = (int64_t)bins * C;
-        hipLaunchKernelGGL(k_radix_count, dim3(nblk), dim3(64 * kRadixWaves), 0, st, n, kin, kstride, shift, bins,
+        const size_t lds = (size_t)kRadixWaves * bins * sizeof(int);
+        hipLaunchKernelGGL(k_radix_count, dim3(nblk), dim3(64 * kRadixWaves), lds, st, n, kin, kstride, shift, bins,
                            chunk_len, (int)C, cnt);
         e = hipGetLastError();
-        if (e == hipSuccess) e = device_scan(cnt, nbins, bsum, st);
+        if (e == hipSuccess) e = device_scan(cnt, (int64_t)bins * C, bsum, sc);
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_radix_scatter, dim3(nblk), dim3(64 * kRadixWaves), 0, st, n, kin, kstride, vin, shift,
-                               bits, chunk_len, (int)C, cnt, kout[o], vout[o]);
+            hipLaunchKernelGGL(k_radix_scatter, dim3(nblk), dim3(64 * kRadixWaves), lds, st, n, kin, kstride, vin,
+                               shift, bits, chunk_len, (int)C, cnt, bsum, kout[o], vout[o]);
             e = hipGetLastError();
         }
         kin = kout[o];
@@ -2475,12 +2595,8 @@ int stable_sort_by_key(int64_t n, const int *keys, int stride, int64_t K, int *s
         kstride = 1;
         shift += bits;
     }
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_bin_starts_sorted, dim3(grid_blocks(n + 1, 256, INT32_MAX)), dim3(256), 0, st, n, kin, K,
-                           bin_start);
-        e = hipGetLastError();
-    }
     if (e != hipSuccess) return hip_fail(e, "stable sort");
+    *skeys = kin;
     return GN_OK;
 }
 
@@ -2604,14 +2720,17 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
     R.npairs = 0;
 
     Scratch sc(st);
-    std::vector<int> h_home(Kg + 1, 0);
-    int counts[4] = {0, 0, 0, 0}; // items of tiles with pairs, partial slots, reduce items, empty tiles
+    if ((rc = sc.pool.init())) return rc;
+    int *ticket = sc.pool.ticket;
+    volatile int *ret = sc.pool.ret;
     int *tile_pairs = nullptr; // K + 1 offsets of each spread tile's pairs (scratch)
+    if ((rc = sc.alloc(&tile_pairs, (size_t)K + 1, "pairs"))) return rc;
 
     if (M > 0) {
         int4 *cell = nullptr;
         float4 *frac = nullptr;
         int *sorted = nullptr;
+        const int *skeys = nullptr;
         if ((rc = sc.alloc(&cell, (size_t)M, "sort scratch")) || (rc = sc.alloc(&frac, (size_t)M, "sort scratch")) ||
             (rc = sc.alloc(&sorted, (size_t)M, "sort scratch")))
             return rc;
@@ -2632,13 +2751,13 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
         pa.cell = cell;
         pa.frac = frac;
         pa.err = p->err_flag;
-        GN_HIP(hipMemsetAsync(p->err_flag, 0, sizeof(int), st));
+        pa.seq = p->points_seq = p->points_seq == INT32_MAX ? 1 : p->points_seq + 1;
         hipLaunchKernelGGL(k_prep, dim3(grid_blocks(M, 256, INT32_MAX)), dim3(256), 0, st, pa);
         GN_HIP(hipGetLastError());
         // gather-tile sort (stable) -> records in tile order
-        if ((rc = stable_sort_by_key(M, &cell[0].w, 4, Kg, sorted, R.bin_start, st, sc))) return rc;
-        hipLaunchKernelGGL(k_make_records, dim3(grid_blocks(M, 256, INT32_MAX)), dim3(256), 0, st, M, sorted, cell,
-                           frac, dcf, R.cell, R.frac);
+        if ((rc = stable_sort_by_key(M, &cell[0].w, 4, Kg, sorted, &skeys, st, sc))) return rc;
+        hipLaunchKernelGGL(k_make_records, dim3(grid_blocks(M + 1, 256, INT32_MAX)), dim3(256), 0, st, M, sorted, cell,
+                           frac, dcf, skeys, Kg, R.bin_start, R.cell, R.frac);
         GN_HIP(hipGetLastError());
 
         // (spread tile, sample) pairs: keys in record order, sorted by tile, records rebuilt in tile order
@@ -2654,44 +2773,39 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
         const int64_t nbp = (M + kScanTile - 1) / kScanTile;
         if ((rc = sc.alloc(&pcnt, (size_t)M, "pair counts")) || (rc = sc.alloc(&pbsum, (size_t)nbp + 1, "pair scan")))
             return rc;
-        hipLaunchKernelGGL(k_pair_count, dim3(grid_blocks(M, 256, INT32_MAX)), dim3(256), 0, st, M, R.cell, tg, pcnt);
+        // one host round trip returns the pair total and the coordinate error flag
+        hipLaunchKernelGGL(k_pair_scan, dim3((unsigned)nbp), dim3(kScanThreads), 0, st, M, R.cell, tg, pcnt, pbsum,
+                           ticket, sc.pool.ret + kRetPairs, p->err_flag);
         GN_HIP(hipGetLastError());
-        // the pair total is the scan's grand total (pbsum[nb]); one host round trip
-        // returns it together with the coordinate error flag
-        GN_HIP(device_scan(pcnt, M, pbsum, st));
-        int hv[2] = {0, 0};
-        GN_HIP(hipMemcpyAsync(&hv[0], pbsum + nbp, sizeof(int), hipMemcpyDeviceToHost, st));
-        GN_HIP(hipMemcpyAsync(&hv[1], p->err_flag, sizeof(int), hipMemcpyDeviceToHost, st));
         GN_HIP(hipStreamSynchronize(st));
-        if (hv[1]) return fail(GN_EINVAL, "non-finite sample coordinate");
-        const int64_t P = (int64_t)(unsigned)hv[0];
+        if (ret[kRetErr] == p->points_seq) return fail(GN_EINVAL, "non-finite sample coordinate");
+        const int64_t P = (int64_t)(unsigned)ret[kRetPairs];
         if (P > (int64_t)INT32_MAX) return fail(GN_EINVAL, "too many (tile, sample) pairs");
-        int *pkey = nullptr, *psamp = nullptr, *psorted = nullptr, *pstart = nullptr;
+        int *pkey = nullptr, *psamp = nullptr, *psorted = nullptr;
         if ((rc = sc.alloc(&pkey, (size_t)P, "pairs")) || (rc = sc.alloc(&psamp, (size_t)P, "pairs")) ||
-            (rc = sc.alloc(&psorted, (size_t)P, "pairs")) || (rc = sc.alloc(&pstart, (size_t)K + 1, "pairs")))
+            (rc = sc.alloc(&psorted, (size_t)P, "pairs")))
             return rc;
         hipLaunchKernelGGL(k_pair_keys, dim3(grid_blocks(M, 256, INT32_MAX)), dim3(256), 0, st, M, R.cell, tg, pcnt,
-                           pkey, psamp);
+                           pbsum, pkey, psamp);
         GN_HIP(hipGetLastError());
-        if ((rc = stable_sort_by_key(P, pkey, 1, K, psorted, pstart, st, sc))) return rc;
+        if ((rc = stable_sort_by_key(P, pkey, 1, K, psorted, &skeys, st, sc))) return rc;
         if (P > R.pairs_cap) {
             if ((rc = dev_alloc(&R.pair_a, (size_t)P, "pairs")) || (rc = dev_alloc(&R.pair_b, (size_t)P, "pairs")))
                 return rc;
             R.pairs_cap = P;
         }
-        hipLaunchKernelGGL(k_pair_records, dim3(grid_blocks(P, 256, INT32_MAX)), dim3(256), 0, st, P, psorted, psamp,
-                           pcnt, R.cell, R.frac, tg, R.pair_a, R.pair_b);
+        hipLaunchKernelGGL(k_pair_records, dim3(grid_blocks(P + 1, 256, INT32_MAX)), dim3(256), 0, st, P, psorted,
+                           psamp, pcnt, pbsum, skeys, K, tile_pairs, R.cell, R.frac, tg, R.pair_a, R.pair_b);
         GN_HIP(hipGetLastError());
-        tile_pairs = pstart;
         R.npairs = P;
     } else {
         GN_HIP(hipMemsetAsync(R.bin_start, 0, sizeof(int) * (Kg + 1), st));
-        if ((rc = sc.alloc(&tile_pairs, (size_t)K + 1, "pairs"))) return rc;
         GN_HIP(hipMemsetAsync(tile_pairs, 0, sizeof(int) * (K + 1), st));
     }
 
-    // spread work items, partial slots, reduce items and occupancy masks on the device;
-    // their counts come back with the gather bin offsets in one synchronisation
+    // spread work items, partial slots, reduce items, occupancy masks (the spread leaves
+    // tiles without pairs unwritten where the first adjoint FFT pass skips them) and gather
+    // work items on the device; their counts come back in one synchronisation
     {
         const int64_t P = R.npairs;
         const int chunk = spread_chunk(P);
@@ -2699,52 +2813,38 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
         const int64_t ncolt = (int64_t)g.ntiles[1] * g.ntiles[2];
         if ((rc = grow_alloc(&R.spread_items, &R.spread_items_cap, (size_t)cap_items, "work items")) ||
             (rc = grow_alloc(&R.reduce_items, &R.reduce_items_cap, (size_t)cap_red, "work items")) ||
+            (rc = grow_alloc(&R.gather_items, &R.gather_items_cap, (size_t)(Kg + M / kGatherChunk + 1), "work items")) ||
             (rc = grow_alloc(&R.occ_mask, &R.occ_mask_cap, (size_t)ncolt, "tile masks")))
             return rc;
-        const int64_t nbk = (K + kScanTile - 1) / kScanTile;
-        int *ni = nullptr, *ne = nullptr, *ns = nullptr, *nr = nullptr;
-        int *bi = nullptr, *be = nullptr, *bs = nullptr, *br = nullptr;
-        if ((rc = sc.alloc(&ni, (size_t)K, "work items")) || (rc = sc.alloc(&ne, (size_t)K, "work items")) ||
-            (rc = sc.alloc(&ns, (size_t)K, "work items")) || (rc = sc.alloc(&nr, (size_t)K, "work items")) ||
-            (rc = sc.alloc(&bi, (size_t)nbk + 1, "work items")) || (rc = sc.alloc(&be, (size_t)nbk + 1, "work items")) ||
-            (rc = sc.alloc(&bs, (size_t)nbk + 1, "work items")) || (rc = sc.alloc(&br, (size_t)nbk + 1, "work items")))
+        auto items = [&](int64_t n, const int *start, int len, int ret_at, int4 *out, int4 *reduce) -> int {
+            const int64_t nb = (n + kItemTile - 1) / kItemTile;
+            int4 *off = nullptr, *bs = nullptr;
+            int r;
+            if ((r = sc.alloc(&off, (size_t)n, "work items")) || (r = sc.alloc(&bs, (size_t)nb + 1, "work items")))
+                return r;
+            hipLaunchKernelGGL(k_item_scan, dim3((unsigned)nb), dim3(kScanThreads), 0, st, n, start, len, off, (int *)bs,
+                               ticket, sc.pool.ret + ret_at);
+            GN_HIP(hipGetLastError());
+            hipLaunchKernelGGL(k_item_write, dim3(grid_blocks(n, 256, INT32_MAX)), dim3(256), 0, st, n, start, len, off,
+                               bs, nb, out, reduce);
+            GN_HIP(hipGetLastError());
+            return GN_OK;
+        };
+        if ((rc = items(K, tile_pairs, chunk, kRetSpread, R.spread_items, R.reduce_items)) ||
+            (rc = items(Kg, R.bin_start, kGatherChunk, kRetGather, R.gather_items, nullptr)))
             return rc;
-        const dim3 gk(grid_blocks(K, 256, INT32_MAX));
-        hipLaunchKernelGGL(k_item_counts, gk, dim3(256), 0, st, K, tile_pairs, chunk, ni, ne, ns, nr);
-        GN_HIP(hipGetLastError());
-        GN_HIP(device_scan(ni, K, bi, st));
-        GN_HIP(device_scan(ne, K, be, st));
-        GN_HIP(device_scan(ns, K, bs, st));
-        GN_HIP(device_scan(nr, K, br, st));
-        hipLaunchKernelGGL(k_item_write, gk, dim3(256), 0, st, K, tile_pairs, chunk, ni, ne, bi + nbk, ns, nr,
-                           R.spread_items, R.reduce_items);
-        GN_HIP(hipGetLastError());
         R.mask_k = (g.ntiles[0] + 63) / 64;
-        hipLaunchKernelGGL(k_occ_masks, dim3(grid_blocks(ncolt, 256, INT32_MAX)), dim3(256), 0, st, ncolt, g.ntiles[0],
+        hipLaunchKernelGGL(k_occ_masks, dim3(grid_blocks(ncolt, 4, INT32_MAX)), dim3(256), 0, st, ncolt, g.ntiles[0],
                            R.mask_k, tile_pairs, R.occ_mask);
         GN_HIP(hipGetLastError());
-        GN_HIP(hipMemcpyAsync(&counts[0], bi + nbk, sizeof(int), hipMemcpyDeviceToHost, st));
-        GN_HIP(hipMemcpyAsync(&counts[1], bs + nbk, sizeof(int), hipMemcpyDeviceToHost, st));
-        GN_HIP(hipMemcpyAsync(&counts[2], br + nbk, sizeof(int), hipMemcpyDeviceToHost, st));
-        GN_HIP(hipMemcpyAsync(&counts[3], be + nbk, sizeof(int), hipMemcpyDeviceToHost, st));
-        GN_HIP(hipMemcpyAsync(h_home.data(), R.bin_start, sizeof(int) * (Kg + 1), hipMemcpyDeviceToHost, st));
         GN_HIP(hipStreamSynchronize(st));
     }
-
-    // work items: every spread tile gets at least one item (empty tiles write zeros),
-    // and the occupancy row masks for the first adjoint FFT pass (the spread leaves
-    // tiles without pairs unwritten where that pass skips them)
-    std::vector<host::Item> gitems;
-    host::build_gather_items(Kg, h_home.data(), kGatherChunk, gitems);
-    if ((rc = grow_alloc(&R.gather_items, &R.gather_items_cap, gitems.size(), "work items"))) return rc;
-    if (!gitems.empty())
-        GN_HIP(hipMemcpy(R.gather_items, gitems.data(), sizeof(int4) * gitems.size(), hipMemcpyHostToDevice));
-    R.n_spread_items = counts[0] + counts[3];
-    R.n_spread_full = counts[0];
-    R.n_slots = counts[1];
-    R.n_reduce_items = counts[2];
-    R.n_gather_items = (int)gitems.size();
-    const int slots = counts[1];
+    R.n_spread_full = ret[kRetSpread];
+    R.n_spread_items = ret[kRetSpread] + ret[kRetSpread + 1];
+    R.n_slots = ret[kRetSpread + 2];
+    R.n_reduce_items = ret[kRetSpread + 3];
+    R.n_gather_items = ret[kRetGather];
+    const int slots = R.n_slots;
     if (R.n_gather_items > 0) {
         const GatherArgs ga = make_gather_args(p, nullptr);
         if (g.dim == 3)

@@ -177,3 +177,32 @@ def test_spread_tiles(modes, ns, nc, layout):
     grid = P.grid_spread(yl)
     ref = np.moveaxis(O.spread(c64, y.astype(np.complex128), p.nf, p.ns, p.tau), -1, 0)
     assert rel(grid, ref) <= TOL
+
+
+@pytest.mark.parametrize("modes", [(5, 6), (64, 60), (6, 5, 7), (40, 33, 36)])
+@pytest.mark.parametrize("M", [1, 64, 2047, 2049, 9000])
+def test_set_points_sizes(modes, M):
+    """Scan tiles, digit widths and item counts at their edges: the sample order is the stable
+    order by gather tile, and both directions match the oracle.  A plan that has refused a
+    non-finite coordinate takes the next points."""
+    from mripy_amd.plan import Plan
+    print("case: set_points", modes, M, flush=True)
+    rng = np.random.default_rng(M)
+    coords = [(np.pi * (2 * rng.random(M) - 1)).astype(np.float32) for _ in modes]
+    c64 = [c.astype(np.float64) for c in coords]
+    P = Plan(modes, ncoils=1, rat=2, nspread=3)
+    bad = [c.copy() for c in coords]
+    bad[1][M // 2] = np.nan
+    for _ in range(2):
+        with pytest.raises(ValueError):
+            P.set_points(bad)
+        P.set_points(coords)
+        s = [(1 + np.floor(np.mod(c, 2 * np.pi) / (2 * np.pi / n)).astype(int) - 3) % n for c, n in zip(c64, P.nf)]
+        key = 0
+        for a, t in enumerate(P.gather_tiles):
+            key = key * -(-P.nf[a] // t) + s[a] // t
+        assert np.array_equal(P.sample_order(), np.argsort(key, kind="stable"))
+    p = O.Params(modes, rat=2, nspread=3)
+    F, y = _cnormal(rng, modes + (1,)), _cnormal(rng, (M, 1))
+    assert rel(P.type2(F), O.type2(c64, F.astype(np.complex128), p)) <= TOL
+    assert rel(P.type1(y), O.type1(c64, y.astype(np.complex128), p)) <= TOL
