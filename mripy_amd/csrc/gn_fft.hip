@@ -46,6 +46,7 @@ namespace {
 #define GN_FFT_CB 16
 #endif
 constexpr int kFFTThreads = GN_FFT_THREADS;       // row passes
+constexpr int kFFTSenseThreads = 1024;            // pass A' with every coil of a line in one block
 constexpr int kLoadUnroll = 8;                    // global loads in flight per thread
 constexpr int kPadLoadUnroll = 4;                 // the same in pass A (a 256-thread block loads
                                                   // 128 x 8 cells in one step)
@@ -418,17 +419,55 @@ __device__ __forceinline__ void fft_rows_crop_body(const RowArgs &a, int64_t lin
     const int half = a.m / 2;
     const bool cl = a.layout == GN_COIL_LAST;
     if (a.sens) { // SENSE: the block holds every coil (ncl == nc): sum_c conj(S_c) * image_c
+        // The products replace the cropped line values (each is its own thread's), with the
+        // maps read in their memory order, kLoadUnroll loads in flight; a thread per image
+        // point that walked the coils instead read coil-last maps 8 bytes per cache line.
+        float2 *w = const_cast<float2 *>(res);
+        const int total = a.m * ncl;
+        for (int e0 = threadIdx.x; e0 < total; e0 += kLoadUnroll * blockDim.x) {
+            float2 sc[kLoadUnroll];
+            float dl[kLoadUnroll];
+            int at[kLoadUnroll];
+#pragma unroll
+            for (int u = 0; u < kLoadUnroll; ++u) {
+                const int e = e0 + u * blockDim.x;
+                int n, c;
+                if (cl) {
+                    n = fdiv(e, ncl, rncl);
+                    c = e - n * ncl;
+                } else {
+                    c = fdiv(e, a.m, rm);
+                    n = e - c * a.m;
+                }
+                int p = n - half;
+                if (p < 0) p += a.L;
+                at[u] = c * ls + p;
+                sc[u] = make_float2(0.f, 0.f);
+                dl[u] = 0.f;
+                if (e < total) {
+                    sc[u] = cl ? a.sens[line * a.m * a.nc + e] : a.sens[c * a.nlines * a.m + line * a.m + n];
+                    dl[u] = a.deap_last[n];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kLoadUnroll; ++u) {
+                if (e0 + u * (int)blockDim.x < total) {
+                    const float2 v = w[at[u]];
+                    const float d = d01 * dl[u];
+                    const float2 o = make_float2(v.x * d, v.y * d);
+                    w[at[u]] = make_float2(sc[u].x * o.x + sc[u].y * o.y, sc[u].x * o.y - sc[u].y * o.x);
+                }
+            }
+        }
+        __syncthreads();
         for (int n = threadIdx.x; n < a.m; n += blockDim.x) {
             int p = n - half;
             if (p < 0) p += a.L;
-            const float d = d01 * a.deap_last[n];
             float2 acc = make_float2(0.f, 0.f);
+#pragma unroll 8
             for (int c = 0; c < ncl; ++c) {
-                const float2 v = res[c * ls + p];
-                const float2 o = make_float2(v.x * d, v.y * d);
-                const float2 sc = cl ? a.sens[(line * a.m + n) * a.nc + c] : a.sens[c * a.nlines * a.m + line * a.m + n];
-                acc.x += sc.x * o.x + sc.y * o.y;
-                acc.y += sc.x * o.y - sc.y * o.x;
+                acc.x += w[c * ls + p].x;
+                acc.y += w[c * ls + p].y;
             }
             a.img_out[line * a.m + n] = acc;
         }
@@ -495,7 +534,7 @@ __global__ __launch_bounds__(kFFTThreads) void k_fft_rows_pad(RowArgs a)
     fft_rows_pad_body<GEN>(a, blockIdx.x, blockIdx.y);
 }
 template <bool GEN>
-__global__ __launch_bounds__(kFFTThreads) void k_fft_rows_crop(RowArgs a)
+__global__ __launch_bounds__(kFFTSenseThreads) void k_fft_rows_crop(RowArgs a)
 {
     fft_rows_crop_body<GEN>(a, blockIdx.x, blockIdx.y);
 }
@@ -529,6 +568,16 @@ int pick_cb(int L, bool dbl)
     int cb = GN_FFT_CB;
     while (cb > 1 && col_lds(L, cb, dbl) > (dbl ? 80 * 1024 : GN_FFT_COL_LDS_MAX)) cb /= 2;
     return cb;
+}
+
+// A row-pass launch of fewer than two blocks per CU lasts as long as one block's chain of
+// loads, stages and stores: fewer coils per block shorten it and use more CUs (192^2 x 8
+// coils: pad 14.5 -> 11.1, crop 13.5 -> 11.7 us).  Column passes gain nothing that way:
+// narrower blocks load the tables more often (the same case 13.3 -> 18.6 us at 4 columns).
+constexpr int64_t kFewBlocks = 512;
+void shrink_rows(RowArgs &a)
+{
+    while (a.CL > 1 && a.nlines * ((a.nc + a.CL - 1) / a.CL) < kFewBlocks) a.CL = (a.CL + 1) / 2;
 }
 
 // Coils per row-pass block: at most 16, fewer while the block's LDS exceeds this cap.
@@ -592,7 +641,12 @@ void launch_rows(void (*kernel)(RowArgs), dim3 grid, const RowArgs &a, hipStream
 {
     const size_t lds = row_lds(a.L, a.CL, a.st.dbl);
     allow_lds((const void *)kernel, lds);
-    hipLaunchKernelGGL(kernel, grid, dim3(kFFTThreads), lds, st, a);
+    // A SENSE combine holds every coil.  Blocks of which fewer than four fit a CU's 160 KiB
+    // take 16 waves, or the CU waits out each load and stage with too few (256 lines of 512
+    // points x 32 coils, one 137 KiB block per CU: 33.2 us with 4 waves, 24.1 with 16; 22.5
+    // with the maps read in memory order as well).
+    const int threads = lds > 40 * 1024 && a.img_out ? kFFTSenseThreads : kFFTThreads;
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, a);
 }
 
 RowArgs row_args(const gn_plan_s *p, const FFTAxis &ax, float sign, float scale)
@@ -768,6 +822,7 @@ int pruned_type2_rows_sense(gn_plan_s *p, const float2 *image, float scale, floa
     RowArgs ra = row_args(p, az, sign, scale);
     ra.img_in = image;
     ra.sens = p->sens;
+    shrink_rows(ra);
     dim3 ga((unsigned)ra.nlines, (unsigned)((p->nc + ra.CL - 1) / ra.CL));
     launch_rows(ra.st.gen ? k_fft_rows_pad<true> : k_fft_rows_pad<false>, ga, ra, p->stream);
     hipError_t e = hipGetLastError();
@@ -805,6 +860,7 @@ int pruned_type2_rows(gn_plan_s *p, const float2 *image, float scale, float sign
     const FFTAxis &az = p->fft_ax[g.dim - 1];
     RowArgs ra = row_args(p, az, sign, scale);
     ra.img_in = image;
+    shrink_rows(ra);
     dim3 ga((unsigned)ra.nlines, (unsigned)((p->nc + ra.CL - 1) / ra.CL));
     launch_rows(ra.st.gen ? k_fft_rows_pad<true> : k_fft_rows_pad<false>, ga, ra, p->stream);
     hipError_t e = hipGetLastError();
@@ -871,6 +927,7 @@ int pruned_type1_rows(gn_plan_s *p, float2 *image, float scale, float sign)
     const FFTAxis &az = p->fft_ax[g.dim - 1];
     RowArgs ra = row_args(p, az, sign, scale);
     ra.img_out = image;
+    shrink_rows(ra);
     dim3 ga((unsigned)ra.nlines, (unsigned)((p->nc + ra.CL - 1) / ra.CL));
     launch_rows(ra.st.gen ? k_fft_rows_crop<true> : k_fft_rows_crop<false>, ga, ra, p->stream);
     hipError_t e = hipGetLastError();

@@ -206,3 +206,28 @@ def test_set_points_sizes(modes, M):
     F, y = _cnormal(rng, modes + (1,)), _cnormal(rng, (M, 1))
     assert rel(P.type2(F), O.type2(c64, F.astype(np.complex128), p)) <= TOL
     assert rel(P.type1(y), O.type1(c64, y.astype(np.complex128), p)) <= TOL
+
+
+@pytest.mark.parametrize("layout", ["coil_last", "coil_major"])
+@pytest.mark.parametrize("modes,nc", [((30, 40), 7), ((40, 2), 33), ((50, 3, 4), 5), ((160, 250), 16),
+                                      ((160, 251), 9), ((32, 17), 64)])
+def test_row_pass_blocks(modes, nc, layout):
+    """Row passes of few lines (fewer coils per block) and SENSE combines whose block holds
+    all coils, below and above the size that takes more threads, odd sizes.  (The window's
+    width follows the first mode count, which must not be far below the others.)"""
+    print("case: row passes", modes, nc, layout, flush=True)
+    from mripy_amd.plan import Plan
+    rng = np.random.default_rng(nc)
+    M = 700
+    coords = [(np.pi * (2 * rng.random(M) - 1)).astype(np.float32) for _ in modes]
+    c64 = [c.astype(np.float64) for c in coords]
+    S, y, x = _cnormal(rng, modes + (nc,)), _cnormal(rng, (M, nc)), _cnormal(rng, modes)
+    P = Plan(modes, ncoils=nc, rat=2, nspread=3, layout=layout).set_points(coords)
+    out = (lambda a: np.ascontiguousarray(np.moveaxis(a, -1, 0))) if layout == "coil_major" else (lambda a: a)
+    p = O.Params(modes, rat=2, nspread=3)
+    img, smp = O.type1(c64, y.astype(np.complex128), p), O.type2(c64, S.astype(np.complex128), p)
+    assert rel(P.type1(out(y)), out(img)) <= TOL
+    assert rel(P.type2(out(S)), out(smp)) <= TOL
+    P.set_sense(out(S))
+    assert rel(P.sense_type1(out(y)), (np.conj(S) * img).sum(-1)) <= TOL
+    assert rel(P.sense_type2(x), out(O.type2(c64, x[..., None] * S.astype(np.complex128), p))) <= TOL
