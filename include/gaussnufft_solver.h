@@ -15,6 +15,9 @@
  *                     (grad, Div, amp) pics/tvop_class.py:59-129 (ndim 2), and prox_tv3d /
  *                     prox_tv3d_r pics/proximal_func.py:136-177 with TV3d / TV3d_r
  *                     pics/tvop_class.py:131-253 (ndim 3)
+ *   gn_soft_step   <- the vector updates of one IST or FISTA iteration
+ *                     pics/CS_MRI_solvers_func.py:30-53, 151-186 with prox_l1_soft_thresh2
+ *                     pics/proximal_func.py:19-23
  *
  * Reductions accumulate in FP64 in a fixed order that depends only on n, so a
  * result is bitwise reproducible run to run.  They need a caller-provided device
@@ -65,6 +68,15 @@ int64_t gn_tv_work_bytes(int ndim, const int64_t *shape, int64_t nt);
    has at least 2 samples.  shape is a host array. */
 int gn_tv_prox(int dtype, int ndim, const int64_t *shape, int64_t nt, const void *y, double lambda, double step,
                int niter, int amp_rule, void *work, void *f, void *stream);
+
+/* One IST or FISTA update of n complex64 elements:
+     acc = acc - step * (g - b)                          (b NULL: acc - step * g)
+     x   = acc / (|acc| + 1e-6) * max(|acc| - th, 0)
+     y   = x + beta * (x - x_pre)                        (y NULL: left out)
+   acc is updated in place; x and y alias none of the others.  Infinities and NaN propagate
+   as in complex arithmetic with the real factors as complex numbers. */
+int gn_soft_step(int64_t n, const void *g, const void *b, void *acc, double step, double th, void *x,
+                 const void *x_pre, double beta, void *y, void *stream);
 
 #ifdef __cplusplus
 }

@@ -60,6 +60,8 @@ SIGNATURES = {
     "gn_tv_work_bytes": ([ctypes.c_int, _i64p, ctypes.c_int64], ctypes.c_int64),
     "gn_tv_prox": ([ctypes.c_int, ctypes.c_int, _i64p, ctypes.c_int64, _vp, ctypes.c_double, ctypes.c_double,
                     ctypes.c_int, ctypes.c_int, _vp, _vp, _vp], ctypes.c_int),
+    "gn_soft_step": ([ctypes.c_int64, _vp, _vp, _vp, ctypes.c_double, ctypes.c_double, _vp, _vp, ctypes.c_double, _vp,
+                      _vp], ctypes.c_int),
 }
 
 

@@ -231,3 +231,68 @@ def test_row_pass_blocks(modes, nc, layout):
     P.set_sense(out(S))
     assert rel(P.sense_type1(out(y)), (np.conj(S) * img).sum(-1)) <= TOL
     assert rel(P.sense_type2(x), out(O.type2(c64, x[..., None] * S.astype(np.complex128), p))) <= TOL
+
+
+class _Diag:
+    """x -> d x, with or without the forward_backward the wrappers dispatch on."""
+
+    def __init__(self, d, fb):
+        self.forward = lambda x: d * x
+        self.backward = lambda x: d.conj() * x
+        if fb:
+            self.forward_backward = lambda x: d.conj() * (d * x)
+
+
+@pytest.mark.parametrize("shape", [(1,), (255, 1), (16, 16), (17, 31, 3), (300, 219)])
+@pytest.mark.parametrize("wrap", ["IST_wrap", "FIST_wrap"])
+@pytest.mark.parametrize("fb", [True, False])
+def test_ist_fista_update(shape, wrap, fb):
+    """The update kernel against the same iteration in 64 bits (which takes the separate
+    operations), for a start that has zeros; complex views and tensor thresholds keep the
+    separate operations and agree.  Tolerance: ten FP32 roundings of acc per iteration,
+    |acc| <= |x| + th."""
+    import torch
+    from mripy_amd import solvers as S
+    print("case: update", shape, wrap, fb, flush=True)
+    g = torch.Generator().manual_seed(3)
+    b, d = (torch.randn(shape, generator=g, dtype=torch.complex64).cuda() for _ in range(2))
+    b.view(-1)[1::5] = 0
+    N, kw = 6, dict(Nite=6, step=0.3, th=0.05)
+    want = getattr(S, wrap)(_Diag(d.to(torch.complex128), fb), b=b.to(torch.complex128), **kw)
+    got = getattr(S, wrap)(_Diag(d, fb), b=b, **kw)
+    lim = N * 10 * 6e-8 * float(want.norm() + 0.05 * want.numel() ** 0.5)
+    assert got.dtype == torch.complex64 and float((got - want).norm()) <= lim
+    th = torch.full(shape, 0.05, device="cuda")
+    for v in (getattr(S, wrap)(_Diag(d, fb), b=b, Nite=N, step=0.3, th=th),
+              getattr(S, wrap)(_Diag(d.conj(), fb), b=b.conj(), **kw).conj()):
+        assert float((got - v).norm()) <= 2 * lim
+
+
+@pytest.mark.parametrize("th", [0.5, 0.0, -1.0, 1e30])
+def test_ist_fista_update_extreme_values(th):
+    """Infinities, NaN, the largest and smallest values: as the separate operations."""
+    import torch
+    from mripy_amd import solvers as S
+    inf, nan, big, tiny = float("inf"), float("nan"), 3e38, 1e-42
+    v = [0.0, -0.0, 1.5, -inf, inf, nan, big, -big, tiny]
+    a = torch.tensor([complex(p, q) for p in v for q in v], dtype=torch.complex64, device="cuda")
+    g, xp = torch.zeros_like(a), torch.ones_like(a)
+    for step, b in ((0.5, None), (0.5, a.flip(0))):
+        want_acc = a - step * (g if b is None else g - b)
+        want_x = S.prox_l1_soft_thresh2(want_acc, th)
+        want_y = want_x + 0.25 * (want_x - xp)
+        acc, x, y = S._descend(g, b, step, a.clone(), th, xp, 0.25)
+        for got, want in ((acc, want_acc), (x, want_x), (y, want_y)):
+            got, want = torch.view_as_real(got).cpu().numpy(), torch.view_as_real(want).cpu().numpy()
+            np.testing.assert_allclose(got, want, rtol=1e-6, atol=1e-40)
+
+
+def test_ist_fista_update_keeps_gradients():
+    import torch
+    from mripy_amd import solvers as S
+    d = torch.ones(7, dtype=torch.complex64, device="cuda") * 0.5
+    b = torch.ones(7, dtype=torch.complex64, device="cuda").requires_grad_()
+    for wrap in ("IST_wrap", "FIST_wrap"):
+        x = getattr(S, wrap)(_Diag(d, True), b=b, Nite=3, step=0.5, th=0.01)
+        (grad,) = torch.autograd.grad(x.abs().sum(), b)
+        assert bool((grad.abs() > 0).all())
