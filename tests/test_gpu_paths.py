@@ -296,3 +296,22 @@ def test_ist_fista_update_keeps_gradients():
         x = getattr(S, wrap)(_Diag(d, True), b=b, Nite=3, step=0.5, th=0.01)
         (grad,) = torch.autograd.grad(x.abs().sum(), b)
         assert bool((grad.abs() > 0).all())
+
+
+@pytest.mark.parametrize("modes,ns", [((24, 30), 3), ((20, 17, 22), 3), ((4, 4, 4), 3), ((14, 13, 16), 5), ((5, 6), 9)])
+@pytest.mark.parametrize("nc", [1, 2, 3, 4])
+@pytest.mark.parametrize("layout", ["coil_last", "coil_major"])
+def test_traj_grad_coil_pairs(modes, ns, nc, layout):
+    """Even and odd coil counts, both layouts, and grids that a window region wraps whole."""
+    print("case: trajectory gradient", modes, ns, nc, layout, flush=True)
+    from mripy_amd.plan import Plan
+    rng = np.random.default_rng(nc)
+    M = 1100
+    coords = [(np.pi * (2 * rng.random(M) - 1)).astype(np.float32) for _ in modes]
+    F, w = _cnormal(rng, modes + (nc,)), _cnormal(rng, (M, nc))
+    out = (lambda a: np.ascontiguousarray(np.moveaxis(a, -1, 0))) if layout == "coil_major" else (lambda a: a)
+    import torch
+    P = Plan(modes, ncoils=nc, rat=2, nspread=ns, layout=layout).set_points(coords)
+    got = P.traj_grad(torch.as_tensor(out(F)).cuda(), torch.as_tensor(out(w)).cuda()).cpu().numpy()
+    want = O.traj_grad([c.astype(np.float64) for c in coords], F, w, O.Params(modes, rat=2, nspread=ns))
+    assert rel(got, want) <= TOL
