@@ -269,45 +269,54 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(int *__restrict__ data, i
 // ---------------------------------------------------------------------------
 // Digit passes of the stable counting sort.  A key in [0, K) is sorted by
 // ceil(log2 K / kRadixBits) stable counting sorts on successive digits, least significant
-// first.  Each wave owns one chunk of consecutive items:
+// first.  Each workgroup owns one chunk of consecutive items, each of its waves a quarter:
 //   k_radix_count   : per-chunk digit histogram (LDS), written digit-major
 //                     cnt[digit * C + chunk]
 //   exclusive scan  : cnt -> global start of every (digit, chunk) run; digit-major
 //                     order keeps chunks, hence items, in index order
-//   k_radix_scatter : the wave walks its chunk 64 items at a time; the lanes holding
-//                     the same digit find each other with one ballot per digit bit
-//                     (match mask), rank themselves by lane, and the lowest lane of
-//                     each group advances that digit's running offset in LDS.
-// Every pass is stable, so the result is the stable order by key.
+//   k_radix_scatter : the waves count their quarters again (the chunk is in cache) and take
+//                     their starts within the chunk's runs in wave order; then a wave walks
+//                     its quarter 64 items at a time: the lanes holding the same digit find
+//                     each other with one ballot per digit bit (match mask), rank themselves
+//                     by lane, and the lowest lane of each group advances that digit's
+//                     running offset in LDS.
+// Every pass is stable, so the result is the stable order by key.  A count per workgroup
+// instead of per wave makes the count array, whose digit-major writes and reads touch a
+// cache line each, a quarter as long: set_points of 1048576 samples on a 256^3 grid
+// 645 -> 546 us (nspread 3) and 1390 -> 1143 us (5), of 13056 on 384^2 142 -> 120 us.
 // ---------------------------------------------------------------------------
 
 // Digits are of equal width, at most kRadixBits: fewer bins mean shorter count arrays to
 // scan (17-bit keys as 9 + 8 instead of 10 + 7 bits).
 constexpr int kRadixBits = 11;
 constexpr int kRadixWaves = 4;
+constexpr int kRadixUnroll = 4; // steps of 64 items whose loads are in flight together
 
 __global__ __launch_bounds__(64 * kRadixWaves) void k_radix_count(int64_t n, const int *__restrict__ keys, int stride,
                                                                   int shift, int bins, int64_t chunk_len, int C,
                                                                   int *__restrict__ cnt)
 {
-    extern __shared__ int lds_radix[]; // [kRadixWaves][bins]
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    int *hist = lds_radix + wave * bins;
-    const int chunk = blockIdx.x * kRadixWaves + wave;
-    for (int d = lane; d < bins; d += 64) hist[d] = 0;
+    extern __shared__ int lds_radix[]; // [bins]
+    for (int d = threadIdx.x; d < bins; d += blockDim.x) lds_radix[d] = 0;
     __syncthreads();
-    if (chunk < C) {
-        const int64_t beg = (int64_t)chunk * chunk_len;
-        const int64_t end = min(n, beg + chunk_len);
-        for (int64_t i = beg + lane; i < end; i += 64)
-            atomicAdd(&hist[(keys[i * stride] >> shift) & (bins - 1)], 1);
+    const int64_t beg = (int64_t)blockIdx.x * chunk_len;
+    const int64_t end = min(n, beg + chunk_len);
+    for (int64_t i0 = beg + threadIdx.x; i0 < end; i0 += kRadixUnroll * blockDim.x) {
+        int key[kRadixUnroll];
+#pragma unroll
+        for (int u = 0; u < kRadixUnroll; ++u) {
+            const int64_t i = i0 + u * blockDim.x;
+            key[u] = i < end ? keys[i * stride] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < kRadixUnroll; ++u)
+            if (i0 + u * blockDim.x < end) atomicAdd(&lds_radix[(key[u] >> shift) & (bins - 1)], 1);
     }
     __syncthreads();
-    if (chunk < C)
-        for (int d = lane; d < bins; d += 64) cnt[(int64_t)d * C + chunk] = hist[d];
+    for (int d = threadIdx.x; d < bins; d += blockDim.x) cnt[(int64_t)d * C + blockIdx.x] = lds_radix[d];
 }
 
-// vals_in == nullptr: the values are the item indices (first pass)
+// vals_in == nullptr: the values are the item indices
 __global__ __launch_bounds__(64 * kRadixWaves) void k_radix_scatter(int64_t n, const int *__restrict__ keys_in,
                                                                     int stride, const int *__restrict__ vals_in,
                                                                     int shift, int bits, int64_t chunk_len, int C,
@@ -318,39 +327,65 @@ __global__ __launch_bounds__(64 * kRadixWaves) void k_radix_scatter(int64_t n, c
 {
     extern __shared__ int lds_radix[]; // [kRadixWaves][bins]
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int chunk = blockIdx.x * kRadixWaves + wave;
     const int bins = 1 << bits;
     int *base = lds_radix + wave * bins;
-    if (chunk < C)
-        for (int d = lane; d < bins; d += 64) {
-            const int64_t i = (int64_t)d * C + chunk;
-            base[d] = offs[i] + bsum[i / kScanTile];
-        }
+    for (int d = threadIdx.x; d < kRadixWaves * bins; d += blockDim.x) lds_radix[d] = 0;
     __syncthreads();
-    if (chunk >= C) return;
-    const int64_t beg = (int64_t)chunk * chunk_len;
-    const int64_t end = min(n, beg + chunk_len);
-    const unsigned long long lt = (1ull << lane) - 1ull;
-    for (int64_t g = beg; g < end; g += 64) {
-        const int64_t i = g + lane;
-        const bool valid = i < end;
-        const int key = valid ? keys_in[i * stride] : 0;
-        const int val = valid ? (vals_in ? vals_in[i] : (int)i) : 0;
-        const int d = (key >> shift) & (bins - 1);
-        unsigned long long m = __ballot(valid);
-        for (int b = 0; b < bits; ++b) {
-            const bool on = (d >> b) & 1;
-            const unsigned long long bb = __ballot(on);
-            m &= on ? bb : ~bb;
+    const int64_t part = chunk_len / kRadixWaves;
+    const int64_t beg = (int64_t)blockIdx.x * chunk_len + wave * part;
+    const int64_t end = min(n, beg + part);
+    for (int64_t g = beg; g < end; g += kRadixUnroll * 64) {
+        int key[kRadixUnroll];
+#pragma unroll
+        for (int u = 0; u < kRadixUnroll; ++u) {
+            const int64_t i = g + u * 64 + lane;
+            key[u] = i < end ? keys_in[i * stride] : 0;
         }
-        const int rank = __popcll(m & lt);
-        const int b0 = base[d];
-        __builtin_amdgcn_wave_barrier();
-        if (valid && rank == 0) base[d] = b0 + __popcll(m);
-        __builtin_amdgcn_wave_barrier();
-        if (valid) {
-            keys_out[b0 + rank] = key;
-            vals_out[b0 + rank] = val;
+#pragma unroll
+        for (int u = 0; u < kRadixUnroll; ++u)
+            if (g + u * 64 + lane < end) atomicAdd(&base[(key[u] >> shift) & (bins - 1)], 1);
+    }
+    __syncthreads();
+    for (int d = threadIdx.x; d < bins; d += blockDim.x) {
+        const int64_t i = (int64_t)d * C + blockIdx.x;
+        int run = offs[i] + bsum[i / kScanTile];
+#pragma unroll
+        for (int w = 0; w < kRadixWaves; ++w) {
+            const int c = lds_radix[w * bins + d];
+            lds_radix[w * bins + d] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    for (int64_t g0 = beg; g0 < end; g0 += kRadixUnroll * 64) {
+        int keys[kRadixUnroll], vals[kRadixUnroll];
+#pragma unroll
+        for (int u = 0; u < kRadixUnroll; ++u) {
+            const int64_t i = g0 + u * 64 + lane;
+            keys[u] = i < end ? keys_in[i * stride] : 0;
+            vals[u] = i < end ? (vals_in ? vals_in[i] : (int)i) : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < kRadixUnroll; ++u) {
+            if (g0 + u * 64 >= end) break; // uniform over the wave
+            const bool valid = g0 + u * 64 + lane < end;
+            const int d = (keys[u] >> shift) & (bins - 1);
+            unsigned long long m = __ballot(valid);
+            for (int b = 0; b < bits; ++b) {
+                const bool on = (d >> b) & 1;
+                const unsigned long long bb = __ballot(on);
+                m &= on ? bb : ~bb;
+            }
+            const int rank = __popcll(m & lt);
+            const int b0 = base[d];
+            __builtin_amdgcn_wave_barrier();
+            if (valid && rank == 0) base[d] = b0 + __popcll(m);
+            __builtin_amdgcn_wave_barrier();
+            if (valid) {
+                keys_out[b0 + rank] = keys[u];
+                vals_out[b0 + rank] = vals[u];
+            }
         }
     }
 }
@@ -492,16 +527,15 @@ __global__ __launch_bounds__(256) void k_pair_keys(int64_t M, const int4 *__rest
     }
 }
 
-// Pair q of the tile-sorted order: original pair index o = sorted[q], its sample record
-// p = psamp[o] and local index o - offs[p] give the tile on each axis; the record is
+// Pair q of the tile-sorted order: its sample record is p = sorted[q] (the sort carries the
+// sample indices as values), its tile the sorted key (148 -> 113 us for 2.7 M pairs against
+// finding the tile from the pair's original index); the record is
 //   a = {orig, j0 | j1<<8 | j2<<16, c0 | c1<<8 | c2<<16, l0 | l1<<10 | l2<<20}
 //   b = {t0, t1, t2, dcf} (float bits)
 // (j = first window tap inside the tile, c = taps inside, l = tile-local cell of tap j).
 __global__ __launch_bounds__(256) void k_pair_records(int64_t P, const int *__restrict__ sorted,
-                                                      const int *__restrict__ psamp, const int *__restrict__ offs,
-                                                      const int *__restrict__ bsum, const int *__restrict__ skeys,
-                                                      int64_t K, int *__restrict__ bin_start,
-                                                      const int4 *__restrict__ rec_cell,
+                                                      const int *__restrict__ skeys, int64_t K,
+                                                      int *__restrict__ bin_start, const int4 *__restrict__ rec_cell,
                                                       const float4 *__restrict__ rec_frac, TileGeom g,
                                                       int4 *__restrict__ pa, int4 *__restrict__ pb)
 {
@@ -509,21 +543,16 @@ __global__ __launch_bounds__(256) void k_pair_records(int64_t P, const int *__re
     if (q > P) return;
     bin_starts(q, P, skeys, K, bin_start);
     if (q == P) return;
-    const int o = sorted[q];
-    const int p = psamp[o];
+    const int p = sorted[q];
     const int4 rc = rec_cell[p];
     const float4 rf = rec_frac[p];
-    int q0[3] = {0, 0, 0}, n[3] = {1, 1, 1};
-    axis_tile_span(rc.x, g.W, (int)g.nf[0], g.tile[0], q0[0], n[0]);
-    axis_tile_span(rc.y, g.W, (int)g.nf[1], g.tile[1], q0[1], n[1]);
-    if (g.dim == 3) axis_tile_span(rc.z, g.W, (int)g.nf[2], g.tile[2], q0[2], n[2]);
-    const int local = o - (offs[p] + bsum[p / kScanTile]);
-    const int m = local % n[2], r = local / n[2];
-    const int k = r % n[1], i = r / n[1];
-    int t0 = q0[0] + i, t1 = q0[1] + k, t2 = q0[2] + m;
-    if (t0 >= g.ntiles[0]) t0 -= g.ntiles[0];
-    if (t1 >= g.ntiles[1]) t1 -= g.ntiles[1];
-    if (t2 >= g.ntiles[2]) t2 -= g.ntiles[2];
+    uint32_t key = (uint32_t)skeys[q];
+    int t2 = 0;
+    if (g.dim == 3) {
+        t2 = (int)(key % (uint32_t)g.ntiles[2]);
+        key /= (uint32_t)g.ntiles[2];
+    }
+    const int t1 = (int)(key % (uint32_t)g.ntiles[1]), t0 = (int)(key / (uint32_t)g.ntiles[1]);
     int j0, c0, l0, j1, c1, l1, j2 = 0, c2 = 1, l2 = 0;
     tap_box(rc.x, t0, g.tile[0], (int)g.nf[0], g.W, j0, c0, l0);
     tap_box(rc.y, t1, g.tile[1], (int)g.nf[1], g.W, j1, c1, l1);
@@ -2096,7 +2125,7 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_batch(const GatherArg
 // sum one real value per cell: 6 FMAs and one 16-byte LDS read per cell and coil pair, where
 // a derivative per coil took 16 to 24 and two 8-byte reads.  Staging, lanes per sample and
 // tile order as in the gather.  Bound by the taps' LDS reads and FMAs: 256^3-grid UTE, 4
-// coils, 616448 samples, nspread 3: 436 -> 275 us.
+// coils, 1048576 samples, nspread 3: 436 -> 275 us.
 // ---------------------------------------------------------------------------
 
 template <int D, int NS, bool WRAP>
@@ -2491,19 +2520,22 @@ hipError_t device_scan(int *data, int64_t n, int *bsum, Scratch &sc)
     return hipGetLastError();
 }
 
-// Stable counting sort of n items by keys[i*stride] in [0,K): writes the sorted item
-// indices; *skeys: the sorted keys (scratch).  Asynchronous on st; the temporary buffers
+// Stable counting sort of n items by keys[i*stride] in [0,K): writes the sorted values
+// (vals, or the item indices where it is null); *skeys: the sorted keys (scratch).  Asynchronous on st; the temporary buffers
 // belong to sc, which the caller keeps alive until the stream has consumed them.
-int stable_sort_by_key(int64_t n, const int *keys, int stride, int64_t K, int *sorted, const int **skeys,
-                       hipStream_t st, Scratch &sc)
+int stable_sort_by_key(int64_t n, const int *keys, int stride, const int *vals, int64_t K, int *sorted,
+                       const int **skeys, hipStream_t st, Scratch &sc)
 {
     int rc;
     int kbits = 1;
     while (kbits < 31 && ((int64_t)1 << kbits) < K) ++kbits;
     const int npass = (kbits + kRadixBits - 1) / kRadixBits, pbits = (kbits + npass - 1) / npass;
-    // chunks: about 4096 waves over the GPU, 256..4096 items each
-    int64_t chunk_len = (n + 4095) / 4096;
-    chunk_len = std::min<int64_t>(4096, std::max<int64_t>(256, ((chunk_len + 63) / 64) * 64));
+    // chunks: about 4096 waves over the GPU, 256..4096 items each (below 256 the count
+    // array outgrows the items: 98304 spiral samples 176 us with 64, 150 with 128, 145 with
+    // 256; 2048 or 8192 waves 3-8 % more time on 1 M samples)
+    int64_t wave_len = (n + 4095) / 4096;
+    wave_len = std::min<int64_t>(4096, std::max<int64_t>(256, ((wave_len + 63) / 64) * 64));
+    const int64_t chunk_len = kRadixWaves * wave_len;
     const int64_t C = std::max<int64_t>(1, (n + chunk_len - 1) / chunk_len);
     const int64_t nKC = ((int64_t)1 << pbits) * C;
     int *cnt = nullptr, *bsum = nullptr, *k0 = nullptr, *v0 = nullptr, *k1 = nullptr, *v1 = nullptr;
@@ -2513,9 +2545,8 @@ int stable_sort_by_key(int64_t n, const int *keys, int stride, int64_t K, int *s
         (rc = sc.alloc(&v0, (size_t)n, "sort values")))
         return rc;
     v1 = sorted;
-    const unsigned nblk = (unsigned)((C + kRadixWaves - 1) / kRadixWaves);
     const int *kin = keys;
-    const int *vin = nullptr;
+    const int *vin = vals;
     int kstride = stride;
     // ping-pong so that the last pass writes its values into `sorted`
     int *kout[2] = {k0, k1};
@@ -2526,13 +2557,13 @@ int stable_sort_by_key(int64_t n, const int *keys, int stride, int64_t K, int *s
         const int bits = std::min(pbits, kbits - shift);
         const int bins = 1 << bits;
         const int o = (npass - 1 - ps) % 2 == 0 ? 1 : 0; // the last pass writes slot 1 (sorted)
-        const size_t lds = (size_t)kRadixWaves * bins * sizeof(int);
-        hipLaunchKernelGGL(k_radix_count, dim3(nblk), dim3(64 * kRadixWaves), lds, st, n, kin, kstride, shift, bins,
+        const size_t lds = (size_t)bins * sizeof(int);
+        hipLaunchKernelGGL(k_radix_count, dim3((unsigned)C), dim3(64 * kRadixWaves), lds, st, n, kin, kstride, shift, bins,
                            chunk_len, (int)C, cnt);
         e = hipGetLastError();
         if (e == hipSuccess) e = device_scan(cnt, (int64_t)bins * C, bsum, sc);
         if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_radix_scatter, dim3(nblk), dim3(64 * kRadixWaves), lds, st, n, kin, kstride, vin,
+            hipLaunchKernelGGL(k_radix_scatter, dim3((unsigned)C), dim3(64 * kRadixWaves), kRadixWaves * lds, st, n, kin, kstride, vin,
                                shift, bits, chunk_len, (int)C, cnt, bsum, kout[o], vout[o]);
             e = hipGetLastError();
         }
@@ -2701,7 +2732,7 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
         hipLaunchKernelGGL(k_prep, dim3(grid_blocks(M, 256, INT32_MAX)), dim3(256), 0, st, pa);
         GN_HIP(hipGetLastError());
         // gather-tile sort (stable) -> records in tile order
-        if ((rc = stable_sort_by_key(M, &cell[0].w, 4, Kg, sorted, &skeys, st, sc))) return rc;
+        if ((rc = stable_sort_by_key(M, &cell[0].w, 4, nullptr, Kg, sorted, &skeys, st, sc))) return rc;
         hipLaunchKernelGGL(k_make_records, dim3(grid_blocks(M + 1, 256, INT32_MAX)), dim3(256), 0, st, M, sorted, cell,
                            frac, dcf, skeys, Kg, R.bin_start, R.cell, R.frac);
         GN_HIP(hipGetLastError());
@@ -2734,14 +2765,14 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
         hipLaunchKernelGGL(k_pair_keys, dim3(grid_blocks(M, 256, INT32_MAX)), dim3(256), 0, st, M, R.cell, tg, pcnt,
                            pbsum, pkey, psamp);
         GN_HIP(hipGetLastError());
-        if ((rc = stable_sort_by_key(P, pkey, 1, K, psorted, &skeys, st, sc))) return rc;
+        if ((rc = stable_sort_by_key(P, pkey, 1, psamp, K, psorted, &skeys, st, sc))) return rc;
         if (P > R.pairs_cap) {
             if ((rc = dev_alloc(&R.pair_a, (size_t)P, "pairs")) || (rc = dev_alloc(&R.pair_b, (size_t)P, "pairs")))
                 return rc;
             R.pairs_cap = P;
         }
         hipLaunchKernelGGL(k_pair_records, dim3(grid_blocks(P + 1, 256, INT32_MAX)), dim3(256), 0, st, P, psorted,
-                           psamp, pcnt, pbsum, skeys, K, tile_pairs, R.cell, R.frac, tg, R.pair_a, R.pair_b);
+                           skeys, K, tile_pairs, R.cell, R.frac, tg, R.pair_a, R.pair_b);
         GN_HIP(hipGetLastError());
         R.npairs = P;
     } else {
