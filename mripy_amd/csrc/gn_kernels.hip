@@ -1528,18 +1528,21 @@ __global__ __launch_bounds__(64) void k_spread_tile_batch(const SpreadArgs *__re
 // and NG matrix products whose columns are the reals of 8 coils.  A window of 6 cells
 // fills 0.44 of a 4 x 4 block it reaches, against 0.22 of an 8 x 8 block, so the products
 // are half of k_spread_mfma's; the tables and records serve up to 32 coils.
-// Bound by the matrix cores and, at few coils, by the latency of the batches: 256^2, 98304
-// spiral samples, nspread 3, with equal work items: 32 coils 107 -> 82 us, 8 coils
-// 43 -> 36 us.
+// Bound by the batches' vector instructions and latency (matrix cores about 0.4 busy), so a
+// batch's records are held a pair per lane: a wave forms one quad of weights of every pair
+// without divisions, tests its own sub-blocks, and takes values' sample indices by lane
+// exchange; two list steps' LDS reads are in flight together; 6 waves per SIMD.  256^2,
+// 98304 spiral samples, nspread 3 (spread and reduction): 32 coils 112 (8 x 8 blocks) -> 65
+// -> 60 us, 8 coils 34 -> 30 us; 16 instances of 128 to 320 with up to 32 coils, forward and
+// adjoint, 1579 -> 1485 us.
 // LDS rows, one per pair: weights x[8] y[16] | reals [16 NG]; row B is zero (list padding).
 // ---------------------------------------------------------------------------
 constexpr int kSpreadSubWaves = 4;
-constexpr int spread_sub_row(int NG) { return 24 + 16 * NG; }
+constexpr int spread_sub_row(int NG) { return 28 + 16 * NG; } // 4 floats of padding: 16 banks of 16 bytes
 
 inline size_t spread_sub_lds(int NG)
 {
-    return (size_t)(kSpreadBatch + 1) * spread_sub_row(NG) * 4 + (size_t)kSpreadBatch * 4 +
-           (size_t)kSpreadSubWaves * 2 * kSpreadBatch * 4;
+    return (size_t)(kSpreadBatch + 1) * spread_sub_row(NG) * 4 + (size_t)kSpreadSubWaves * 2 * kSpreadBatch * 4;
 }
 
 template <int NG>
@@ -1551,8 +1554,7 @@ __device__ __forceinline__ void spread_sub_body(const SpreadArgs &a, const int4 
     if (tile_skippable(a, item)) return; // uniform over the workgroup
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int *s_msk = (int *)(lds_sp + (B + 1) * ROW);
-    int *s_list = s_msk + B + wave * 2 * B;
+    int *s_list = (int *)(lds_sp + (B + 1) * ROW) + wave * 2 * B;
     const int cg0 = cgi * NC;
     const int ncg = (int)min((int64_t)NC, a.nc - cg0);
     const int ri = lane & 15, kg = lane >> 4;
@@ -1570,72 +1572,79 @@ __device__ __forceinline__ void spread_sub_body(const SpreadArgs &a, const int4 
             for (int v = 0; v < 4; ++v) S[s][g][v] = K[s][g][v] = 0.f;
     for (int base = item.y; base < item.z; base += B) {
         const int n = min(B, item.z - base);
-        if (base != item.y) __syncthreads(); // previous batch fully consumed (uniform)
-        // values: one 16-byte coil pair per step
-        for (int q = tid; q < n * (NC / 2); q += NT) {
-            const int k = q / (NC / 2), c = 2 * (q - k * (NC / 2));
-            const int orig = a.pair_a[base + k].x;
-            const float scale = a.use_dcf ? __int_as_float(a.pair_b[base + k].w) : 1.0f;
-            float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (v4) {
-                if (c < ncg) t = *reinterpret_cast<const float4 *>(a.in + (int64_t)orig * a.nc + cg0 + c);
-            } else {
-                float2 x = make_float2(0.f, 0.f), y = x;
-                if (c < ncg) x = a.layout == GN_COIL_LAST ? a.in[(int64_t)orig * a.nc + cg0 + c] : a.in[(int64_t)(cg0 + c) * a.M + orig];
-                if (c + 1 < ncg) y = a.layout == GN_COIL_LAST ? a.in[(int64_t)orig * a.nc + cg0 + c + 1] : a.in[(int64_t)(cg0 + c + 1) * a.M + orig];
-                t = make_float4(x.x, x.y, y.x, y.y);
-            }
-            *(float4 *)(lds_sp + k * ROW + 24 + 2 * c) = make_float4(t.x * scale, t.y * scale, t.z * scale, t.w * scale);
+        // every wave holds the batch's records, a pair per lane
+        int4 pa = make_int4(0, 0, 0, 0), pb = pa;
+        if (lane < n) {
+            pa = a.pair_a[base + lane];
+            pb = a.pair_b[base + lane];
         }
-        // weight tables: 4 consecutive tile-local cells of one axis per step; the first
-        // step of a pair also forms its sub-block masks (x halves | y quarters << 2)
-        for (int q = tid; q < n * 6; q += NT) {
-            const int k = q / 6, e = q - k * 6, ax = e < 2 ? 0 : 1;
+        // values: one 16-byte coil pair per step, loaded before the weights are formed
+        constexpr int NV = B * (NC / 2) / NT;
+        float4 val[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int q = tid + v * NT, k = q / (NC / 2), c = 2 * (q - k * (NC / 2));
+            const int orig = __shfl(pa.x, k);
+            float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (k < n) {
+                if (v4) {
+                    if (c < ncg) t = *reinterpret_cast<const float4 *>(a.in + (int64_t)orig * a.nc + cg0 + c);
+                } else {
+                    float2 x = make_float2(0.f, 0.f), y = x;
+                    if (c < ncg) x = a.layout == GN_COIL_LAST ? a.in[(int64_t)orig * a.nc + cg0 + c] : a.in[(int64_t)(cg0 + c) * a.M + orig];
+                    if (c + 1 < ncg) y = a.layout == GN_COIL_LAST ? a.in[(int64_t)orig * a.nc + cg0 + c + 1] : a.in[(int64_t)(cg0 + c + 1) * a.M + orig];
+                    t = make_float4(x.x, x.y, y.x, y.y);
+                }
+            }
+            val[v] = t;
+        }
+        if (base != item.y) __syncthreads(); // previous batch fully consumed (uniform)
+        // weight tables: wave w forms quads e = w, w + 4 of 4 consecutive tile-local cells of
+        // one axis (two along x, four along y) for the pair of each lane
+#pragma unroll
+        for (int e = wave; e < 6; e += kSpreadSubWaves) {
+            const int ax = e < 2 ? 0 : 1;
             const int L0 = 4 * (ax ? e - 2 : e), T = ax ? T1 : T0;
-            const int4 pa = a.pair_a[base + k], pb = a.pair_b[base + k];
             const int l = (pa.w >> (10 * ax)) & 0x3ff, c = (pa.z >> (8 * ax)) & 0xff;
             const int j = a.ns - ((pa.y >> (8 * ax)) & 0xff);
             const float t = __int_as_float(ax ? pb.y : pb.x), coef = ax ? a.coef[1] : a.coef[0];
-            int rel0 = L0 - l; // (L - l) mod T of the quad's first cell
-            if (rel0 < 0) rel0 += T;
+            const int rel0 = (L0 - l) & (T - 1); // (L - l) mod T of the quad's first cell
             float w[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                int rel = rel0 + i;
-                if (i > 0 && rel >= T) rel -= T;
+                const int rel = (rel0 + i) & (T - 1);
                 const float u = t + (float)(j - rel);
                 const float g = __builtin_amdgcn_exp2f(-coef * u * u);
                 w[i] = rel < c ? g : 0.f;
             }
-            *(float4 *)(lds_sp + k * ROW + 4 * e) = make_float4(w[0], w[1], w[2], w[3]);
-            if (e == 0) {
-                uint32_t h = 0;
-#pragma unroll
-                for (int x = 0; x < 2; ++x) {
-                    const int lx = x ? (pa.w >> 10) & 0x3ff : pa.w & 0x3ff, cx = x ? (pa.z >> 8) & 0xff : pa.z & 0xff;
-                    const int Tx = x ? T1 : T0;
-                    uint64_t m = ((1ull << cx) - 1) << lx; // window cells (L - l) mod T < c
-                    m = (m | (m >> Tx)) & ((1ull << Tx) - 1);
-#pragma unroll
-                    for (int b = 0; b < (x ? 4 : 2); ++b)
-                        if ((m >> (4 * b)) & 0xf) h |= 1u << ((x ? 2 : 0) + b);
-                }
-                s_msk[k] = (int)h;
-            }
+            if (lane < n) *(float4 *)(lds_sp + lane * ROW + 4 * e) = make_float4(w[0], w[1], w[2], w[3]);
         }
-        __syncthreads();
-        const uint32_t h = lane < n ? (uint32_t)s_msk[lane] : 0u;
-        const bool hy = (h >> (2 + wave)) & 1u;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int q = tid + v * NT, k = q / (NC / 2), c = 2 * (q - k * (NC / 2));
+            const float scale = a.use_dcf ? __int_as_float(__shfl(pb.w, k)) : 1.0f;
+            if (k < n)
+                *(float4 *)(lds_sp + k * ROW + 24 + 2 * c) =
+                    make_float4(val[v].x * scale, val[v].y * scale, val[v].z * scale, val[v].w * scale);
+        }
+        // pairs that reach this wave's sub-blocks: window cells are (l + i) mod T, i < c, so a
+        // block at b is reached when (b - l) mod T is below c or its 4 cells pass T
+        const int ly = (4 * wave - (pa.w >> 10)) & (T1 - 1);
+        const bool hy = lane < n && (ly < ((pa.z >> 8) & 0xff) || ly > T1 - 4);
         int cnt[2];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            const bool hit = hy && ((h >> s) & 1u);
+            const int lx = (4 * s - pa.w) & (T0 - 1);
+            const bool hit = hy && (lx < (pa.z & 0xff) || lx > T0 - 4);
             const unsigned long long hm = __ballot(hit);
             cnt[s] = __popcll(hm);
-            const int pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0));
-            if (hit) s_list[s * B + pos] = lane * (ROW * 4);
-            if (lane >= cnt[s] && lane < ((cnt[s] + 3) & ~3)) s_list[s * B + lane] = B * (ROW * 4);
+            const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(hm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hm, 0));
+            // listed pairs first, then the zero row; entry i of the list is the row of step
+            // i / 4 and k group i % 4, kept as 16 steps per k group
+            const int i = hit ? rank : cnt[s] + lane - rank;
+            s_list[s * B + (i & 3) * (B / 4) + (i >> 2)] = (hit ? lane : B) * (ROW * 4);
         }
+        __syncthreads();
         // the lists were written by this wave's own lanes: order the LDS accesses
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 #pragma unroll
@@ -1643,13 +1652,22 @@ __device__ __forceinline__ void spread_sub_body(const SpreadArgs &a, const int4 
             f32x4 acc[NG];
 #pragma unroll
             for (int g = 0; g < NG; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
-            const int *lst = s_list + s * B + kg;
-            for (int t = 0; t < cnt[s]; t += 4) {
-                const int off = lst[t]; // byte offset of the pair's row
-                const float w = *(const float *)(qx + 16 * s + off) * *(const float *)(qy + off);
+            // two steps of 4 pairs together: their LDS reads are in flight at once
+            const int *lst = s_list + s * B + kg * (B / 4);
+            for (int t = 0; t < cnt[s]; t += 8) {
+                const int2 off = *(const int2 *)(lst + (t >> 2)); // byte offsets of the pairs' rows
+                const float w0 = *(const float *)(qx + 16 * s + off.x) * *(const float *)(qy + off.x);
+                const float w1 = *(const float *)(qx + 16 * s + off.y) * *(const float *)(qy + off.y);
+                float v0[NG], v1[NG];
 #pragma unroll
-                for (int g = 0; g < NG; ++g)
-                    acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, *(const float *)(qv + 64 * g + off), acc[g], 0, 0, 0);
+                for (int g = 0; g < NG; ++g) {
+                    v0[g] = *(const float *)(qv + 64 * g + off.x);
+                    v1[g] = *(const float *)(qv + 64 * g + off.y);
+                }
+#pragma unroll
+                for (int g = 0; g < NG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(w0, v0[g], acc[g], 0, 0, 0);
+#pragma unroll
+                for (int g = 0; g < NG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(w1, v1[g], acc[g], 0, 0, 0);
             }
 #pragma unroll
             for (int g = 0; g < NG; ++g)
@@ -1705,7 +1723,7 @@ __device__ __forceinline__ void spread_sub_body(const SpreadArgs &a, const int4 
 }
 
 template <int NG>
-__global__ __launch_bounds__(64 * kSpreadSubWaves) void k_spread_sub(SpreadArgs a)
+__global__ __launch_bounds__(64 * kSpreadSubWaves, 6) void k_spread_sub(SpreadArgs a)
 {
     const uint32_t n = gridDim.x * gridDim.y;
     const uint32_t w = xcd_swizzle(blockIdx.x + gridDim.x * blockIdx.y, n);
