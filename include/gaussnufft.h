@@ -69,8 +69,8 @@ extern "C" {
 #define GN_GRID_GATHER 42    /* y_j = (1/G) sum_g w_j(g) grid[g]                            */
 
 /* FFT engines for gn_plan_set_fft_engine */
-#define GN_FFT_AUTO 0   /* pruned in-place passes fused with pad/crop when every nf is a product of
-                           2, 3 and 5 (<= 2048); rocFFT otherwise */
+#define GN_FFT_AUTO 0   /* pruned in-place passes fused with pad/crop when every nf is at most 2048
+                           without prime factors above 256; rocFFT otherwise */
 #define GN_FFT_ROCFFT 1 /* separate pad, rocFFT and crop */
 
 typedef struct gn_plan_s gn_plan;

@@ -276,8 +276,8 @@ class Plan:
         return out
 
     def set_fft_engine(self, engine="auto"):
-        """"auto": pruned FFT passes fused with pad/crop where every nf is a product of
-        2, 3 and 5; "rocfft": separate pad, rocFFT, crop."""
+        """"auto": pruned FFT passes fused with pad/crop where every nf is at most 2048
+        and has no prime factor above 256; "rocfft": separate pad, rocFFT, crop."""
         check(_lib.load().gn_plan_set_fft_engine(self._h, _lib.GN_FFT_ROCFFT if engine == "rocfft"
                                                  else _lib.GN_FFT_AUTO))
 
