@@ -22,6 +22,11 @@ struct Item {
 };
 static_assert(sizeof(Item) == 16, "work items are int4");
 
+// The device scans' grand total: block totals (or sums of them) modulo 2^32 added in 64
+// bits, and the same number from the two ints that return it to the host.
+constexpr int64_t scan_carry(int64_t carry, int total) { return carry + (int64_t)(uint32_t)total; }
+constexpr int64_t scan_total(int lo, int hi) { return (int64_t)((uint64_t)(uint32_t)hi << 32 | (uint32_t)lo); }
+
 // Default spread (output) and gather (home) tile shapes.  Wide windows shrink the
 // gather tile, largest axis first, until tile + halo of a coil pair fits 160 KiB.
 inline void default_tiles(int dim, int ns, const int64_t *nf, int *tile, int *gtile)

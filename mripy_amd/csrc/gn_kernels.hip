@@ -139,7 +139,7 @@ constexpr int kScanTile = kScanThreads * kScanItems;
 constexpr int kItemTile = kScanThreads * 4; // tiles per block of the work-item scan
 
 // Exclusive scan of N ints per thread over the 256 threads of the block (all threads call
-// it); total is the block's.
+// it); total is the block's, modulo 2^32.
 template <int N>
 __device__ inline void block_exclusive_scan(int (&x)[N], int (&total)[N])
 {
@@ -160,23 +160,27 @@ __device__ inline void block_exclusive_scan(int (&x)[N], int (&total)[N])
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < N; ++c) {
-        int before = 0, all = 0;
+        uint32_t before = 0, all = 0;
         for (int w = 0; w < kScanThreads / 64; ++w) {
-            const int t = s_wave[c][w];
+            const uint32_t t = (uint32_t)s_wave[c][w];
             before += w < wave ? t : 0;
             all += t;
         }
-        x[c] = inc[c] - x[c] + before;
-        total[c] = all;
+        x[c] = (int)((uint32_t)(inc[c] - x[c]) + before);
+        total[c] = (int)all;
     }
     __syncthreads(); // s_wave may be written again
 }
 
 // Publish this block's totals and, in the block that finishes last, turn all of them into
 // exclusive offsets; bsum holds (gridDim.x + 1) * N ints.  True in the last block, with the
-// grand totals in total (thread 0).  The ticket is left at zero for the next scan.
+// grand totals in grand (thread 0).  The ticket is left at zero for the next scan.
+// The grand totals are 64-bit, so that a caller can refuse one that does not fit an int
+// (the offsets past it are modulo 2^32): a sample has at most 16^3 (tile, sample) pairs, so
+// a tile of the scan totals at most 2^23 and 256 of them at most 2^31, which scan_carry adds
+// as an unsigned number.
 template <int N>
-__device__ inline bool scan_block_totals(int *bsum, int *ticket, int (&total)[N])
+__device__ inline bool scan_block_totals(int *bsum, int *ticket, const int (&total)[N], int64_t (&grand)[N])
 {
     __shared__ int s_last;
     if (threadIdx.x == 0) {
@@ -188,7 +192,7 @@ __device__ inline bool scan_block_totals(int *bsum, int *ticket, int (&total)[N]
     }
     __syncthreads();
     if (!s_last) return false;
-    int carry[N] = {};
+    int64_t carry[N] = {};
     const int64_t nb = gridDim.x;
     for (int64_t b0 = 0; b0 < nb; b0 += kScanThreads) {
         const int64_t i = b0 + threadIdx.x;
@@ -199,23 +203,23 @@ __device__ inline bool scan_block_totals(int *bsum, int *ticket, int (&total)[N]
         block_exclusive_scan<N>(x, all);
 #pragma unroll
         for (int c = 0; c < N; ++c) {
-            if (i < nb) bsum[i * N + c] = x[c] + carry[c];
-            carry[c] += all[c];
+            if (i < nb) bsum[i * N + c] = (int)((uint32_t)x[c] + (uint32_t)carry[c]);
+            carry[c] = host::scan_carry(carry[c], all[c]);
         }
     }
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int c = 0; c < N; ++c) {
-            bsum[nb * N + c] = carry[c];
-            total[c] = carry[c];
+            bsum[nb * N + c] = (int)carry[c];
+            grand[c] = carry[c];
         }
         *ticket = 0;
     }
     return true;
 }
 
-// data[i] = exclusive scan within the tile of load(i), i < n.  ret (null: none): ret[0] =
-// the grand total, ret[1] = *err.
+// data[i] = exclusive scan within the tile of load(i), i < n.  ret (null: none): ret[0],
+// ret[1] = the grand total's low and high half, ret[2] = *err.
 template <typename F>
 __device__ inline void scan_tile(F load, int *__restrict__ data, int64_t n, int *bsum, int *ticket, int *ret, int *err)
 {
@@ -255,9 +259,11 @@ __device__ inline void scan_tile(F load, int *__restrict__ data, int64_t n, int 
         const int i = k * kScanThreads + threadIdx.x;
         if (base + i < n) data[base + i] = sv[i];
     }
-    if (scan_block_totals<1>(bsum, ticket, total) && ret && threadIdx.x == 0) {
-        ret[0] = total[0];
-        ret[1] = *err;
+    int64_t grand[1];
+    if (scan_block_totals<1>(bsum, ticket, total, grand) && ret && threadIdx.x == 0) {
+        ret[0] = (int)(uint32_t)grand[0];
+        ret[1] = (int)(grand[0] >> 32);
+        ret[2] = *err;
     }
 }
 
@@ -594,8 +600,9 @@ __global__ __launch_bounds__(kScanThreads) void k_item_scan(int64_t K, const int
 #pragma unroll
         for (int j = 0; j < 4; ++j) sum[j] += c[i][j];
     }
-    if (scan_block_totals<4>(bsum, ticket, total) && threadIdx.x == 0)
-        for (int j = 0; j < 4; ++j) ret[j] = total[j];
+    int64_t grand[4];
+    if (scan_block_totals<4>(bsum, ticket, total, grand) && threadIdx.x == 0)
+        for (int j = 0; j < 4; ++j) ret[j] = (int)grand[j]; // at most tiles + pairs / chunk
 }
 
 // reduce null: gather items (none for empty tiles).  bsum: the block offsets of
@@ -2471,7 +2478,7 @@ struct ScratchPool {
         return GN_OK;
     }
 };
-enum { kRetPairs = 0, kRetErr = 1, kRetSpread = 4, kRetGather = 8 };
+enum { kRetPairs = 0, kRetErr = 2, kRetSpread = 4, kRetGather = 8 };
 
 ScratchPool &scratch_pool()
 {
@@ -2774,7 +2781,7 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
         GN_HIP(hipGetLastError());
         GN_HIP(hipStreamSynchronize(st));
         if (ret[kRetErr] == p->points_seq) return fail(GN_EINVAL, "non-finite sample coordinate");
-        const int64_t P = (int64_t)(unsigned)ret[kRetPairs];
+        const int64_t P = host::scan_total(ret[kRetPairs], ret[kRetPairs + 1]);
         if (P > (int64_t)INT32_MAX) return fail(GN_EINVAL, "too many (tile, sample) pairs");
         int *pkey = nullptr, *psamp = nullptr, *psorted = nullptr;
         if ((rc = sc.alloc(&pkey, (size_t)P, "pairs")) || (rc = sc.alloc(&psamp, (size_t)P, "pairs")) ||
