@@ -214,79 +214,90 @@ int axis_table(int dev, int L, FFTAxis **ax)
     return GN_OK;
 }
 
-// The axis passes apply: every length is 1 or covered, and the output is the input or
-// does not overlap it.
+// Lines (columns x slabs) a block of the axis pass may hold: 16, fewer while they exceed
+// kAxisLdsMax.
+int axis_lines(int L)
+{
+    int lines = kAxisLines;
+    while (lines > 1 && col_lds(L, lines, host::fft_direct_sums(L)) > kAxisLdsMax) lines /= 2;
+    return lines;
+}
+
+// The axis passes apply: every length is 1 or covered, the output is the input or does not
+// overlap it, and the blocks of every axis fit one launch (an axis of length L takes up to
+// about 2^27 L elements; larger arrays are left to rocFFT, whose shift passes loop).
 bool axis_passes_ok(int rank, const int64_t *n, int64_t total, const void *in, const void *out)
 {
     bool any = false;
+    int64_t slabs = 1;
     for (int a = 0; a < rank; ++a) {
         if (n[a] == 1) continue;
         if (!fft_length_supported(n[a])) return false;
+        const auto sp = host::axis_split(slabs, total / (slabs * n[a]), axis_lines((int)n[a]), kAxisBlocks);
+        if (!host::launch_fits(sp.blocks, kAxisThreads)) return false;
         any = true;
+        slabs *= n[a];
     }
     const uintptr_t i = (uintptr_t)in, o = (uintptr_t)out, bytes = (uintptr_t)total * sizeof(float2);
     const bool overlap = i != o && i < o + bytes && o < i + bytes;
-    return any && !overlap && total < ((int64_t)1 << 40);
+    return any && !overlap;
 }
 
+// Everything that can fail is done for every axis before the first launch: a pass
+// overwrites the output, which may be the input.
 int axis_passes(const ShiftArgs &sh, bool fwd, const float2 *in, float2 *out, hipStream_t st)
 {
     int dev = 0;
     (void)hipGetDevice(&dev);
-    int last = sh.rank - 1;
-    while (sh.n[last] == 1) --last;
-    const float2 *src = in;
+    AxisArgs pass[3];
+    unsigned blocks[3];
+    int np = 0;
     int64_t slabs = 1;
-    for (int ax = 0; ax <= last; ++ax) {
+    for (int ax = 0; ax < sh.rank; ++ax) {
         const int64_t n = sh.n[ax];
         if (n == 1) continue;
         FFTAxis *t = nullptr;
         const int rc = axis_table(dev, (int)n, &t);
         if (rc) return rc;
-        AxisArgs a;
-        a.src = src;
+        AxisArgs &a = pass[np];
+        a.src = np ? out : in;
         a.dst = out;
         a.L = (int)n;
         a.nslabs = slabs;
         a.ncols = sh.total / (slabs * n);
-        const bool even = (a.ncols & 1) == 0;
         a.st = make_stages(*t);
-        int lines = kAxisLines;
-        while (lines > 1 && col_lds(a.L, lines, a.st.dbl) > kAxisLdsMax) lines /= 2;
-        if (a.ncols >= lines) {
-            a.C = lines;
-            a.S = 1;
-            while (a.C > 4 && (a.ncols + a.C - 1) / a.C * slabs < kAxisBlocks) a.C /= 2;
-        } else {
-            a.C = (int)a.ncols;
-            a.S = (int)std::min<int64_t>(lines / a.C, slabs);
-            while (a.S > 1 && (slabs + a.S - 1) / a.S < kAxisBlocks) a.S = (a.S + 1) / 2;
-        }
-        a.ncb = (a.ncols + a.C - 1) / a.C;
-        a.vec = even && a.C % 2 == 0 && (((uintptr_t)a.src | (uintptr_t)a.dst) & 15) == 0 ? 1 : 0;
+        const auto sp = host::axis_split(slabs, a.ncols, axis_lines(a.L), kAxisBlocks);
+        a.C = sp.C;
+        a.S = sp.S;
+        a.ncb = sp.ncb;
+        blocks[np] = (unsigned)sp.blocks;
+        a.vec = a.ncols % 2 == 0 && a.C % 2 == 0 && (((uintptr_t)a.src | (uintptr_t)a.dst) & 15) == 0 ? 1 : 0;
         // fftshift: input row n sits at position n + L/2; ifftshift: output row n is index n + L/2
         a.in_off = sh.pre ? a.L / 2 : 0;
         a.out_off = sh.post ? a.L / 2 : 0;
         a.sign = fwd ? -1.0f : 1.0f;
-        a.scale = ax == last ? sh.scale : 1.0f;
-        a.mask = ax == last ? sh.mask : nullptr;
+        a.scale = 1.0f;
+        a.mask = nullptr;
         a.mask_div = sh.mask_batch > 1 ? 1 : sh.batch;
         a.tw = t->tw;
         a.pinv = t->pinv;
-        const int64_t nblk = (slabs + a.S - 1) / a.S * a.ncb;
-        if (nblk >= ((int64_t)1 << 31)) return fail(GN_EINVAL, "gn_fft_c2c: array too large");
-        auto kernel = a.st.gen ? k_fft_axis<true> : k_fft_axis<false>;
         const size_t lds = col_lds(a.L, a.C * a.S, a.st.dbl);
-        hipError_t e = hipSuccess;
-        if (lds > kAxisLdsMax) // long lines with a second buffer
-            e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(kAxisThreads), lds, st, a);
-            e = hipGetLastError();
+        if (lds > kAxisLdsMax) { // long lines with a second buffer
+            const hipError_t e = hipFuncSetAttribute(a.st.gen ? (const void *)k_fft_axis<true> : (const void *)k_fft_axis<false>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return hip_fail(e, "FFT axis pass");
         }
-        if (e != hipSuccess) return hip_fail(e, "FFT axis pass");
-        src = out;
         slabs *= n;
+        ++np;
+    }
+    pass[np - 1].scale = sh.scale;
+    pass[np - 1].mask = sh.mask;
+    for (int k = 0; k < np; ++k) {
+        const AxisArgs &a = pass[k];
+        hipLaunchKernelGGL(a.st.gen ? k_fft_axis<true> : k_fft_axis<false>, dim3(blocks[k]), dim3(kAxisThreads),
+                           col_lds(a.L, a.C * a.S, a.st.dbl), st, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return hip_fail(e, "FFT axis pass");
     }
     return GN_OK;
 }

@@ -115,6 +115,41 @@ inline std::vector<int> fft_radices_prime(int L)
     return big;
 }
 
+// Whether a length has a prime factor above kFFTRadixMax (its lines need a second buffer).
+inline bool fft_direct_sums(int L)
+{
+    for (int p : {2, 3, 5, 7, 11, 13})
+        while (L % p == 0) L /= p;
+    return L > 1;
+}
+
+// HIP takes launches of fewer than 2^32 threads per grid axis.
+constexpr bool launch_fits(int64_t blocks, int threads) { return blocks < (((int64_t)1 << 32) + threads - 1) / threads; }
+
+// Blocks of a Cartesian FFT pass over (slabs, L, ncols): C columns of one slab, or S slabs of
+// all C = ncols columns where they are fewer than the lines a block may hold; fewer of either
+// while the launch has less than `want` blocks.
+struct AxisSplit {
+    int C, S;
+    int64_t ncb, blocks;
+};
+inline AxisSplit axis_split(int64_t slabs, int64_t ncols, int lines, int64_t want)
+{
+    AxisSplit s;
+    if (ncols >= lines) {
+        s.C = lines;
+        s.S = 1;
+        while (s.C > 4 && (ncols + s.C - 1) / s.C * slabs < want) s.C /= 2;
+    } else {
+        s.C = (int)ncols;
+        s.S = (int)std::min<int64_t>(lines / s.C, slabs);
+        while (s.S > 1 && (slabs + s.S - 1) / s.S < want) s.S = (s.S + 1) / 2;
+    }
+    s.ncb = (ncols + s.C - 1) / s.C;
+    s.blocks = (slabs + s.S - 1) / s.S * s.ncb;
+    return s;
+}
+
 // Digit-reversal map (pinv[position] = LDS slot) and twiddles e^{-2 pi i k/L}
 // (tw[2k], tw[2k+1]) of a length-L transform with radices r.
 inline void fft_tables(int L, const std::vector<int> &r, std::vector<int> &pinv, std::vector<float> &tw)

@@ -1,5 +1,5 @@
 // Size limits that the library checks on the host (mripy_amd/csrc/gn_host_plan.h), at sizes
-// too large to run: the pair total of set_points.  Built and run by
+// too large to run: the pair total of set_points, launches of the Cartesian FFT passes.  Built and run by
 // tests/test_host_limits.py with the undefined-behaviour sanitizer; prints "OK".
 #include <stdio.h>
 #include <stdlib.h>
@@ -42,9 +42,35 @@ static void check_pair_total()
             CHECK(scanned_total(samples, pairs) == samples * pairs);
 }
 
+// A launch has fewer than 2^32 threads; a split covers every line once.
+static void check_launches()
+{
+    for (int L = 1; L <= 2048; ++L) {
+        const std::vector<int> r = fft_radices_prime(L);
+        if (!r.empty()) CHECK(fft_direct_sums(L) == (*std::max_element(r.begin(), r.end()) > kFFTRadixMax));
+    }
+    for (int threads : {64, 256, 512, 1000, 1024}) {
+        const int64_t last = (((int64_t)1 << 32) - 1) / threads;
+        CHECK(launch_fits(last, threads) && !launch_fits(last + 1, threads));
+    }
+    for (int lines : {1, 2, 16})
+        for (int64_t slabs : {(int64_t)1, (int64_t)3, (int64_t)513, (int64_t)1 << 22, (int64_t)1 << 29})
+            for (int64_t ncols : {(int64_t)1, (int64_t)2, (int64_t)15, (int64_t)17, (int64_t)4096, ((int64_t)1 << 27) - 1, (int64_t)1 << 27}) {
+                const AxisSplit s = axis_split(slabs, ncols, lines, 512);
+                CHECK(s.C >= 1 && s.S >= 1 && (int64_t)s.C * s.S <= lines && (s.S == 1 || s.C == ncols));
+                CHECK(s.ncb * s.C >= ncols && (s.ncb - 1) * s.C < ncols && s.blocks % s.ncb == 0);
+                CHECK(s.blocks / s.ncb * s.S >= slabs && (s.blocks / s.ncb - 1) * s.S < slabs);
+            }
+    // 2 points x 2^28 and 16 x 512 x 512 x 512, 16 lines per block: too many blocks for a launch
+    CHECK(!launch_fits(axis_split(1, (int64_t)1 << 28, 16, 512).blocks, 512));
+    CHECK(!launch_fits(axis_split(1, (int64_t)512 * 512 * 512, 16, 512).blocks, 512));
+    CHECK(launch_fits(axis_split(1, ((int64_t)1 << 27) - 16, 16, 512).blocks, 512));
+}
+
 int main()
 {
     check_pair_total();
+    check_launches();
     printf("OK\n");
     return 0;
 }

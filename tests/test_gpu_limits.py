@@ -35,3 +35,22 @@ def test_pair_total_is_refused(M):
     y = _cnormal(rng, (300, 1))
     want = O.type1([c.astype(np.float64) for c in few], y.astype(np.complex128), O.Params((16, 16, 16), rat=2, nspread=8))
     assert rel(P.type1(y), want) <= TOL
+
+
+@pytest.mark.parametrize("n,batch", [(2, 1 << 28), (2, (1 << 27) - 16)])
+def test_cartesian_fft_of_many_columns(n, batch):
+    """2 points x 2^28 columns: more blocks than a launch of the axis passes takes (rocFFT),
+    and just as many as it takes.  Out of place and in place."""
+    import ctypes
+    import torch
+    from mripy_amd import _lib
+    from mripy_amd.cfft import _c2c
+    print("case: many columns", n, batch, flush=True)
+    x = torch.empty(n, batch, dtype=torch.complex64, device="cuda")
+    torch.view_as_real(x).random_(-8, 8)
+    want = torch.stack([x[0] + x[1], x[0] - x[1]])      # exact: small whole numbers
+    assert torch.equal(_c2c(x, 1, _lib.GN_FFT_FORWARD), want)
+    shp = (ctypes.c_int64 * 3)(n, 1, 1)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(_lib.load().gn_fft_c2c(1, shp, batch, _lib.GN_FFT_FORWARD, 0, None, 1, x.data_ptr(), x.data_ptr(), st))
+    assert torch.equal(x, want)
