@@ -247,6 +247,69 @@ template <int NDIM, int AMP> __device__ inline void tv_project(double2 *v)
     }
 }
 
+// A Chambolle step as two kernels, one thread per cell: D = Div(G) - y / lambda, then G.
+template <int NDIM> __device__ inline void tv_coords(const TVGeom &g, int idx, int *c)
+{
+    int r = idx / g.nt;
+    if (NDIM == 3) {
+        c[2] = r % g.s[2];
+        r /= g.s[2];
+    }
+    c[1] = r % g.s[1];
+    c[0] = r / g.s[1];
+}
+
+// adjD_a(p) at idx, position i of s on the axis
+__device__ inline double2 adj_at(const double2 *__restrict__ p, int i, int s, int stride, int idx)
+{
+    if (i == 0) return make_double2(-p[idx].x, -p[idx].y);
+    if (i == s - 1) return p[idx - stride];
+    return csub(p[idx - stride], p[idx]);
+}
+
+// D = Div(G) - y/lambda (FINAL: f = y - lambda*Div(G)).  first: G is zero.
+template <typename T, int NDIM, bool FINAL>
+__global__ __launch_bounds__(256) void k_tv_div(TVGeom g, const double2 *__restrict__ G, const T *__restrict__ y,
+                                                double lambda, int first, double2 *__restrict__ D, T *__restrict__ f)
+{
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= g.n) return;
+    int c[3];
+    tv_coords<NDIM>(g, idx, c);
+    const double2 yv = ld2<T>(y, idx);
+    double2 dv = make_double2(0.0, 0.0);
+    if (!first) {
+#pragma unroll
+        for (int a = 0; a < NDIM; ++a) dv = cadd(dv, adj_at(G + (int64_t)a * g.n, c[a], g.s[a], g.stride[a], idx));
+    }
+    if (FINAL)
+        st2(f, idx, make_double2(yv.x - lambda * dv.x, yv.y - lambda * dv.y));
+    else
+        D[idx] = make_double2(dv.x - yv.x / lambda, dv.y - yv.y / lambda);
+}
+
+// G = G - step*grad(D); G = G / max(amp(G), 1).  first: G is zero on entry.
+template <int NDIM, int AMP>
+__global__ __launch_bounds__(256) void k_tv_step(TVGeom g, double2 *__restrict__ G, const double2 *__restrict__ D,
+                                                 double step, int first)
+{
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= g.n) return;
+    int c[3];
+    tv_coords<NDIM>(g, idx, c);
+    const double2 d0 = D[idx];
+    double2 v[NDIM];
+#pragma unroll
+    for (int a = 0; a < NDIM; ++a) {
+        const double2 dd = (c[a] < g.s[a] - 1) ? csub(D[idx + g.stride[a]], d0) : make_double2(0.0, 0.0);
+        const double2 old = first ? make_double2(0.0, 0.0) : G[(int64_t)a * g.n + idx];
+        v[a] = make_double2(old.x - step * dd.x, old.y - step * dd.y);
+    }
+    tv_project<NDIM, AMP>(v);
+#pragma unroll
+    for (int a = 0; a < NDIM; ++a) G[(int64_t)a * g.n + idx] = v[a];
+}
+
 // Several Chambolle steps per launch.  A step is D = Div(G) - y / lambda, then
 // G = G - step grad(D), G = G / max(amp(G), 1); D at a cell needs G there and one cell
 // before it on each axis, the new G needs D there and one cell after it.  A block loads
@@ -257,9 +320,10 @@ template <int NDIM, int AMP> __device__ inline void tv_project(double2 *v)
 // launch, so the result does not depend on the split.
 // In 2-D the steps of small images are bound by launches and by the latency of the FP64
 // chain (square roots and quotients), so up to 7 steps (tiles of 18 x 18) run per launch:
-// 256^2, 40 steps: 82 us, against 276 us as two kernels per step (512^2: 221 / 477 us).  In 3-D the field is
+// 256^2, 40 steps: 76 us, against 276 us as two kernels per step (512^2: 208 / 477 us).  In 3-D the field is
 // 48 bytes per cell and a halo of more than one cell costs more than it saves: one step
 // per launch, D never stored (96^3: 1.06 ms for 40 steps, two kernels 1.49 ms).
+// See tv_regions for the shapes that take two kernels per step.
 constexpr int kTVThreads = 1024;
 constexpr int kTVSteps2 = 7, kTVSteps3 = 1;
 
@@ -357,38 +421,90 @@ __global__ __launch_bounds__(kTVThreads) void k_tv_steps(TVGeom g, TVLaunch L, c
     if (in && tile) st2(f, idx, make_double2(yv.x - lambda * dv.x, yv.y - lambda * dv.y));
 }
 
-template <typename T, int NDIM>
-int tv_prox(TVGeom g, const T *y, double lambda, double step, int niter, int amp, double2 *work, T *f,
-            hipStream_t s)
+// Steps and tiles of launch k of n.
+template <int NDIM> TVLaunch tv_launch(const TVGeom &g, int niter, int k, int n, int64_t *blocks)
 {
     using R = TVRegion<NDIM>;
     const int r[3] = {R::r0, R::r1, R::r2};
-    const int most = NDIM == 2 ? kTVSteps2 : kTVSteps3;
-    const int n = std::max(1, (niter + most - 1) / most); // launches, the steps shared out evenly
-    double2 *cur = work, *next = work + (int64_t)NDIM * g.n;
-    for (int k = 0; k < n; ++k) {
-        TVLaunch L;
-        L.iters = (int)((int64_t)niter * (k + 1) / n - (int64_t)niter * k / n);
-        L.first = k == 0;
-        L.last = k == n - 1;
-        L.lo = L.iters + L.last;
-        int64_t blocks = g.nt;
-        for (int a = 0; a < 3; ++a) {
-            L.t[a] = a < NDIM ? r[a] - L.iters - L.lo : 1;
-            L.nt[a] = a < NDIM ? (g.s[a] + L.t[a] - 1) / L.t[a] : 1;
-            blocks *= L.nt[a];
-        }
-        if (amp == GN_TV_AMP_SQUARE)
-            k_tv_steps<T, NDIM, GN_TV_AMP_SQUARE>
-                <<<(unsigned)blocks, kTVThreads, 0, s>>>(g, L, y, lambda, step, cur, next, f);
-        else
-            k_tv_steps<T, NDIM, GN_TV_AMP_MODULUS>
-                <<<(unsigned)blocks, kTVThreads, 0, s>>>(g, L, y, lambda, step, cur, next, f);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return hip_fail(e, "TV prox launch");
-        std::swap(cur, next);
+    TVLaunch L;
+    L.iters = (int)((int64_t)niter * (k + 1) / n - (int64_t)niter * k / n);
+    L.first = k == 0;
+    L.last = k == n - 1;
+    L.lo = L.iters + L.last;
+    *blocks = g.nt;
+    for (int a = 0; a < 3; ++a) {
+        L.t[a] = a < NDIM ? r[a] - L.iters - L.lo : 1;
+        L.nt[a] = a < NDIM ? (g.s[a] + L.t[a] - 1) / L.t[a] : 1;
+        *blocks *= L.nt[a];
     }
-    return GN_OK;
+    return L;
+}
+
+template <int NDIM> int tv_launches(int niter)
+{
+    const int most = NDIM == 2 ? kTVSteps2 : kTVSteps3;
+    return std::max(1, (int)(((int64_t)niter + most - 1) / most)); // the steps are shared out evenly
+}
+
+// Whether the steps run on LDS regions.  A region costs its block the same however few of
+// its cells the array fills (thin axes, small images with many trailing elements), and a
+// trailing dimension makes its accesses uncoalesced; two kernels per step cost launches and
+// passes over the field.  Microseconds for all steps, two kernels / regions:
+//   2-D, up to 1024 blocks: 3 x 3 x 1000, 40 steps 265 / 130; 16384 x 2, 40 steps 255 / 250
+//   2-D, more: 8 x 8 x 4096 (64 cells per block) 343 / 481, 65536 x 2 (36) 288 / 760,
+//     24 x 24 x 4096 (144) x 1.32, 14 x 14 x 4096 (196) x 0.67, 40 x 40 x 4096 (213) x 0.94;
+//     a single step: 40 x 40 x 4096 (400) x 1.13, 64 x 64 x 256 (455) x 0.86
+//   3-D, one trailing element: 256 x 256 x 2 (127) 382 / 569, 256 x 256 x 8, 3 steps (329)
+//     54 / 66, 128^3, 1 step (306) 65 / 79, 10 steps (480) 702 / 554; 32^3 (125 blocks) 285 / 233
+//   3-D, more trailing elements: 64^3 x 8 (501) 2956 / 3506
+template <int NDIM> bool tv_regions(const TVGeom &g, int niter)
+{
+    const int n = tv_launches<NDIM>(niter);
+    int64_t block_steps = 0;
+    for (int k = 0; k < n; ++k) {
+        int64_t blocks = 0;
+        const TVLaunch L = tv_launch<NDIM>(g, niter, k, n, &blocks);
+        block_steps += blocks * L.iters;
+    }
+    const int64_t few = NDIM == 2 ? 1024 : 128;
+    const int64_t cells = NDIM == 2 ? (niter == 1 ? 430 : 200) : 440; // per block and step
+    return block_steps <= few * niter || ((NDIM == 2 || g.nt == 1) && (int64_t)g.n * niter >= cells * block_steps);
+}
+
+template <typename T, int NDIM, int AMP>
+int tv_prox(TVGeom g, const T *y, double lambda, double step, int niter, double2 *work, T *f, hipStream_t s)
+{
+    if (tv_regions<NDIM>(g, niter)) {
+        const int n = tv_launches<NDIM>(niter);
+        double2 *cur = work, *next = work + (int64_t)NDIM * g.n;
+        for (int k = 0; k < n; ++k) {
+            int64_t blocks = 0;
+            const TVLaunch L = tv_launch<NDIM>(g, niter, k, n, &blocks);
+            k_tv_steps<T, NDIM, AMP><<<(unsigned)blocks, kTVThreads, 0, s>>>(g, L, y, lambda, step, cur, next, f);
+            std::swap(cur, next);
+        }
+    } else {
+        double2 *G = work, *D = work + (int64_t)NDIM * g.n;
+        const unsigned nb = (unsigned)(((int64_t)g.n + 255) / 256);
+        for (int it = 0; it < niter; ++it) {
+            k_tv_div<T, NDIM, false><<<nb, 256, 0, s>>>(g, G, y, lambda, it == 0, D, f);
+            k_tv_step<NDIM, AMP><<<nb, 256, 0, s>>>(g, G, D, step, it == 0);
+        }
+        k_tv_div<T, NDIM, true><<<nb, 256, 0, s>>>(g, G, y, lambda, niter == 0, D, f);
+    }
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? GN_OK : hip_fail(e, "TV prox launch");
+}
+
+template <typename T>
+int tv_prox_any(int ndim, int amp, TVGeom g, const T *y, double lambda, double step, int niter, double2 *work, T *f,
+                hipStream_t s)
+{
+    if (amp == GN_TV_AMP_SQUARE)
+        return ndim == 2 ? tv_prox<T, 2, GN_TV_AMP_SQUARE>(g, y, lambda, step, niter, work, f, s)
+                         : tv_prox<T, 3, GN_TV_AMP_SQUARE>(g, y, lambda, step, niter, work, f, s);
+    return ndim == 2 ? tv_prox<T, 2, GN_TV_AMP_MODULUS>(g, y, lambda, step, niter, work, f, s)
+                     : tv_prox<T, 3, GN_TV_AMP_MODULUS>(g, y, lambda, step, niter, work, f, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -486,15 +602,10 @@ int gn_tv_prox(int dtype, int ndim, const int64_t *shape, int64_t nt, const void
     g.n = (int)n;
     hipStream_t s = (hipStream_t)stream;
     double2 *w = (double2 *)work;
-    if (dtype == GN_C64) {
-        if (ndim == 2) return tv_prox<float2, 2>(g, (const float2 *)y, lambda, step, niter, amp_rule, w, (float2 *)f, s);
-        return tv_prox<float2, 3>(g, (const float2 *)y, lambda, step, niter, amp_rule, w, (float2 *)f, s);
-    }
-    if (dtype == GN_C128) {
-        if (ndim == 2)
-            return tv_prox<double2, 2>(g, (const double2 *)y, lambda, step, niter, amp_rule, w, (double2 *)f, s);
-        return tv_prox<double2, 3>(g, (const double2 *)y, lambda, step, niter, amp_rule, w, (double2 *)f, s);
-    }
+    if (dtype == GN_C64)
+        return tv_prox_any<float2>(ndim, amp_rule, g, (const float2 *)y, lambda, step, niter, w, (float2 *)f, s);
+    if (dtype == GN_C128)
+        return tv_prox_any<double2>(ndim, amp_rule, g, (const double2 *)y, lambda, step, niter, w, (double2 *)f, s);
     return fail(GN_EINVAL, "TV prox: dtype must be GN_C64 or GN_C128");
 }
 
