@@ -8,6 +8,7 @@
 #include <utility>
 
 #include "gaussnufft_solver.h"
+#include "gn_host_plan.h"
 #include "gn_internal.h"
 
 namespace gn {
@@ -457,6 +458,8 @@ template <int NDIM> int tv_launches(int niter)
 //   3-D, one trailing element: 256 x 256 x 2 (127) 382 / 569, 256 x 256 x 8, 3 steps (329)
 //     54 / 66, 128^3, 1 step (306) 65 / 79, 10 steps (480) 702 / 554; 32^3 (125 blocks) 285 / 233
 //   3-D, more trailing elements: 64^3 x 8 (501) 2956 / 3506
+// Regions also need every launch's blocks to fit one launch (2^22 of 1024 threads: from about
+// 1.4e9 cells in 3-D); the two kernels' 256-thread blocks fit for every array that is taken.
 template <int NDIM> bool tv_regions(const TVGeom &g, int niter)
 {
     const int n = tv_launches<NDIM>(niter);
@@ -464,6 +467,7 @@ template <int NDIM> bool tv_regions(const TVGeom &g, int niter)
     for (int k = 0; k < n; ++k) {
         int64_t blocks = 0;
         const TVLaunch L = tv_launch<NDIM>(g, niter, k, n, &blocks);
+        if (!host::launch_fits(blocks, kTVThreads)) return false;
         block_steps += blocks * L.iters;
     }
     const int64_t few = NDIM == 2 ? 1024 : 128;

@@ -54,3 +54,18 @@ def test_cartesian_fft_of_many_columns(n, batch):
     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     _lib.check(_lib.load().gn_fft_c2c(1, shp, batch, _lib.GN_FFT_FORWARD, 0, None, 1, x.data_ptr(), x.data_ptr(), st))
     assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("niter", [0, 3])
+def test_tv_prox_of_many_images(niter):
+    """2^22 trailing elements of 2 x 2 pixels: a region each would be 2^32 threads.  The
+    elements repeat 1024 different ones, whose prox is taken separately."""
+    import torch
+    from mripy_amd import solvers as S
+    print("case: tv of many images", niter, flush=True)
+    g = torch.Generator().manual_seed(1)
+    few = torch.randn(2, 2, 1, 1024, generator=g, dtype=torch.complex128).cuda()
+    x = few.expand(2, 2, 4096, 1024).contiguous()
+    f = S.prox_tv2d_r(x, 0.3, niter=niter)
+    want = S.prox_tv2d_r(few, 0.3, niter=niter) if niter else few
+    assert float((f - want).abs().max()) <= 1e-12
