@@ -617,15 +617,20 @@ int gn_soft_step(int64_t n, const void *g, const void *b, void *acc, double step
                  const void *x_pre, double beta, void *y, void *stream)
 {
     constexpr int kThreads = 256;
-    if (n < 0 || n > (int64_t)0x7fffffff * kThreads) return fail(GN_EINVAL, "soft step: element count out of range");
+    if (n < 0) return fail(GN_EINVAL, "soft step: element count out of range");
     if (n == 0) return GN_OK;
     if (!g || !acc || !x || (y && !x_pre)) return fail(GN_EINVAL, "soft step: null pointer");
     if (x == acc || x == g || x == b || x == x_pre || x == y || (y && (y == acc || y == g || y == b || y == x_pre)) ||
         acc == g || acc == b || acc == x_pre)
         return fail(GN_EINVAL, "soft step: outputs must not alias");
-    k_soft_step<<<(unsigned)((n + kThreads - 1) / kThreads), kThreads, 0, (hipStream_t)stream>>>(
-        n, (const float2 *)g, (const float2 *)b, (float2 *)acc, (float)step, (float)th, (float2 *)x,
-        (const float2 *)x_pre, (float)beta, (float2 *)y);
+    constexpr int64_t kPart = (int64_t)1 << 31; // elements of one launch, which has fewer than 2^32 threads
+    static_assert(host::launch_fits(kPart / kThreads, kThreads), "one launch");
+    for (int64_t o = 0; o < n; o += kPart) {
+        const int64_t m = std::min(kPart, n - o);
+        k_soft_step<<<(unsigned)((m + kThreads - 1) / kThreads), kThreads, 0, (hipStream_t)stream>>>(
+            m, (const float2 *)g + o, b ? (const float2 *)b + o : nullptr, (float2 *)acc + o, (float)step, (float)th,
+            (float2 *)x + o, y ? (const float2 *)x_pre + o : nullptr, (float)beta, y ? (float2 *)y + o : nullptr);
+    }
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? GN_OK : hip_fail(e, "soft step launch");
 }

@@ -69,3 +69,26 @@ def test_tv_prox_of_many_images(niter):
     f = S.prox_tv2d_r(x, 0.3, niter=niter)
     want = S.prox_tv2d_r(few, 0.3, niter=niter) if niter else few
     assert float((f - want).abs().max()) <= 1e-12
+
+
+def test_update_of_many_elements():
+    """The IST update of 2^32 + 64 elements (more than a launch has threads) into buffers of
+    the same size, every one of them checked by the least and the greatest."""
+    import torch
+    from mripy_amd import _lib
+    n = (1 << 32) + 64
+    if torch.cuda.mem_get_info()[0] < 4.5 * 8 * n:
+        pytest.skip("needs 150 GB of free device memory")
+    print("case: update of many elements", flush=True)
+    import ctypes
+    ones = torch.ones(2 * n, dtype=torch.float32, device="cuda")     # complex: 1 + 1i
+    acc = torch.full((2 * n,), 3.0, dtype=torch.float32, device="cuda")
+    x = torch.zeros(2 * n, dtype=torch.float32, device="cuda")
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(_lib.load().gn_soft_step(n, ones.data_ptr(), None, acc.data_ptr(), 2.0, 0.0, x.data_ptr(), None, 0.0, None, st))
+    # acc = 3 - 2 * 1 in both parts everywhere, x = acc / (|acc| + 1e-6) * |acc|
+    assert float(acc.amin()) == 1.0 and float(acc.amax()) == 1.0
+    m = 2 ** 0.5
+    assert abs(float(x.amin()) - m / (m + 1e-6)) <= 1e-6 and abs(float(x.amax()) - m / (m + 1e-6)) <= 1e-6
+    del ones, acc, x
+    torch.cuda.empty_cache()
