@@ -639,18 +639,18 @@ __global__ __launch_bounds__(256) void k_item_write(int64_t K, const int *__rest
 __global__ __launch_bounds__(256) void k_occ_masks(int64_t ncolt, int nt0, int mask_k, const int *__restrict__ pstart,
                                                    unsigned long long *__restrict__ occ)
 {
-    const int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (c >= ncolt) return;
     const int lane = threadIdx.x & 63;
-    bool on = false;
-    for (int i = 0; i < mask_k; ++i) {
-        const int t0 = lane * mask_k + i;
-        if (t0 >= nt0) break;
-        const int64_t k = t0 * ncolt + c;
-        on = on || pstart[k + 1] > pstart[k];
+    for (int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); c < ncolt; c += (int64_t)gridDim.x * 4) {
+        bool on = false;
+        for (int i = 0; i < mask_k; ++i) {
+            const int t0 = lane * mask_k + i;
+            if (t0 >= nt0) break;
+            const int64_t k = t0 * ncolt + c;
+            on = on || pstart[k + 1] > pstart[k];
+        }
+        const unsigned long long m = __ballot(on);
+        if (lane == 0) occ[c] = m;
     }
-    const unsigned long long m = __ballot(on);
-    if (lane == 0) occ[c] = m;
 }
 
 // ---------------------------------------------------------------------------
@@ -2836,7 +2836,7 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
             (rc = items(Kg, R.bin_start, kGatherChunk, kRetGather, R.gather_items, nullptr)))
             return rc;
         R.mask_k = (g.ntiles[0] + 63) / 64;
-        hipLaunchKernelGGL(k_occ_masks, dim3(grid_blocks(ncolt, 4, INT32_MAX)), dim3(256), 0, st, ncolt, g.ntiles[0],
+        hipLaunchKernelGGL(k_occ_masks, dim3(grid_blocks(ncolt, 4)), dim3(256), 0, st, ncolt, g.ntiles[0],
                            R.mask_k, tile_pairs, R.occ_mask);
         GN_HIP(hipGetLastError());
         GN_HIP(hipStreamSynchronize(st));

@@ -92,3 +92,23 @@ def test_update_of_many_elements():
     assert abs(float(x.amin()) - m / (m + 1e-6)) <= 1e-6 and abs(float(x.amax()) - m / (m + 1e-6)) <= 1e-6
     del ones, acc, x
     torch.cuda.empty_cache()
+
+
+def test_many_tile_columns():
+    """One-cell tiles on two axes of 8192 cells: 2^26 tile columns, whose occupancy words one
+    wave each would be 2^32 threads.  The points are taken, and a gather of ones gives each
+    sample the sum of its window."""
+    import torch
+    from mripy_amd.plan import Plan
+    print("case: many tile columns", flush=True)
+    modes, M = (2, 4096, 4096), 64
+    rng = np.random.default_rng(5)
+    coords = [(np.pi * (2 * rng.random(M) - 1)).astype(np.float32) for _ in modes]
+    P = Plan(modes, ncoils=1, rat=2, nspread=2, tiles=(4, 1, 1)).set_points(coords)
+    G = float(np.prod(P.nf))
+    got = P.grid_gather(torch.ones((1,) + P.nf, dtype=torch.complex64, device="cuda")).cpu().numpy()[:, 0] * G
+    p = O.Params(modes, rat=2, nspread=2)
+    want = np.ones(M)
+    for c, n in zip(coords, P.nf):
+        want = want * O.window_direct(c.astype(np.float64), n, 2, p.tau)[1].sum(1)
+    assert rel(got, want) <= TOL
