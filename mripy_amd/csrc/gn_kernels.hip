@@ -2945,12 +2945,28 @@ SpreadShape spread_shape(const SpreadArgs &a, int dim)
 
 namespace {
 
+// f(first, count) over n work items in parts that one launch takes: fewer than 2^32 threads,
+// and with `rest` blocks per item fewer than 2^31 blocks (the dispatch order is 32-bit).
+template <typename F>
+hipError_t item_parts(int n, int threads, int64_t rest, F f)
+{
+    const int64_t most = std::min((((int64_t)1 << 32) - 1) / threads, (((int64_t)1 << 31) - 1) / rest);
+    if (most < 1) return hipErrorInvalidConfiguration;
+    hipError_t e = hipSuccess;
+    for (int64_t o = 0; o < n && e == hipSuccess; o += most) e = f(o, (unsigned)std::min(most, n - o));
+    return e;
+}
+
 template <typename K>
-hipError_t spread_go(K kernel, dim3 grid, const SpreadShape &sh, const SpreadArgs &a, hipStream_t st)
+hipError_t spread_go(K kernel, int nitems, int64_t ng, const SpreadShape &sh, const SpreadArgs &a, hipStream_t st)
 {
     lds_limit(kernel, sh.lds);
-    hipLaunchKernelGGL(kernel, grid, dim3(64 * sh.waves), sh.lds, st, a);
-    return hipGetLastError();
+    return item_parts(nitems, 64 * sh.waves, ng * sh.nbg, [&](int64_t o, unsigned n) {
+        SpreadArgs part = a;
+        part.items += o;
+        hipLaunchKernelGGL(kernel, dim3(n, (unsigned)ng, (unsigned)sh.nbg), dim3(64 * sh.waves), sh.lds, st, part);
+        return hipGetLastError();
+    });
 }
 
 template <int D>
@@ -2958,24 +2974,23 @@ hipError_t spread_dispatch(const SpreadArgs &a, int nitems, int nritems, const i
                            hipStream_t st)
 {
     const SpreadShape sh = spread_shape(a, D);
-    const dim3 grid((unsigned)nitems, (unsigned)((nc + sh.coils - 1) / sh.coils), (unsigned)sh.nbg);
-    if (!grid_ok(grid)) return hipErrorInvalidConfiguration;
+    const int64_t ng = (nc + sh.coils - 1) / sh.coils;
     hipError_t e = hipSuccess;
     if (nitems > 0) {
         switch (sh.kind * 16 + sh.width) {
-        case kSpreadSub * 16 + 1: e = spread_go(k_spread_sub<1>, grid, sh, a, st); break;
-        case kSpreadSub * 16 + 2: e = spread_go(k_spread_sub<2>, grid, sh, a, st); break;
-        case kSpreadTile * 16 + 8: e = spread_go(k_spread_tile<3, 8>, grid, sh, a, st); break; // 3-D only
-        case kSpreadTile * 16 + 4: e = spread_go(k_spread_tile<D, 4>, grid, sh, a, st); break;
-        case kSpreadTile * 16 + 2: e = spread_go(k_spread_tile<D, 2>, grid, sh, a, st); break;
-        case kSpreadMfma * 16 + 8: e = spread_go(k_spread_mfma<D, 8>, grid, sh, a, st); break;
-        case kSpreadMfma * 16 + 4: e = spread_go(k_spread_mfma<D, 4>, grid, sh, a, st); break;
-        case kSpreadMfma * 16 + 2: e = spread_go(k_spread_mfma<D, 2>, grid, sh, a, st); break;
-        case kSpreadMfma * 16 + 1: e = spread_go(k_spread_mfma<D, 1>, grid, sh, a, st); break;
-        case kSpreadValu * 16 + 8: e = spread_go(k_spread<D, 8>, grid, sh, a, st); break;
-        case kSpreadValu * 16 + 4: e = spread_go(k_spread<D, 4>, grid, sh, a, st); break;
-        case kSpreadValu * 16 + 2: e = spread_go(k_spread<D, 2>, grid, sh, a, st); break;
-        case kSpreadValu * 16 + 1: e = spread_go(k_spread<D, 1>, grid, sh, a, st); break;
+        case kSpreadSub * 16 + 1: e = spread_go(k_spread_sub<1>, nitems, ng, sh, a, st); break;
+        case kSpreadSub * 16 + 2: e = spread_go(k_spread_sub<2>, nitems, ng, sh, a, st); break;
+        case kSpreadTile * 16 + 8: e = spread_go(k_spread_tile<3, 8>, nitems, ng, sh, a, st); break; // 3-D only
+        case kSpreadTile * 16 + 4: e = spread_go(k_spread_tile<D, 4>, nitems, ng, sh, a, st); break;
+        case kSpreadTile * 16 + 2: e = spread_go(k_spread_tile<D, 2>, nitems, ng, sh, a, st); break;
+        case kSpreadMfma * 16 + 8: e = spread_go(k_spread_mfma<D, 8>, nitems, ng, sh, a, st); break;
+        case kSpreadMfma * 16 + 4: e = spread_go(k_spread_mfma<D, 4>, nitems, ng, sh, a, st); break;
+        case kSpreadMfma * 16 + 2: e = spread_go(k_spread_mfma<D, 2>, nitems, ng, sh, a, st); break;
+        case kSpreadMfma * 16 + 1: e = spread_go(k_spread_mfma<D, 1>, nitems, ng, sh, a, st); break;
+        case kSpreadValu * 16 + 8: e = spread_go(k_spread<D, 8>, nitems, ng, sh, a, st); break;
+        case kSpreadValu * 16 + 4: e = spread_go(k_spread<D, 4>, nitems, ng, sh, a, st); break;
+        case kSpreadValu * 16 + 2: e = spread_go(k_spread<D, 2>, nitems, ng, sh, a, st); break;
+        case kSpreadValu * 16 + 1: e = spread_go(k_spread<D, 1>, nitems, ng, sh, a, st); break;
         default: return hipErrorInvalidValue;
         }
     }
@@ -3289,8 +3304,10 @@ hipError_t spread_batch_go(K kernel, const SpreadShape &sh, const SpreadArgs *d_
                            hipStream_t st)
 {
     lds_limit(kernel, sh.lds);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)n, (unsigned)sh.nbg), dim3(64 * sh.waves), sh.lds, st, d_args, d_items);
-    return hipGetLastError();
+    return item_parts(n, 64 * sh.waves, sh.nbg, [&](int64_t o, unsigned part) {
+        hipLaunchKernelGGL(kernel, dim3(part, (unsigned)sh.nbg), dim3(64 * sh.waves), sh.lds, st, d_args, d_items + o);
+        return hipGetLastError();
+    });
 }
 
 template <int D>
@@ -3336,7 +3353,6 @@ hipError_t launch_spread_batch(int dim, const SpreadShape &sh, const SpreadArgs 
                                hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
-    if (!grid_ok(dim3((unsigned)n, (unsigned)sh.nbg))) return hipErrorInvalidConfiguration;
     return dim == 3 ? spread_batch_dispatch<3>(sh, d_args, d_items, n, st)
                     : spread_batch_dispatch<2>(sh, d_args, d_items, n, st);
 }

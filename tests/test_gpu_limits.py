@@ -112,3 +112,30 @@ def test_many_tile_columns():
     for c, n in zip(coords, P.nf):
         want = want * O.window_direct(c.astype(np.float64), n, 2, p.tau)[1].sum(1)
     assert rel(got, want) <= TOL
+
+
+def test_spread_of_many_tiles():
+    """2^24 spread tiles with 256 threads each (3 coils on 32768 x 65536 cells): the spread
+    alone, cell by cell at every sample's window, and its norm (no other cell is set)."""
+    import torch
+    from mripy_amd.plan import Plan
+    nf, nc, M, ns = (32768, 65536), 3, 40, 2
+    if torch.cuda.mem_get_info()[0] < 4.5 * 8 * nc * nf[0] * nf[1]:
+        pytest.skip("needs 230 GB of free device memory")
+    print("case: many tiles", flush=True)
+    rng = np.random.default_rng(2)
+    coords = [(np.pi * (2 * rng.random(M) - 1)).astype(np.float32) for _ in nf]
+    coords[0][:2], coords[1][:2] = (-1e-3, 1e-3), (-1e-3, 1e-3)       # the last tile and the first
+    P = Plan(tuple(n // 2 for n in nf), ncoils=nc, rat=2, nspread=ns).set_points(coords)
+    y = _cnormal(rng, (M, nc))
+    out = P.grid_spread(torch.as_tensor(y).cuda())
+    p = O.Params(P.modes, rat=2, nspread=ns)
+    (i0, w0), (i1, w1) = [O.window_direct(c.astype(np.float64), n, ns, p.tau) for c, n in zip(coords, nf)]
+    got = torch.stack([out[c][torch.as_tensor(i0[:, :, None]).cuda(), torch.as_tensor(i1[:, None, :]).cuda()]
+                       for c in range(nc)], -1).cpu().numpy()
+    want = (w0[:, :, None] * w1[:, None, :])[..., None] * y[:, None, None, :]
+    assert rel(got, want) <= TOL
+    norm = sum(float(torch.view_as_real(o).view(-1)[k::8].double().square().sum()) for o in out for k in range(8)) ** 0.5
+    assert abs(norm - np.linalg.norm(want.ravel())) <= TOL * norm
+    del out, P
+    torch.cuda.empty_cache()
