@@ -93,9 +93,12 @@ __global__ __launch_bounds__(256) void k_shift_copy(ShiftArgs a, const float2 *_
 // lines (128-byte row segments), fewer lines while the launch has fewer than two blocks
 // per CU.  Measured at 256 x 256 x 32 (16.8 MB), masked forward then inverse through the
 // operator: 47 us, against 147 us for shift pass, rocFFT, shift pass and a wait per call.
+// Short lines come by the hundred, 2048 elements a block: 16 lines of 2 or 3 points are a
+// block of 256 bytes (2-D 1024 x 2 of 8192: 1381 us, with 1024 lines 172, rocFFT 717).
 // ---------------------------------------------------------------------------
 constexpr int kAxisThreads = 512;
 constexpr int kAxisLines = 16;
+constexpr int kAxisElems = 2048;              // elements of a block of short lines, at least
 constexpr int kAxisUnroll = 4;                // global loads in flight per thread
 constexpr int64_t kAxisBlocks = 512;          // two blocks per CU
 constexpr size_t kAxisLdsMax = 64 * 1024;
@@ -214,18 +217,19 @@ int axis_table(int dev, int L, FFTAxis **ax)
     return GN_OK;
 }
 
-// Lines (columns x slabs) a block of the axis pass may hold: 16, fewer while they exceed
-// kAxisLdsMax.
+// Lines (columns x slabs) a block of the axis pass may hold: 16, more of short ones so that
+// the block has kAxisElems elements, fewer while they exceed kAxisLdsMax.
 int axis_lines(int L)
 {
     int lines = kAxisLines;
+    while (2 * lines * L <= kAxisElems) lines *= 2;
     while (lines > 1 && col_lds(L, lines, host::fft_direct_sums(L)) > kAxisLdsMax) lines /= 2;
     return lines;
 }
 
 // The axis passes apply: every length is 1 or covered, the output is the input or does not
-// overlap it, and the blocks of every axis fit one launch (an axis of length L takes up to
-// about 2^27 L elements; larger arrays are left to rocFFT, whose shift passes loop).
+// overlap it, and the blocks of every axis fit one launch (2^23 blocks of about 2048
+// elements; larger arrays are left to rocFFT, whose shift passes loop).
 bool axis_passes_ok(int rank, const int64_t *n, int64_t total, const void *in, const void *out)
 {
     bool any = false;

@@ -39,8 +39,8 @@ def test_pair_total_is_refused(M):
 
 @pytest.mark.parametrize("n,batch", [(2, 1 << 28), (2, (1 << 27) - 16)])
 def test_cartesian_fft_of_many_columns(n, batch):
-    """2 points x 2^28 columns: more blocks than a launch of the axis passes takes (rocFFT),
-    and just as many as it takes.  Out of place and in place."""
+    """2 points x 2^28 columns: with 16 columns a block more blocks than a launch takes, and
+    just as many.  Out of place and in place."""
     import ctypes
     import torch
     from mripy_amd import _lib
