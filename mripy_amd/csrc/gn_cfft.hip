@@ -227,7 +227,7 @@ int axis_lines(int L)
     return lines;
 }
 
-// The axis passes apply: every length is 1 or covered, the output is the input or does not
+// The axis passes apply: every length is 1 or covered (and not faster with rocFFT), the output is the input or does not
 // overlap it, and the blocks of every axis fit one launch (2^23 blocks of about 2048
 // elements; larger arrays are left to rocFFT, whose shift passes loop).
 bool axis_passes_ok(int rank, const int64_t *n, int64_t total, const void *in, const void *out)
@@ -236,8 +236,9 @@ bool axis_passes_ok(int rank, const int64_t *n, int64_t total, const void *in, c
     int64_t slabs = 1;
     for (int a = 0; a < rank; ++a) {
         if (n[a] == 1) continue;
-        if (!fft_length_supported(n[a])) return false;
-        const auto sp = host::axis_split(slabs, total / (slabs * n[a]), axis_lines((int)n[a]), kAxisBlocks);
+        const int64_t ncols = total / (slabs * n[a]);
+        if (n[a] > 2048 || (ncols > 1 && !host::axis_strided_ok((int)n[a])) || !fft_length_supported(n[a])) return false;
+        const auto sp = host::axis_split(slabs, ncols, axis_lines((int)n[a]), kAxisBlocks);
         if (!host::launch_fits(sp.blocks, kAxisThreads)) return false;
         any = true;
         slabs *= n[a];

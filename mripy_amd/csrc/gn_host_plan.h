@@ -123,6 +123,21 @@ inline bool fft_direct_sums(int L)
     return L > 1;
 }
 
+// Whether a strided axis of this length (several columns) is left to the Cartesian axis
+// passes: not where a block's LDS holds one column, so that a row segment is 8 bytes.  Microseconds, rocFFT with its shift passes /
+// axis passes, n x n x 2: 1834 (prime 131) 352 / 295, 1820 206 / 150, 1875 218 / 233,
+// 2000 228 / 272, 2048 230 / 286, 1912 (prime 239) 361 / 522; rocFFT has radix 17:
+// 1088 105 / 79, 1156 121 / 132, 1360 135 / 159, 1530 162 / 210, 1700 184 / 235.
+inline bool axis_strided_ok(int L)
+{
+    int n = L;
+    for (int p : {2, 3, 5, 7, 11, 13})
+        while (n % p == 0) n /= p;
+    const bool direct = n > 1;
+    while (n % 17 == 0) n /= 17;
+    return L <= 1860 && !(direct && n == 1 && L > 1100);
+}
+
 // HIP takes launches of fewer than 2^32 threads per grid axis.
 constexpr bool launch_fits(int64_t blocks, int threads) { return blocks < (((int64_t)1 << 32) + threads - 1) / threads; }
 

@@ -42,6 +42,13 @@ static void check_pair_total()
             CHECK(scanned_total(samples, pairs) == samples * pairs);
 }
 
+// Long strided axes of the Cartesian FFT: the lengths that were measured.
+static void check_strided()
+{
+    for (int L : {2, 16, 17, 34, 1000, 1024, 1088, 1820, 1834, 1850, 1860, 1444 /* 4 19^2 */}) CHECK(axis_strided_ok(L));
+    for (int L : {1156, 1224, 1360, 1530, 1700, 1836, 1862, 1875, 1904, 1912, 2000, 2048}) CHECK(!axis_strided_ok(L));
+}
+
 // A launch has fewer than 2^32 threads; a split covers every line once.
 static void check_launches()
 {
@@ -71,6 +78,7 @@ int main()
 {
     check_pair_total();
     check_launches();
+    check_strided();
     printf("OK\n");
     return 0;
 }

@@ -1,5 +1,5 @@
 """The Cartesian FFT where the choice of its passes changes, against numpy in 64 bits:
-short lines by the hundred in a block.  Tolerance: rel-L2 2e-6."""
+short lines by the hundred in a block, long strided axes.  Tolerance: rel-L2 2e-6."""
 import numpy as np
 import pytest
 
@@ -31,4 +31,12 @@ def check(shape, rank):
                                         ((600, 5, 3), 2), ((90, 2, 90, 3), 3), ((2, 90, 91), 3), ((400, 90, 2), 3),
                                         ((17, 4001), 1), ((300, 34), 2), ((13, 600, 8), 2)])
 def test_short_lines(shape, rank):
+    check(shape, rank)
+
+
+# strided axes on both sides of the lengths left to rocFFT (1860; 1100 with the prime 17), the
+# same lengths contiguous, and one of each in a call
+@pytest.mark.parametrize("shape,rank", [((1848, 3), 1), ((1875, 3), 1), ((5, 1875), 2), ((1088, 2), 1), ((1156, 2), 1),
+                                        ((3, 1156), 2), ((1904, 4, 2), 2), ((4, 2000, 3), 2), ((1862, 1), 2)])
+def test_long_axes(shape, rank):
     check(shape, rank)
