@@ -70,7 +70,8 @@ extern "C" {
 
 /* FFT engines for gn_plan_set_fft_engine */
 #define GN_FFT_AUTO 0   /* pruned in-place passes fused with pad/crop when every nf is at most 2048
-                           without prime factors above 256; rocFFT otherwise */
+                           with prime factors 2, 3, 5, or others where they are faster than
+                           rocFFT; rocFFT otherwise */
 #define GN_FFT_ROCFFT 1 /* separate pad, rocFFT and crop */
 
 typedef struct gn_plan_s gn_plan;

@@ -15,8 +15,8 @@
  * Each stage (gather, spread, split-tile reduce, and the pruned FFT passes
  * fused with pad / crop) is one kernel launch over the work items of all
  * instances (a few launches when instances differ in grid length, coil-count
- * class or tile shape).  When a grid length is above 2048 or has a prime
- * factor above 256, pad, one batched rocFFT execution per grid size and crop are used
+ * class or tile shape).  When a plan of one of the instances would use
+ * rocFFT (GN_FFT_AUTO in gaussnufft.h), pad, one batched rocFFT execution per grid size and crop are used
  * instead of the pruned passes.
  */
 #ifndef GAUSSNUFFT_BATCH_H

@@ -296,8 +296,7 @@ int plan_create_impl(int dim, const int64_t *modes, int rat, int nspread, int if
         return hip_fail(e, "plan tables upload");
     }
     if (with_grid) {
-        p->fft_custom = true;
-        for (int a = 0; a < dim; ++a) p->fft_custom &= fft_length_supported(g.nf[a]);
+        p->fft_custom = pruned_passes_ok(p);
         for (int a = 0; a < dim && p->fft_custom && !rc; ++a) rc = fft_axis_init(&p->fft_ax[a], (int)g.nf[a]);
         if (!rc && !p->fft_custom) rc = create_fft(p);
         if (rc) {

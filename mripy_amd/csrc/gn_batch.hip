@@ -672,10 +672,9 @@ int gn_batch_create(int dim, int n, const gn_instance *inst, int rat, int nsprea
         b->maxN = std::max(b->maxN, p->geo.N);
     }
     if (!rc) {
-        // pruned FFT passes when every instance's grid lengths are supported
+        // pruned FFT passes when every instance would use them
         b->custom = true;
-        for (auto *p : b->m)
-            for (int a = 0; a < dim; ++a) b->custom &= fft_length_supported(p->geo.nf[a]);
+        for (auto *p : b->m) b->custom &= pruned_passes_ok(p);
         for (auto *p : b->m)
             for (int a = 0; a < dim && b->custom && !rc; ++a) rc = fft_axis_init(&p->fft_ax[a], (int)p->geo.nf[a]);
     }

@@ -776,7 +776,7 @@ Stages make_stages(const FFTAxis &ax)
 // crop the pass A + columns of a type 2 took: 224^3 x 8 coils 0.49 instead of 1.89 ms,
 // 182 x 218 x 150 x 3 0.24 / 0.48, 226^3 x 4 0.69 / 1.97, 502^2 x 16 (prime 251) 0.136 /
 // 0.143, 142^2 x 1 0.022 / 0.040: primes above 256 would cost more than rocFFT's
-// Bluestein passes.
+// Bluestein passes.  Which of the covered grids use the passes: host::pruned_passes_pay.
 bool fft_length_supported(int64_t L)
 {
     if (L < 2 || L > 2048) return false; // LDS: one line of 2048 + twiddles fits in 64 KiB
@@ -785,6 +785,13 @@ bool fft_length_supported(int64_t L)
 }
 
 bool fft_length_smooth(int64_t L) { return L >= 1 && L <= 2048 && !host::fft_radices((int)L).empty(); }
+
+bool pruned_passes_ok(const gn_plan_s *p)
+{
+    for (int a = 0; a < p->geo.dim; ++a)
+        if (!fft_length_supported(p->geo.nf[a])) return false;
+    return host::pruned_passes_pay(p->geo.dim, p->geo.nf, p->nc);
+}
 
 int fft_axis_init(FFTAxis *ax, int L)
 {

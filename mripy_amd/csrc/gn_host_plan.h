@@ -123,6 +123,43 @@ inline bool fft_direct_sums(int L)
     return L > 1;
 }
 
+inline int largest_prime(int64_t L)
+{
+    int64_t big = 1;
+    for (int64_t p = 2; p * p <= L; ++p)
+        while (L % p == 0) {
+            big = p;
+            L /= p;
+        }
+    return (int)std::max(big, L);
+}
+
+// Whether the pruned FFT passes of a plan are to be used on grids whose lengths they cover:
+// always for the primes 2, 3, 5.  rocFFT has radices up to 17 as well and takes other lengths
+// as Bluestein transforms, which double where 2 L passes a power of two (1024); a column pass
+// slows down as its blocks hold fewer columns (LDS: 8, 4, 2 of them up to 780, 1260, 1820
+// points, or 525, 890, 1365 with a second buffer).  Type 2, pad + rocFFT / passes, as a
+// ratio (type 1 gains more or loses less):
+//   primes up to 17, n x n x 8 coils: 770 0.88, 784 1.01, 858 1.07, 952 1.50, 1300 1.81;
+//     last axis, 256 x n x 1: 448 0.89, 910 1.08, 1260 1.03, 1750 1.09
+//   others, n x n x 8: 844 (211) 0.84, 892 (223) 1.04, 916 (229) 1.16, 1002 (167) 1.14, 1010
+//     (101) 0.94, 1038 (173) 0.66, 1834 (131) 0.79, 1912 (239) 1.31; last axis, 256 x 1910 0.70
+//   a 3-D grid with few columns beside a long first axis, where rocFFT has more blocks:
+//     154 x 32 x 32 1.18, 112 x 32 x 32 x 4 coils 1.13, 220 x 32 x 32 x 8 0.79; 530 x 32 x 32 (53)
+//     0.74, 502 x 32 x 32 (251) 0.92 and 1.03 in type 1, 942 x 32 x 32 (157) 0.94 and 1.13
+inline bool pruned_passes_pay(int dim, const int64_t *nf, int64_t ncoils)
+{
+    for (int a = 0; a < dim; ++a) {
+        const int64_t L = nf[a];
+        const int p = largest_prime(L);
+        if (p <= 5) continue;
+        const bool rows = a == dim - 1; // contiguous lines
+        if (p <= 17 ? L > 780 : !rows && (L > 1860 || (L > 890 && L <= 1024 && p > 128))) return false;
+        if (dim == 3 && a == 0 && nf[1] * nf[2] * ncoils <= 4096 && (p <= 17 || p > 180 || L > 890)) return false;
+    }
+    return true;
+}
+
 // Whether a strided axis of this length (several columns) is left to the Cartesian axis
 // passes: not where a block's LDS holds one column, so that a row segment is 8 bytes.  Microseconds, rocFFT with its shift passes /
 // axis passes, n x n x 2: 1834 (prime 131) 352 / 295, 1820 206 / 150, 1875 218 / 233,

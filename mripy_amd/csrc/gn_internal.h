@@ -268,7 +268,7 @@ struct gn_plan_s {
     int *err_flag = nullptr;  // device: number of the last set_points that met bad coordinates
     int points_seq = 0;       // number of set_points calls
 
-    // FFT engine: the pruned in-place passes (gn_fft.hip) when they cover every nf
+    // FFT engine: the pruned in-place passes (gn_fft.hip) where pruned_passes_ok
     // (fft_custom), else rocFFT; GN_FFT_ROCFFT forces rocFFT
     bool fft_custom = false;
     int fft_engine = GN_FFT_AUTO;
@@ -311,6 +311,7 @@ void default_tiles(int dim, int ns, const int64_t *nf, int *tile, int *gtile);
 
 // fft.hip
 bool fft_length_supported(int64_t L);
+bool pruned_passes_ok(const gn_plan_s *p); // every grid length covered, and the passes faster than rocFFT
 int fft_axis_init(FFTAxis *ax, int L);
 void fft_axis_free(FFTAxis *ax);
 Stages make_stages(const FFTAxis &ax);

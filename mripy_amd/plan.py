@@ -277,7 +277,8 @@ class Plan:
 
     def set_fft_engine(self, engine="auto"):
         """"auto": pruned FFT passes fused with pad/crop where every nf is at most 2048
-        and has no prime factor above 256; "rocfft": separate pad, rocFFT, crop."""
+        with prime factors 2, 3, 5, or others where the passes are faster than rocFFT;
+        "rocfft": separate pad, rocFFT, crop."""
         check(_lib.load().gn_plan_set_fft_engine(self._h, _lib.GN_FFT_ROCFFT if engine == "rocfft"
                                                  else _lib.GN_FFT_AUTO))
 

@@ -49,6 +49,24 @@ static void check_strided()
     for (int L : {1156, 1224, 1360, 1530, 1700, 1836, 1862, 1875, 1904, 1912, 2000, 2048}) CHECK(!axis_strided_ok(L));
 }
 
+// Which grids with primes above 5 use the pruned passes: the measured ones, and every grid
+// of the primes 2, 3, 5.
+static void check_passes()
+{
+    auto pay2 = [](int64_t a, int64_t b, int64_t nc) { const int64_t nf[3] = {a, b, 1}; return pruned_passes_pay(2, nf, nc); };
+    auto pay3 = [](int64_t a, int64_t b, int64_t c, int64_t nc) { const int64_t nf[3] = {a, b, c}; return pruned_passes_pay(3, nf, nc); };
+    for (int L = 2; L <= 2048; ++L) {
+        CHECK(largest_prime(L) == 2 || L % largest_prime(L) == 0);
+        if (!fft_radices(L).empty()) CHECK(largest_prime(L) <= 5 && pay2(L, L, 8) && pay3(L, 32, 32, 1));
+    }
+    CHECK(largest_prime(2008) == 251 && largest_prime(289) == 17 && largest_prime(2) == 2 && largest_prime(1) == 1);
+    for (int L : {14, 254, 502, 770, 844, 890, 1010, 1038, 1834}) CHECK(pay2(L, L, 8));
+    for (int L : {784, 858, 952, 1300, 916, 1002, 1904, 1912, 2002, 2008}) CHECK(!pay2(L, L, 8));
+    CHECK(pay2(256, 1910, 1) && !pay2(1910, 256, 1) && pay2(256, 770, 1) && !pay2(256, 910, 1));
+    CHECK(pay3(182, 218, 150, 3) && pay3(220, 32, 32, 8) && !pay3(220, 32, 32, 4) && pay3(32, 32, 220, 1));
+    CHECK(pay3(530, 32, 32, 1) && !pay3(502, 32, 32, 1) && !pay3(942, 32, 32, 1) && pay3(940, 64, 128, 1));
+}
+
 // A launch has fewer than 2^32 threads; a split covers every line once.
 static void check_launches()
 {
@@ -79,6 +97,7 @@ int main()
     check_pair_total();
     check_launches();
     check_strided();
+    check_passes();
     printf("OK\n");
     return 0;
 }
