@@ -361,6 +361,19 @@ int gn_plan_set_tiles(gn_plan *p, const int *tile)
     return GN_OK;
 }
 
+// The coil images of a SENSE combine that does not fit one row-pass block.  Made with the
+// maps, so that executing allocates nothing (a call may be captured); where that failed, or
+// the FFT engine was another, on the first combine.
+static int make_sense_images(gn_plan *p)
+{
+    if (p->sbuf || sense_rows_fit(p)) return GN_OK;
+    if (hipMalloc((void **)&p->sbuf, (size_t)(p->geo.N * p->nc) * sizeof(float2)) != hipSuccess) {
+        p->sbuf = nullptr;
+        return fail(GN_ENOMEM, "hipMalloc failed for the SENSE coil images");
+    }
+    return GN_OK;
+}
+
 int gn_plan_set_sense(gn_plan *p, const void *maps)
 {
     g_err.clear();
@@ -376,6 +389,10 @@ int gn_plan_set_sense(gn_plan *p, const void *maps)
     if (!p->sens && hipMalloc((void **)&p->sens, bytes) != hipSuccess) {
         p->sens = nullptr;
         return fail(GN_ENOMEM, "hipMalloc failed for the SENSE maps");
+    }
+    if (p->fft_custom && p->fft_engine == GN_FFT_AUTO && make_sense_images(p)) {
+        (void)hipGetLastError(); // tried again, and reported, where a combine needs them
+        g_err.clear();
     }
     hipError_t e = hipMemcpyAsync(p->sens, maps, bytes, hipMemcpyDeviceToDevice, p->stream);
     if (e != hipSuccess) return hip_fail(e, "SENSE maps copy");
@@ -479,10 +496,7 @@ static int execute_impl(gn_plan *p, int kind, const void *in, void *out, float2 
             if (!r) r = timed(p, GN_STAGE_FFT1, [&] { return pruned_type1_cols(p, -sign2); });
             if (!r && sense && !sense_rows_fit(p)) {
                 // too many coils for one block: coil images into the plan's buffer, then combine
-                if (!p->sbuf && hipMalloc((void **)&p->sbuf, (size_t)(g.N * p->nc) * sizeof(float2)) != hipSuccess) {
-                    p->sbuf = nullptr;
-                    return fail(GN_ENOMEM, "hipMalloc failed for the SENSE coil images");
-                }
+                if ((r = make_sense_images(p))) return r;
                 r = timed(p, GN_STAGE_CROP, [&] {
                     int q = pruned_type1_rows(p, p->sbuf, scale, -sign2);
                     return q ? q : launch_sense_combine(p, p->sbuf, (float2 *)img);

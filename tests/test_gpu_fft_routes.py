@@ -35,3 +35,31 @@ def test_engines_agree(modes, nc):
         assert rel(a, b) <= 2e-6
     B = BatchPlan([dict(modes=modes, coords=coords, ncoils=nc)])
     assert rel(B.type2([F])[0], auto[0]) <= 2e-6 and rel(B.type1([y])[0], auto[1]) <= 2e-6
+
+
+def test_sense_combine_is_captured():
+    """The first SENSE adjoint of a plan whose coils do not fit one row-pass block (two line
+    buffers of 502 points x 24 coils) inside a graph: nothing is allocated, and every replay
+    equals the eager result."""
+    import torch
+    from mripy_amd.plan import Plan
+    print("case: captured combine", flush=True)
+    modes, nc, M = (251, 251), 24, 300
+    g = torch.Generator().manual_seed(1)
+    coords = [((2 * torch.rand(M, generator=g) - 1) * np.pi).cuda() for _ in modes]
+    F, y = [torch.randn(*s, generator=g, dtype=torch.complex64).cuda() for s in (modes + (nc,), (M, nc))]
+    P = Plan(modes, ncoils=nc, rat=2, nspread=3).set_points(coords)
+    P.set_sense(F)
+    P.type1(y)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x = P.sense_type1(y)
+    want = P.sense_type1(y).clone()
+    for k in range(3):
+        x.zero_()
+        y.mul_(2)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = want * 2
+        assert torch.equal(x, want)
