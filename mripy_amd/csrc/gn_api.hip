@@ -100,7 +100,7 @@ static int setup_tiles(gn_plan_s *p)
         g.Kg *= g.ngtiles[a];
     }
     // LDS limits: the spread keeps per-coil planes of up to kCoilGroup coils of a tile,
-    // the gather stages tile + halo of a coil pair (the trajectory gradient one coil)
+    // the gather stages tile + halo of a coil pair (the trajectory gradient a pair or one coil)
     const int64_t tc = (int64_t)g.tile[0] * g.tile[1] * g.tile[2];
     const int64_t ncg = std::min<int64_t>(p->nc, kCoilGroup);
     int64_t rc = 1;

@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <type_traits>
 #include <vector>
 
 #include <map>
@@ -1836,8 +1837,20 @@ __global__ __launch_bounds__(kReduceThreads) void k_spread_reduce_batch(const Sp
 
 static_assert(kGatherCoils == 2, "the gather stages coil pairs");
 
-template <int D>
-__device__ inline void stage_region_pair(float4 *lds, const float2 *__restrict__ g0, const float2 *__restrict__ g1,
+// A staged cell: coils g0 and g1 (zeros for a missing second coil), or g0 alone.
+template <typename Cell>
+__device__ inline Cell load_cell(const float2 *__restrict__ g0, const float2 *__restrict__ g1, bool two, int64_t i)
+{
+    if constexpr (sizeof(Cell) == sizeof(float4)) {
+        const float2 x0 = g0[i], x1 = two ? g1[i] : make_float2(0.f, 0.f);
+        return make_float4(x0.x, x0.y, x1.x, x1.y);
+    } else {
+        return g0[i];
+    }
+}
+
+template <int D, typename Cell>
+__device__ inline void stage_region_flat(Cell *lds, const float2 *__restrict__ g0, const float2 *__restrict__ g1,
                                          bool two, const int64_t *nf, const int *org, int R1, int R2, int RC)
 {
     // A thread takes cells rr = tid, tid + NT, ... of the region, rr = (r0 * R1 + r1) * R2 + r2
@@ -1852,7 +1865,7 @@ __device__ inline void stage_region_pair(float4 *lds, const float2 *__restrict__
     int r2 = tid - r0 * R12 - r1 * R2;
     const int nf0 = (int)nf[0], nf1 = (int)nf[1], nf2 = D == 3 ? (int)nf[2] : 1;
     for (int base = tid; base < RC; base += kStageUnroll * NT) {
-        float4 v[kStageUnroll];
+        Cell v[kStageUnroll];
 #pragma unroll
         for (int u = 0; u < kStageUnroll; ++u) {
             const int rr = base + u * NT;
@@ -1867,8 +1880,7 @@ __device__ inline void stage_region_pair(float4 *lds, const float2 *__restrict__
                     if (q2 >= nf2) q2 -= nf2;
                     gi = gi * nf2 + q2;
                 }
-                const float2 x0 = g0[gi], x1 = two ? g1[gi] : make_float2(0.f, 0.f);
-                v[u] = make_float4(x0.x, x0.y, x1.x, x1.y);
+                v[u] = load_cell<Cell>(g0, g1, two, gi);
             }
             r2 += d2;
             int c = r2 >= R2 ? 1 : 0;
@@ -1898,10 +1910,9 @@ __device__ inline bool rows_stage_ok(int RL, int64_t G)
 // 64 / RL whole rows per step (lane = row slot * RL + cell), so a lane keeps one
 // last-axis cell for the whole loop (its wrapped grid index is computed once) and
 // only the leading-axis coordinates of its row advance, with one carry; grid indices
-// are 32-bit.  A wave's lanes write consecutive LDS cells of 16 bytes, coils g0 and g1
-// (zeros for a missing second coil).
-template <int D>
-__device__ inline void stage_region_rows(float4 *lds, const float2 *__restrict__ g0, const float2 *__restrict__ g1,
+// are 32-bit.  A wave's lanes write consecutive LDS cells.
+template <int D, typename Cell>
+__device__ inline void stage_region_rows(Cell *lds, const float2 *__restrict__ g0, const float2 *__restrict__ g1,
                                          bool two, const int64_t *nf, const int *org, int R0, int R1, int R2)
 {
     constexpr int U = 4; // rows per lane whose loads are in flight together
@@ -1927,7 +1938,7 @@ __device__ inline void stage_region_rows(float4 *lds, const float2 *__restrict__
     }
     const uint32_t nf2 = D == 3 ? (uint32_t)nf[2] : 1u;
     for (; rho < nrow; rho += U * step) {
-        float4 v[U];
+        Cell v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (rho + u * step < nrow) {
@@ -1941,8 +1952,7 @@ __device__ inline void stage_region_rows(float4 *lds, const float2 *__restrict__
                 } else {
                     off = (uint32_t)q0 * (uint32_t)nf1 + (uint32_t)ql;
                 }
-                const float2 x0 = g0[off], x1 = two ? g1[off] : make_float2(0.f, 0.f);
-                v[u] = make_float4(x0.x, x0.y, x1.x, x1.y);
+                v[u] = load_cell<Cell>(g0, g1, two, off);
             }
             if (D == 3) {
                 r1 += s1;
@@ -2015,7 +2025,7 @@ __device__ __forceinline__ void gather_body(const GatherArgs &a, const int4 item
     if (rows_stage_ok(D == 3 ? R2 : R1, a.G))
         stage_region_rows<D>(lds_pair, g0, g0 + a.G, two, a.nf, org, R0, R1, R2);
     else
-        stage_region_pair<D>(lds_pair, g0, g0 + a.G, two, a.nf, org, R1, R2, RC);
+        stage_region_flat<D>(lds_pair, g0, g0 + a.G, two, a.nf, org, R1, R2, RC);
     __syncthreads();
     // Threads per sample: a work item's samples are spread over all waves of the
     // workgroup.  The tps lanes of a sample take the leading-axis taps t0 = sub,
@@ -2146,20 +2156,25 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_batch(const GatherArg
 //   out[a][j] = sum_c Re( conj(wts[j,c]) * d/dx_a (A image)[j,c] ),
 // with d/dx_a w = w * gscale_a * (t + ns - tap), gscale_a = -h_a df / (2 tau),
 // the analytic derivative of the Gaussian exp(-(xi - h g)^2 / (4 tau)).
-// The coils of a staged cell are contracted with the sample's weights first, so the taps
-// sum one real value per cell: 6 FMAs and one 16-byte LDS read per cell and coil pair, where
-// a derivative per coil took 16 to 24 and two 8-byte reads.  Staging, lanes per sample and
-// tile order as in the gather.  Bound by the taps' LDS reads and FMAs: 256^3-grid UTE, 4
-// coils, 1048576 samples, nspread 3: 436 -> 275 us.
+// The coils of a staged cell (a pair, or one: see traj_grad_dispatch) are contracted with the
+// sample's weights first, so the taps sum one real value per cell: 6 FMAs and one 16-byte
+// LDS read per cell and coil pair, where a derivative per coil took 16 to 24 and two 8-byte
+// reads.  Staging and lanes per sample as in the gather.  Bound by the taps' LDS reads and
+// FMAs: 256^3-grid UTE, 4 coils, 1048576 samples, nspread 3: 436 -> 275 us.
 // ---------------------------------------------------------------------------
 
-template <int D, int NS, bool WRAP>
+template <int D, int NS, bool WRAP, bool PAIR>
 __global__ __launch_bounds__(kGatherThreads) void k_traj_grad(GatherArgs a, const float2 *__restrict__ wts,
                                                                float *__restrict__ out, float gs0, float gs1, float gs2)
 {
-    constexpr int W = 2 * NS;
+    using Cell = std::conditional_t<PAIR, float4, float2>;
+    constexpr int W = 2 * NS, NC = PAIR ? 2 : 1; // coils of a staged cell
     extern __shared__ float4 lds_pair[];
-    const int4 item = a.items[xcd_swizzle(blockIdx.x, gridDim.x)];
+    Cell *cells = reinterpret_cast<Cell *>(lds_pair);
+    // neighbouring tiles on one XCD, as in the gather; not for the long items of wide windows,
+    // whose crowded tiles would share it (64^3 radial, nspread 6, 2 coils: 300 us, in runs 327)
+    constexpr bool kRuns = PAIR || NS <= 5;
+    const int4 item = a.items[kRuns ? xcd_swizzle(blockIdx.x, gridDim.x) : blockIdx.x];
     int org[3] = {0, 0, 0};
     {
         uint32_t r = (uint32_t)item.x; // tile index < 2^31
@@ -2215,8 +2230,8 @@ __global__ __launch_bounds__(kGatherThreads) void k_traj_grad(GatherArgs a, cons
                 v2[t] = w2[t] * u2;
             }
         }
-        for (int64_t c0 = 0; c0 < a.nc; c0 += 2) {
-            const bool two = c0 + 1 < a.nc;
+        for (int64_t c0 = 0; c0 < a.nc; c0 += NC) {
+            const bool two = PAIR && c0 + 1 < a.nc;
             const float2 *g = a.grid + c0 * a.G;
             float2 wa = make_float2(0.f, 0.f), wb = wa; // the pair's weights of this sample
             if (valid) {
@@ -2225,15 +2240,18 @@ __global__ __launch_bounds__(kGatherThreads) void k_traj_grad(GatherArgs a, cons
             }
             if (c0 > 0 || s0 > 0) __syncthreads(); // the previous pair's taps have been read
             if (rows_stage_ok(D == 3 ? R2 : R1, a.G))
-                stage_region_rows<D>(lds_pair, g, g + a.G, two, a.nf, org, R0, R1, R2);
+                stage_region_rows<D>(cells, g, g + a.G, two, a.nf, org, R0, R1, R2);
             else
-                stage_region_pair<D>(lds_pair, g, g + a.G, two, a.nf, org, R1, R2, RC);
+                stage_region_flat<D>(cells, g, g + a.G, two, a.nf, org, R1, R2, RC);
             __syncthreads();
             if (!valid) continue;
-            // sum over the pair of Re(conj(weight) cell)
+            // sum over the cell's coils of Re(conj(weight) value)
             auto cell = [&](int i) {
-                const float4 v = lds_pair[i];
-                return wa.x * v.x + wa.y * v.y + wb.x * v.z + wb.y * v.w;
+                const Cell v = cells[i];
+                if constexpr (PAIR)
+                    return wa.x * v.x + wa.y * v.y + wb.x * v.z + wb.y * v.w;
+                else
+                    return wa.x * v.x + wa.y * v.y;
             };
 #pragma unroll 1
             for (int t0 = sub; t0 < W; t0 += tps) {
@@ -3181,18 +3199,25 @@ template <int D, int NS>
 hipError_t traj_grad_dispatch(const GatherArgs &a, int nitems, const float2 *wts, float *out, const float *gs,
                               hipStream_t st)
 {
-    const size_t lds = (size_t)a.region[0] * a.region[1] * (D == 3 ? a.region[2] : 1) * sizeof(float4);
+    const size_t rc = (size_t)a.region[0] * a.region[1] * (D == 3 ? a.region[2] : 1);
     bool wrap = false;
     for (int ax = 0; ax < D; ++ax) wrap |= a.region[ax] >= a.nf[ax];
-    if (wrap) {
-        lds_limit(k_traj_grad<D, NS, true>, lds);
-        hipLaunchKernelGGL((k_traj_grad<D, NS, true>), dim3((unsigned)nitems), dim3(kGatherThreads), lds, st, a, wts,
-                           out, gs[0], gs[1], gs[2]);
-    } else {
-        lds_limit(k_traj_grad<D, NS, false>, lds);
-        hipLaunchKernelGGL((k_traj_grad<D, NS, false>), dim3((unsigned)nitems), dim3(kGatherThreads), lds, st, a,
-                           wts, out, gs[0], gs[1], gs[2]);
-    }
+    // Coil pairs (16-byte cells) while two workgroups of them fit a CU, else one coil at a time.
+    // 96^3, 600,000 samples, us, in brackets the kernel before the contraction: nspread 3,
+    // 2 coils, pairs 197 (234); pairs / single coils: nspread 5, 4 coils 998 / 901 (970), 3
+    // coils 961 / 697 (745), 1 coil 509 / 287 (300); nspread 8, 2 coils 2717 / 2167 (2340).  A
+    // pair costs a missing second coil in full, which three coils with wide windows in 2-D do
+    // not win back (256^2, nspread 14: 160 / 123 (125)).
+    const bool pair = a.nc > 1 && rc * sizeof(float4) <= 80 * 1024 && !(a.nc == 3 && NS >= 8);
+    const size_t lds = rc * (pair ? sizeof(float4) : sizeof(float2));
+    auto go = [&](auto kernel) {
+        lds_limit(kernel, lds);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nitems), dim3(kGatherThreads), lds, st, a, wts, out, gs[0], gs[1], gs[2]);
+    };
+    if (pair)
+        wrap ? go(k_traj_grad<D, NS, true, true>) : go(k_traj_grad<D, NS, false, true>);
+    else
+        wrap ? go(k_traj_grad<D, NS, true, false>) : go(k_traj_grad<D, NS, false, false>);
     return hipGetLastError();
 }
 
