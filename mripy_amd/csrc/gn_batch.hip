@@ -692,6 +692,9 @@ int gn_batch_create(int dim, int n, const gn_instance *inst, int rat, int nsprea
                            hipMalloc((void **)&t.rowc, n * sizeof(RowArgs)) != hipSuccess)))
             rc = fail(GN_ENOMEM, "batch argument tables");
     }
+    int64_t samples = 0;
+    for (auto *p : b->m) samples += p->M;
+    for (auto *p : b->m) p->launch_share = p->M > 0 ? (double)samples / (double)p->M : 1.0;
     if (!rc) rc = rebin(b);
     if (!rc && ((e = hipStreamCreateWithFlags(&b->gstream, hipStreamNonBlocking)) != hipSuccess || (e = hipEventCreate(&b->ev_in)) != hipSuccess ||
                 (e = hipEventCreate(&b->ev_out)) != hipSuccess))

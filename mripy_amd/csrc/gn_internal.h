@@ -267,6 +267,7 @@ struct gn_plan_s {
     float *deap = nullptr;    // concatenated per-axis exp(tau k^2) tables
     int *err_flag = nullptr;  // device: number of the last set_points that met bad coordinates
     int points_seq = 0;       // number of set_points calls
+    double launch_share = 1;  // samples of a spread launch per sample of this plan (above 1 in a batch)
 
     // FFT engine: the pruned in-place passes (gn_fft.hip) where pruned_passes_ok
     // (fft_custom), else rocFFT; GN_FFT_ROCFFT forces rocFFT

@@ -2496,6 +2496,7 @@ struct ScratchPool {
         return GN_OK;
     }
 };
+enum { kSpreadValu = 0, kSpreadMfma = 1, kSpreadTile = 2, kSpreadSub = 3 }; // SpreadShape::kind
 enum { kRetPairs = 0, kRetErr = 2, kRetSpread = 4, kRetGather = 8 };
 
 ScratchPool &scratch_pool()
@@ -2716,11 +2717,24 @@ __global__ __launch_bounds__(kGatherThreads) void k_bank_order(GatherArgs a, int
 // partial tiles cost more than that saves once the items fill the chip many times over.
 // Items of 512 / 192 / 128 pairs: 43 k pairs (192^2, 8 coils) 36 / 24 / 22 us, 209 k pairs
 // (256^2 spiral, 8 coils) 50 / 36 / 38 us, 1.1 M pairs (64^3, 4 coils) 107 / 83 / 82 us,
-// 2.9 M pairs (64^3, 8 coils) 202 / 225 / 268 us.
-int spread_chunk(int64_t pairs)
+// 2.9 M pairs (64^3, 8 coils) 202 / 225 / 268 us.  The pairs count once per coil group, and
+// in a batch with those of the other instances: 4 instances of 48^3 x 8 coils, 0.8 M pairs
+// each, type 1 451 / 482 us (512 / 192), 2 of 64^3 with 1 M 391 / 409.
+// Samples spread evenly have the same pairs in every tile: an item a little shorter than
+// that would split all of them, so with enough tiles it is 1.5 times the mean (type 1,
+// 48^3, 246 k samples, 293 pairs a tile, 8 coils 159 / 239 us (512 / 192), 32 coils 549 /
+// 876; 512^2 x 32, 213 pairs a tile, 724 / 1004).  The one-wave kernel in 2-D has items
+// enough from 4096 tiles on (128^2, 1 coil, 426 pairs in each of 512 tiles: 37 / 30 us).
+int spread_chunk(const gn_plan_s *p, int64_t pairs)
 {
     static_assert(kSpreadChunk >= 192, "shorter items than the longest");
-    return pairs >= (1 << 21) ? kSpreadChunk : pairs >= (1 << 17) ? 192 : 128;
+    const SpreadShape sh = spread_shape(make_spread_args(p, nullptr, 0), p->geo.dim);
+    const double sets = (double)((p->nc + sh.coils - 1) / sh.coils) * p->launch_share;
+    const double work = (double)pairs * sets;
+    const int chunk = work >= (7 << 18) ? kSpreadChunk : work >= (1 << 17) ? 192 : 128;
+    if ((double)p->geo.K * sets < (sh.kind == kSpreadTile && p->geo.dim == 2 ? 4096 : 512)) return chunk;
+    const int64_t even = (3 * pairs / (2 * p->geo.K) + 63) / 64 * 64;
+    return (int)std::min<int64_t>(kSpreadChunk, std::max<int64_t>(chunk, even));
 }
 
 int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const void *z, int coord_f64, double df,
@@ -2828,7 +2842,7 @@ int bin_and_sort(gn_plan_s *p, int64_t M, const void *x, const void *y, const vo
     // work items on the device; their counts come back in one synchronisation
     {
         const int64_t P = R.npairs;
-        const int chunk = spread_chunk(P);
+        const int chunk = spread_chunk(p, P);
         const int64_t cap_items = K + P / chunk + 1, cap_red = std::min<int64_t>(K, P / chunk + 1);
         const int64_t ncolt = (int64_t)g.ntiles[1] * g.ntiles[2];
         if ((rc = grow_alloc(&R.spread_items, &R.spread_items_cap, (size_t)cap_items, "work items")) ||
@@ -2924,8 +2938,6 @@ inline size_t spread_lds_bytes(const SpreadArgs &a, int ncg)
 // the dispatch-order arithmetic of the spread and gather kernels is 32-bit
 inline bool grid_ok(dim3 g) { return (uint64_t)g.x * g.y * g.z < (1ull << 31); }
 
-enum { kSpreadValu = 0, kSpreadMfma = 1, kSpreadTile = 2, kSpreadSub = 3 };
-
 } // namespace
 
 // Kernel and launch shape of a spread.  Default tiles: k_spread_tile for up to 2 coils in
@@ -3013,7 +3025,10 @@ hipError_t spread_dispatch(const SpreadArgs &a, int nitems, int nritems, const i
         }
     }
     if (e == hipSuccess && nritems > 0) {
-        const int64_t nb = std::min<int64_t>(kReduceBlocks, (a.TC * nc + kReduceThreads - 1) / kReduceThreads);
+        // several blocks per tile while the tiles are few (48^3, every tile split, 32 coils, type
+        // 1: 1103 us with 16 blocks each, 1055 with 4)
+        const int64_t want = std::max<int64_t>(4, std::min<int64_t>(kReduceBlocks, 8192 / nritems));
+        const int64_t nb = std::min<int64_t>(want, (a.TC * nc + kReduceThreads - 1) / kReduceThreads);
         hipLaunchKernelGGL(k_spread_reduce<D>, dim3((unsigned)nritems, (unsigned)nb), dim3(kReduceThreads), 0, st, a,
                            ritems);
         e = hipGetLastError();
