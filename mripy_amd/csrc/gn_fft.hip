@@ -369,7 +369,8 @@ __device__ __forceinline__ void fft_rows_pad_body(const RowArgs &a, int64_t line
     }
 }
 
-template <bool GEN>
+// SENSE: the block holds every coil of a line and writes their combination.
+template <bool GEN, bool SENSE>
 __device__ __forceinline__ void fft_rows_crop_body(const RowArgs &a, int64_t line, int64_t chunk)
 {
     extern __shared__ float2 lds_fft[];
@@ -418,7 +419,7 @@ __device__ __forceinline__ void fft_rows_crop_body(const RowArgs &a, int64_t lin
     const float d01 = a.scale * a.deap_a[n0] * (a.deap_b ? a.deap_b[n1] : 1.0f);
     const int half = a.m / 2;
     const bool cl = a.layout == GN_COIL_LAST;
-    if (a.sens) { // SENSE: the block holds every coil (ncl == nc): sum_c conj(S_c) * image_c
+    if constexpr (SENSE) { // sum_c conj(S_c) * image_c
         // The products replace the cropped line values (each is its own thread's), with the
         // maps read in their memory order, kLoadUnroll loads in flight; a thread per image
         // point that walked the coils instead read coil-last maps 8 bytes per cache line.
@@ -533,10 +534,17 @@ __global__ __launch_bounds__(kFFTThreads) void k_fft_rows_pad(RowArgs a)
 {
     fft_rows_pad_body<GEN>(a, blockIdx.x, blockIdx.y);
 }
+// The SENSE combine has a kernel of its own: the bounds of its 16 waves cost the plain crop
+// registers (32^3 x 32 coils 11.2 -> 13.9 us, 128^3 x 8 86 -> 90).
 template <bool GEN>
-__global__ __launch_bounds__(kFFTSenseThreads) void k_fft_rows_crop(RowArgs a)
+__global__ __launch_bounds__(kFFTThreads) void k_fft_rows_crop(RowArgs a)
 {
-    fft_rows_crop_body<GEN>(a, blockIdx.x, blockIdx.y);
+    fft_rows_crop_body<GEN, false>(a, blockIdx.x, blockIdx.y);
+}
+template <bool GEN>
+__global__ __launch_bounds__(kFFTSenseThreads) void k_fft_rows_combine(RowArgs a)
+{
+    fft_rows_crop_body<GEN, true>(a, blockIdx.x, 0);
 }
 
 // Batched row passes: items[b] = {instance, image line, coil chunk, 0}.
@@ -554,7 +562,7 @@ __global__ __launch_bounds__(kFFTThreads) void k_fft_rows_crop_batch(const RowAr
 {
     const int4 it = items[blockIdx.x];
     const RowArgs &a = args[it.x]; // read in place: uniform scalar loads
-    fft_rows_crop_body<GEN>(a, it.y, it.z);
+    fft_rows_crop_body<GEN, false>(a, it.y, it.z);
 }
 
 #ifndef GN_FFT_COL_LDS_MAX
@@ -645,7 +653,7 @@ void launch_rows(void (*kernel)(RowArgs), dim3 grid, const RowArgs &a, hipStream
     // take 16 waves, or the CU waits out each load and stage with too few (256 lines of 512
     // points x 32 coils, one 137 KiB block per CU: 33.2 us with 4 waves, 24.1 with 16; 22.5
     // with the maps read in memory order as well).
-    const int threads = lds > 40 * 1024 && a.img_out ? kFFTSenseThreads : kFFTThreads;
+    const int threads = lds > 40 * 1024 && a.img_out && a.sens ? kFFTSenseThreads : kFFTThreads;
     hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, a);
 }
 
@@ -849,7 +857,7 @@ int pruned_type1_rows_sense(gn_plan_s *p, float2 *image, float scale, float sign
     ra.CL = (int)p->nc;
     ra.img_out = image;
     ra.sens = p->sens;
-    launch_rows(ra.st.gen ? k_fft_rows_crop<true> : k_fft_rows_crop<false>, dim3((unsigned)ra.nlines, 1), ra, p->stream);
+    launch_rows(ra.st.gen ? k_fft_rows_combine<true> : k_fft_rows_combine<false>, dim3((unsigned)ra.nlines, 1), ra, p->stream);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GN_OK : hip_fail(e, "FFT pass A' (SENSE)");
 }
