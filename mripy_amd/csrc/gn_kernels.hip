@@ -1969,8 +1969,13 @@ __device__ inline void stage_region_rows(Cell *lds, const float2 *__restrict__ g
     }
 }
 
-// acc += w * v on both coils of a staged cell
-__device__ inline void fma4(float4 &acc, float w, const float4 v)
+// acc += w * v on the coils of a staged cell
+__device__ inline void fma_cell(float2 &acc, float w, const float2 v)
+{
+    acc.x += w * v.x;
+    acc.y += w * v.y;
+}
+__device__ inline void fma_cell(float4 &acc, float w, const float4 v)
 {
     acc.x += w * v.x;
     acc.y += w * v.y;
@@ -2089,14 +2094,14 @@ __device__ __forceinline__ void gather_body(const GatherArgs &a, const int4 item
                         for (int t2 = 0; t2 < W; ++t2) {
                             int r2 = l2 + t2;
                             if (WRAP && r2 >= R2) r2 -= (int)a.nf[2];
-                            fma4(q, w2[t2], lds_pair[rowb + r2]);
+                            fma_cell(q, w2[t2], lds_pair[rowb + r2]);
                         }
-                        fma4(p, w1[t1], q);
+                        fma_cell(p, w1[t1], q);
                     } else {
-                        fma4(p, w1[t1], lds_pair[r0 * R1 + r1]);
+                        fma_cell(p, w1[t1], lds_pair[r0 * R1 + r1]);
                     }
                 }
-                fma4(acc, w0, p);
+                fma_cell(acc, w0, p);
             }
         }
         // every lane takes part in the exchange (a sample's lanes are in one wave)
@@ -2156,15 +2161,22 @@ __global__ __launch_bounds__(kGatherThreads) void k_gather_batch(const GatherArg
 //   out[a][j] = sum_c Re( conj(wts[j,c]) * d/dx_a (A image)[j,c] ),
 // with d/dx_a w = w * gscale_a * (t + ns - tap), gscale_a = -h_a df / (2 tau),
 // the analytic derivative of the Gaussian exp(-(xi - h g)^2 / (4 tau)).
-// The coils of a staged cell (a pair, or one: see traj_grad_dispatch) are contracted with the
-// sample's weights first, so the taps sum one real value per cell: 6 FMAs and one 16-byte
-// LDS read per cell and coil pair, where a derivative per coil took 16 to 24 and two 8-byte
-// reads.  Staging and lanes per sample as in the gather.  Bound by the taps' LDS reads and
-// FMAs: 256^3-grid UTE, 4 coils, 1048576 samples, nspread 3: 436 -> 275 us.
+// A staged cell holds a coil pair, or one coil (see traj_grad_dispatch); the window weights
+// times their offsets are formed once per sample, so a cell takes 8 FMAs and one 16-byte LDS
+// read per pair, where the products formed per cell took 16 to 24 and two 8-byte reads.  The
+// sums run per coil and part and meet the sample's weights last: contracting the coils of a
+// cell first takes 6 FMAs (256^3-grid UTE, 4 coils, 1048576 samples, nspread 3: 275 us; this
+// way 308, per coil 436) but rounds before the derivative's cancellation, which made the
+// error of that gradient 4 to 6 % larger.  Staging and lanes per sample as in the gather.
+// Bound by the taps' LDS reads and FMAs.
 // ---------------------------------------------------------------------------
 
+// Two workgroups per CU are four waves per SIMD: at most 128 registers where their LDS allows
+// two (nspread 4 took 131 without the bound: 96^3 x 4 coils 562 -> 780 us).
+constexpr int traj_grad_waves(int D, int NS, bool WRAP, bool PAIR) { return !WRAP && (!PAIR || NS <= 5 || D == 2) ? 4 : 1; }
+
 template <int D, int NS, bool WRAP, bool PAIR>
-__global__ __launch_bounds__(kGatherThreads) void k_traj_grad(GatherArgs a, const float2 *__restrict__ wts,
+__global__ __launch_bounds__(kGatherThreads, traj_grad_waves(D, NS, WRAP, PAIR)) void k_traj_grad(GatherArgs a, const float2 *__restrict__ wts,
                                                                float *__restrict__ out, float gs0, float gs1, float gs2)
 {
     using Cell = std::conditional_t<PAIR, float4, float2>;
@@ -2245,47 +2257,51 @@ __global__ __launch_bounds__(kGatherThreads) void k_traj_grad(GatherArgs a, cons
                 stage_region_flat<D>(cells, g, g + a.G, two, a.nf, org, R1, R2, RC);
             __syncthreads();
             if (!valid) continue;
-            // sum over the cell's coils of Re(conj(weight) value)
-            auto cell = [&](int i) {
-                const Cell v = cells[i];
-                if constexpr (PAIR)
-                    return wa.x * v.x + wa.y * v.y + wb.x * v.z + wb.y * v.w;
-                else
-                    return wa.x * v.x + wa.y * v.y;
-            };
+            // value and derivative sums of every coil and part; the weights come last
+            Cell dx{}, dy{}, dz{};
 #pragma unroll 1
             for (int t0 = sub; t0 < W; t0 += tps) {
                 const float u0 = rf.x + (float)(NS - t0);
                 const float w0 = __builtin_amdgcn_exp2f(-a.coef[0] * u0 * u0);
                 int r0 = l0 + t0;
                 if (WRAP && r0 >= R0) r0 -= (int)a.nf[0];
-                float p = 0.f, py = 0.f, pz = 0.f;
+                Cell p{}, py{}, pz{};
 #pragma unroll
                 for (int t1 = 0; t1 < W; ++t1) {
                     int r1 = l1 + t1;
                     if (WRAP && r1 >= R1) r1 -= (int)a.nf[1];
-                    float q = 0.f, qz = 0.f;
-                    if (D == 3) {
+                    Cell q{};
+                    if constexpr (D == 3) {
+                        Cell qz{};
                         const int rowb = (r0 * R1 + r1) * R2;
 #pragma unroll
                         for (int t2 = 0; t2 < W; ++t2) {
                             int r2 = l2 + t2;
                             if (WRAP && r2 >= R2) r2 -= (int)a.nf[2];
-                            const float v = cell(rowb + r2);
-                            q += w2[t2] * v;
-                            qz += v2[t2] * v;
+                            const Cell v = cells[rowb + r2];
+                            fma_cell(q, w2[t2], v);
+                            fma_cell(qz, v2[t2], v);
                         }
-                        pz += w1[t1] * qz;
+                        fma_cell(pz, w1[t1], qz);
                     } else {
-                        q = cell(r0 * R1 + r1);
+                        q = cells[r0 * R1 + r1];
                     }
-                    p += w1[t1] * q;
-                    py += v1[t1] * q;
+                    fma_cell(p, w1[t1], q);
+                    fma_cell(py, v1[t1], q);
                 }
-                g0 += w0 * u0 * p;
-                g1 += w0 * py;
-                if (D == 3) g2 += w0 * pz;
+                fma_cell(dx, w0 * u0, p);
+                fma_cell(dy, w0, py);
+                if constexpr (D == 3) fma_cell(dz, w0, pz);
             }
+            // sum over the cell's coils of Re(conj(weight) sum)
+            auto contract = [&](const Cell &v) {
+                float r = wa.x * v.x + wa.y * v.y;
+                if constexpr (PAIR) r += wb.x * v.z + wb.y * v.w;
+                return r;
+            };
+            g0 += contract(dx);
+            g1 += contract(dy);
+            if constexpr (D == 3) g2 += contract(dz);
         }
         for (int k = 1; k < tps; ++k) {
             const int src = lane + k * stride;
@@ -3218,11 +3234,11 @@ hipError_t traj_grad_dispatch(const GatherArgs &a, int nitems, const float2 *wts
     bool wrap = false;
     for (int ax = 0; ax < D; ++ax) wrap |= a.region[ax] >= a.nf[ax];
     // Coil pairs (16-byte cells) while two workgroups of them fit a CU, else one coil at a time.
-    // 96^3, 600,000 samples, us, in brackets the kernel before the contraction: nspread 3,
-    // 2 coils, pairs 197 (234); pairs / single coils: nspread 5, 4 coils 998 / 901 (970), 3
-    // coils 961 / 697 (745), 1 coil 509 / 287 (300); nspread 8, 2 coils 2717 / 2167 (2340).  A
-    // pair costs a missing second coil in full, which three coils with wide windows in 2-D do
-    // not win back (256^2, nspread 14: 160 / 123 (125)).
+    // 96^3, 600,000 samples, the whole call, us, in brackets with the products formed per cell:
+    // nspread 3, 2 coils, pairs 201 (233); pairs / single coils: nspread 5, 4 coils 998 / 906
+    // (971), 3 coils 961 / 695 (747), 1 coil 509 / 287 (300); nspread 8, 2 coils 2717 / 2160
+    // (2338).  A pair costs a missing second coil in full, which three coils with wide windows
+    // in 2-D do not win back (256^2, nspread 14: 160 / 123 (125)).
     const bool pair = a.nc > 1 && rc * sizeof(float4) <= 80 * 1024 && !(a.nc == 3 && NS >= 8);
     const size_t lds = rc * (pair ? sizeof(float4) : sizeof(float2));
     auto go = [&](auto kernel) {
