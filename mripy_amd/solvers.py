@@ -348,12 +348,22 @@ def ADMM_l2Afxnb_tvx(Afunc, invAfunc, b, Nite, step, tv_r, rho, cgd_Nite=3, tvnd
 _F32_MAX = 3.4e38
 
 
+def _watched():
+    """Whether tracing, compilation, a dispatch or function mode, forward-mode derivatives or
+    vmap look at the operations.  These have no public query: a torch without one of the
+    names counts as watching."""
+    try:
+        return bool(torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or
+                    torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0 or
+                    torch._C._functorch.peek_interpreter_stack() is not None)
+    except AttributeError:
+        return True
+
+
 def _plain(like, *ts):
     """Whether the tensors are dense complex64 data like ``like`` on the current device that
     nothing but this code looks at: no gradients, tangents, vmap or dispatch modes."""
-    if (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or
-            torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0 or
-            torch._C._functorch.peek_interpreter_stack() is not None):
+    if _watched():
         return False
     grad = torch.is_grad_enabled()
     dev = like.device
