@@ -53,3 +53,19 @@ def test_tv_shapes(shape, ndim, niter):
         got = prox(torch.as_tensor(x.astype(np.complex64)).cuda(), 0.3, niter=niter, amp=amp)
         assert got.dtype == torch.complex64
         assert rel(got.cpu(), tv_numpy(x.astype(np.complex64).astype(complex), ndim, niter, amp=amp)) <= 1e-6
+
+
+@pytest.mark.parametrize("shape,ndim", [((12, 9), 2), ((40000, 2), 2), ((7, 6, 5), 3), ((60, 61, 2), 3)])
+@pytest.mark.parametrize("step", [1e74, 1e75, 1e76, 1e80, 1e140])
+def test_tv_projection_of_large_fields(shape, ndim, step):
+    """Dual fields before, at and beyond the range of the squared square, from images of order
+    1 and a large step: the projected field is of order 1 and so are its errors."""
+    import torch
+    from mripy_amd import solvers as S
+    print("case: tv projection", shape, ndim, step, flush=True)
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    want = tv_numpy(x, ndim, 1, step=step)
+    prox = S.prox_tv2d_r if ndim == 2 else S.prox_tv3d
+    got = prox(torch.as_tensor(x).cuda(), 0.3, step=step, niter=1).cpu().numpy()
+    assert np.isfinite(want).all() and rel(want, x) > 0.1 and rel(got, want) <= 1e-10
