@@ -450,29 +450,35 @@ template <int NDIM> int tv_launches(int niter)
 // Whether the steps run on LDS regions.  A region costs its block the same however few of
 // its cells the array fills (thin axes, small images with many trailing elements), and a
 // trailing dimension makes its accesses uncoalesced; two kernels per step cost launches and
-// passes over the field.  Microseconds for all steps, two kernels / regions:
-//   2-D, up to 1024 blocks: 3 x 3 x 1000, 40 steps 265 / 130; 16384 x 2, 40 steps 255 / 250
-//   2-D, more: 8 x 8 x 4096 (64 cells per block) 343 / 481, 65536 x 2 (36) 288 / 760,
-//     24 x 24 x 4096 (144) x 1.32, 14 x 14 x 4096 (196) x 0.67, 40 x 40 x 4096 (213) x 0.94;
-//     a single step: 40 x 40 x 4096 (400) x 1.13, 64 x 64 x 256 (455) x 0.86
-//   3-D, one trailing element: 256 x 256 x 2 (127) 382 / 569, 256 x 256 x 8, 3 steps (329)
-//     54 / 66, 128^3, 1 step (306) 65 / 79, 10 steps (480) 702 / 554; 32^3 (125 blocks) 285 / 233
-//   3-D, more trailing elements: 64^3 x 8 (501) 2956 / 3506
+// passes over the field.
+// 2-D: up to 1024 blocks, or 200 cells per block and step (430 for a single step).
+// Microseconds, two kernels / regions (cells): 3 x 3 x 1000, 40 steps 265 / 130; 16384 x 2
+// 255 / 250; 8 x 8 x 4096 (64) 343 / 481; 65536 x 2 (36) 288 / 760; 24 x 24 x 4096 (144) x 1.32;
+// 14 x 14 x 4096 (196) x 0.67; 40 x 40 x 4096 (213) x 0.94, a single step (400) x 1.13; 64 x 64
+// x 256, a single step (455) x 0.86.
+// 3-D, one step per launch: one trailing element and 435 cells or more, else the smaller
+// estimate, microseconds from 898 measured calls: a launch of regions 5 or 0.009 per block
+// (6.5 or 0.02 with a trailing dimension), one of the other kernels 3 or 9e-6 per element.
+// 256 x 256 x 2, 40 steps (127 cells) 382 / 569; 256 x 256 x 8, 3 steps (329) 54 / 66; 100^3
+// (449) 1600 / 1221; 61 x 29 x 24, 2 steps 20 / 13; 64^3 x 8 (501) 2956 / 3506.
 // Regions also need every launch's blocks to fit one launch (2^22 of 1024 threads: from about
 // 1.4e9 cells in 3-D); the two kernels' 256-thread blocks fit for every array that is taken.
 template <int NDIM> bool tv_regions(const TVGeom &g, int niter)
 {
     const int n = tv_launches<NDIM>(niter);
     int64_t block_steps = 0;
+    double regions = 0.0;
     for (int k = 0; k < n; ++k) {
         int64_t blocks = 0;
         const TVLaunch L = tv_launch<NDIM>(g, niter, k, n, &blocks);
         if (!host::launch_fits(blocks, kTVThreads)) return false;
         block_steps += blocks * L.iters;
+        regions += g.nt == 1 ? std::max(5.0, 0.009 * (double)blocks) : std::max(6.5, 0.02 * (double)blocks);
     }
-    const int64_t few = NDIM == 2 ? 1024 : 128;
-    const int64_t cells = NDIM == 2 ? (niter == 1 ? 430 : 200) : 440; // per block and step
-    return block_steps <= few * niter || ((NDIM == 2 || g.nt == 1) && (int64_t)g.n * niter >= cells * block_steps);
+    if (niter == 0) return true;
+    const auto filled = [&](int64_t cells) { return (int64_t)g.n * niter >= cells * block_steps; };
+    if (NDIM == 2) return block_steps <= (int64_t)1024 * niter || filled(niter == 1 ? 430 : 200);
+    return (g.nt == 1 && filled(435)) || regions <= (2.0 * niter + 1.0) * std::max(3.0, 9e-6 * (double)g.n);
 }
 
 template <typename T, int NDIM, int AMP>
