@@ -461,10 +461,15 @@ template <int NDIM> int tv_launches(int niter)
 // (6.5 or 0.02 with a trailing dimension), one of the other kernels 3 or 9e-6 per element.
 // 256 x 256 x 2, 40 steps (127 cells) 382 / 569; 256 x 256 x 8, 3 steps (329) 54 / 66; 100^3
 // (449) 1600 / 1221; 61 x 29 x 24, 2 steps 20 / 13; 64^3 x 8 (501) 2956 / 3506.
-// Regions also need every launch's blocks to fit one launch (2^22 of 1024 threads: from about
-// 1.4e9 cells in 3-D); the two kernels' 256-thread blocks fit for every array that is taken.
+// Regions keep the dual field twice, 16 ndim bytes per element against 16 for D: above
+// kTVTwiceMax elements (24 GiB of fields once, in 3-D) the memory is left to the caller.
+// They also need every launch's blocks to fit one launch (2^22 of 1024 threads); the two
+// kernels' 256-thread blocks fit for every array that is taken.
+constexpr int64_t kTVTwiceMax = (int64_t)1 << 29;
+
 template <int NDIM> bool tv_regions(const TVGeom &g, int niter)
 {
+    if (g.n > kTVTwiceMax) return false;
     const int n = tv_launches<NDIM>(niter);
     int64_t block_steps = 0;
     double regions = 0.0;
@@ -579,7 +584,8 @@ int64_t gn_tv_work_bytes(int ndim, const int64_t *shape, int64_t nt)
         if (shape[a] < 0) return 0;
         n *= shape[a];
     }
-    return (int64_t)2 * ndim * n * (int64_t)sizeof(double2); // the dual field before and after a launch
+    // the dual field before and after a launch of regions, or the field and D (see tv_regions)
+    return (n > kTVTwiceMax ? ndim + 1 : 2 * ndim) * n * (int64_t)sizeof(double2);
 }
 
 int gn_tv_prox(int dtype, int ndim, const int64_t *shape, int64_t nt, const void *y, double lambda, double step,
