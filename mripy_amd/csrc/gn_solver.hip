@@ -528,6 +528,10 @@ int tv_prox_any(int ndim, int amp, TVGeom g, const T *y, double lambda, double s
 // 270 us iteration (256^2, 32 coils); as one kernel the iteration takes 37 us less.
 // Products with real factors, and the signs of sums, keep the terms of a complex product with
 // imaginary part 0, so that infinities and NaN end up where complex arithmetic puts them.
+// The quotient is a product with the reciprocal, as in a complex division, so that every
+// rounding is the separate passes': with a / d 20 iterations of 12 inputs ended 1.4 % further
+// from their 64-bit values.  (In FP64, rounded once per output, they end 60 % further: a
+// phantom's regions of one value meet the roundings alike, and these offset the operator's.)
 // ---------------------------------------------------------------------------
 __device__ inline float2 scale_c(float2 v, float s)
 {
@@ -552,7 +556,8 @@ __global__ void k_soft_step(int64_t n, const float2 *__restrict__ g, const float
     a = add_c(a, scale_c(r, step), -1.f);
     acc[i] = a;
     const float m = hypotf(a.x, a.y), d = m + 1e-6f, c = m - th;
-    const float2 u = scale_c(make_float2((a.x + a.y * 0.f) / d, (a.y - a.x * 0.f) / d), c < 0.f ? 0.f : c);
+    const float q = 1.f / d;
+    const float2 u = scale_c(make_float2((a.x + a.y * 0.f) * q, (a.y - a.x * 0.f) * q), c < 0.f ? 0.f : c);
     x[i] = u;
     if (y) y[i] = add_c(u, scale_c(add_c(u, xp, -1.f), beta), 1.f);
 }
