@@ -206,9 +206,9 @@ int gn_plan_destroy(gn_plan *plan);
  * mask: null or float32 of prod(shape) entries (broadcast over the batch, mask_batch
  * = 1) or prod(shape) * batch entries (mask_batch = batch); it multiplies the output.
  * in and out may be the same buffer.  Host-synchronous on `stream`; with GN_FFT_ASYNC the
- * call returns once its kernels are queued on `stream`, except for lengths the library's
- * own passes do not cover (see gn_fft.hip: fft_length_supported), whose workspace is
- * shared by the calls on a device.  Calls from several threads are serialized. */
+ * call returns once its kernels are queued on `stream`, except where rocFFT is used (see
+ * gn_cfft.hip: axis_passes_ok), whose workspace is shared by the calls on a device.
+ * Calls from several threads are serialized. */
 #define GN_FFT_FORWARD 1
 #define GN_FFT_INVERSE -1
 #define GN_FFT_SHIFT_IN 1  /* fftshift the input over the transformed axes  */

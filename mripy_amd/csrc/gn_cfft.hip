@@ -227,9 +227,10 @@ int axis_lines(int L)
     return lines;
 }
 
-// The axis passes apply: every length is 1 or covered (and not faster with rocFFT), the output is the input or does not
-// overlap it, and the blocks of every axis fit one launch (2^23 blocks of about 2048
-// elements; larger arrays are left to rocFFT, whose shift passes loop).
+// The axis passes apply: every length is 1 or covered (and not faster with rocFFT), the
+// output is the input or does not overlap it, and the blocks of every axis fit one launch
+// (2^23 blocks of about 2048 elements; larger arrays are left to rocFFT, whose shift passes
+// loop).
 bool axis_passes_ok(int rank, const int64_t *n, int64_t total, const void *in, const void *out)
 {
     bool any = false;

@@ -161,8 +161,8 @@ inline bool pruned_passes_pay(int dim, const int64_t *nf, int64_t ncoils)
 }
 
 // Whether a strided axis of this length (several columns) is left to the Cartesian axis
-// passes: not where a block's LDS holds one column, so that a row segment is 8 bytes.  Microseconds, rocFFT with its shift passes /
-// axis passes, n x n x 2: 1834 (prime 131) 352 / 295, 1820 206 / 150, 1875 218 / 233,
+// passes: not where a block's LDS holds one column, so that a row segment is 8 bytes.
+// Microseconds, rocFFT with its shift passes / axis passes, n x n x 2: 1834 (prime 131) 352 / 295, 1820 206 / 150, 1875 218 / 233,
 // 2000 228 / 272, 2048 230 / 286, 1912 (prime 239) 361 / 522; rocFFT has radix 17:
 // 1088 105 / 79, 1156 121 / 132, 1360 135 / 159, 1530 162 / 210, 1700 184 / 235.
 inline bool axis_strided_ok(int L)

@@ -25,7 +25,8 @@ constexpr int kCoilGroup = 8;       // coils accumulated together per pass
 // 8.  Every group stages the pairs, fills the weight tables and issues the same matrix
 // products whatever its width (a product has columns for 8 coils), so a second group
 // for the remaining coils costs as much as the first: 91 x 109 x 75, 3 coils, nspread 5
-// took 0.80 ms as two groups of 2 and 0.43 ms as one (k_spread_mfma).
+// took 0.80 ms as two groups of 2 and 0.43 ms as one.  For k_spread_mfma and k_spread; the
+// default tiles take kernels with groups of their own for few coils and in 2-D (spread_shape).
 inline int spread_coil_group(int64_t nc) { return nc > 4 ? kCoilGroup : nc > 2 ? 4 : nc > 1 ? 2 : 1; }
 // coils per gather work-group: a coil pair, staged together as 16-byte cells so
 // that one LDS read serves both coils of a tap

@@ -1535,7 +1535,7 @@ __global__ __launch_bounds__(64) void k_spread_tile_batch(const SpreadArgs *__re
 // reach each sub-block; 4 listed pairs take one weight product wx wy per lane (row = cell)
 // and NG matrix products whose columns are the reals of 8 coils.  A window of 6 cells
 // fills 0.44 of a 4 x 4 block it reaches, against 0.22 of an 8 x 8 block, so the products
-// are half of k_spread_mfma's; the tables and records serve up to 32 coils.
+// are half of k_spread_mfma's; the tables and records serve up to 16 coils.
 // Bound by the batches' vector instructions and latency (matrix cores about 0.4 busy), so a
 // batch's records are held a pair per lane: a wave forms one quad of weights of every pair
 // without divisions, tests its own sub-blocks, and takes values' sample indices by lane
