@@ -2,7 +2,7 @@
 
 This module is the oracle that the HIP implementation in ``mripy_amd`` is checked
 against.  Only ``tests/``, ``__graft_entry__.smoke()`` and the ``cpu_baseline`` leg
-of ``bench.py`` may import it, and only as the checker: the product path never
+of ``bench.py`` may import it, and only to compare against: the product path never
 calls into it.
 
 Every function restates the reference algorithm in float64/complex128 and cites
