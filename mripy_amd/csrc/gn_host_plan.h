@@ -147,14 +147,25 @@ inline int largest_prime(int64_t L)
 //   a 3-D grid with few columns beside a long first axis, where rocFFT has more blocks:
 //     154 x 32 x 32 1.18, 112 x 32 x 32 x 4 coils 1.13, 220 x 32 x 32 x 8 0.79; 530 x 32 x 32 (53)
 //     0.74, 502 x 32 x 32 (251) 0.92 and 1.03 in type 1, 942 x 32 x 32 (157) 0.94 and 1.13
+//   3-D with a short first axis, whose column blocks hold few elements, primes up to 17 and
+//     many coils: 22 x 52 x 220 x 28 coils 1.23 (type 1 1.30), 22 x 96 x 80 x 23 1.09 (1.22), 12 x
+//     220 x 312 x 10 1.02 (1.13), 14 x 196 x 264 x 27 0.98 (1.08); 22 x 44 x 48 x 22 0.78, 24 x 128 x
+//     306 x 3 0.89, 26 x 110 x 32 x 24 0.85 (0.90)
+//   columns of 891 to 1024 points with two line buffers, large 2-D grids: 984 x 502 x 20 (41) 1.29, 950 x 796 x 20
+//     (19) 1.16, 920 x 660 x 24 (23) 1.10; 948 x 728 x 7 (79) 0.98, 1010 x 1010 x 8 (101) 0.94
 inline bool pruned_passes_pay(int dim, const int64_t *nf, int64_t ncoils)
 {
+    const int64_t cells = nf[0] * nf[1] * (dim == 3 ? nf[2] : 1) * ncoils;
+    int most = 1;
+    for (int a = 0; a < dim; ++a) most = std::max(most, largest_prime(nf[a]));
+    if (dim == 3 && nf[0] <= 22 && most > 5 && most <= 17 && ncoils >= 10 && cells >= 1500000) return false;
     for (int a = 0; a < dim; ++a) {
         const int64_t L = nf[a];
         const int p = largest_prime(L);
         if (p <= 5) continue;
         const bool rows = a == dim - 1; // contiguous lines
         if (p <= 17 ? L > 780 : !rows && (L > 1860 || (L > 890 && L <= 1024 && p > 128))) return false;
+        if (dim == 2 && !rows && L > 890 && L <= 1024 && p > 17 && cells > 9000000) return false;
         if (dim == 3 && a == 0 && nf[1] * nf[2] * ncoils <= 4096 && (p <= 17 || p > 180 || L > 890)) return false;
     }
     return true;

@@ -64,6 +64,9 @@ static void check_passes()
     for (int L : {784, 858, 952, 1300, 916, 1002, 1904, 1912, 2002, 2008}) CHECK(!pay2(L, L, 8));
     CHECK(pay2(256, 1910, 1) && !pay2(1910, 256, 1) && pay2(256, 770, 1) && !pay2(256, 910, 1));
     CHECK(pay3(182, 218, 150, 3) && pay3(220, 32, 32, 8) && !pay3(220, 32, 32, 4) && pay3(32, 32, 220, 1));
+    CHECK(!pay3(22, 52, 220, 28) && !pay3(14, 24, 306, 16) && !pay3(12, 220, 312, 10) && !pay3(18, 104, 250, 21));
+    CHECK(pay3(22, 44, 48, 22) && pay3(26, 110, 32, 24) && pay3(20, 44, 272, 9) && pay3(18, 126, 172, 21) && pay3(18, 100, 250, 21));
+    CHECK(!pay2(984, 502, 20) && !pay2(950, 796, 20) && !pay2(920, 660, 24) && pay2(948, 728, 7) && pay2(856, 728, 24) && pay2(1000, 484, 31));
     CHECK(pay3(530, 32, 32, 1) && !pay3(502, 32, 32, 1) && !pay3(942, 32, 32, 1) && pay3(940, 64, 128, 1));
 }
 
