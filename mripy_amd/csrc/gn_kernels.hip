@@ -2967,7 +2967,11 @@ SpreadShape spread_shape(const SpreadArgs &a, int dim)
     const bool tile = dim == 3 ? a.tile[0] == 4 && a.tile[1] == 4 && a.tile[2] == 8 : a.tile[0] == 8 && a.tile[1] == 16;
     if (tile && dim == 2 && a.nc > 2 && mfma_tiles_ok(a, dim)) {
         s.kind = kSpreadSub;
-        s.width = a.nc <= 8 ? 1 : 2; // 16 coils per workgroup; 32 took 132 registers: 96 -> 82 us at 32 coils
+        // 16 coils per workgroup (32 took 132 registers: 96 -> 82 us at 32 coils); 8 of coil-major
+        // samples, each value of which is a cache line of its own, so that a launch's lines stay
+        // cached (type 1, uniform samples, 8 x 8 blocks / 16 coils / 8: 320^2 x 32, 158 k, nspread
+        // 5 300 / 367 / 300 us; 192^2 x 31, 76 k radial, nspread 3 138 / 131 / 111)
+        s.width = a.nc <= 8 || a.layout != GN_COIL_LAST ? 1 : 2;
         s.waves = kSpreadSubWaves;
         s.coils = 8 * s.width;
         s.lds = spread_sub_lds(s.width);
