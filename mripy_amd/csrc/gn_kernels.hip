@@ -2977,7 +2977,9 @@ SpreadShape spread_shape(const SpreadArgs &a, int dim)
         s.lds = spread_sub_lds(s.width);
         return s;
     }
-    if (tile && a.nc <= 4 && mfma_tiles_ok(a, dim)) {
+    // coil-major samples of 4 coils: a value is a cache line of its own, waited for by one wave
+    // (type 1 of 32^3, 117 k uniform samples, nspread 3: k_spread_mfma 87 us, k_spread_tile 95)
+    if (tile && (a.nc < 4 || (a.nc == 4 && a.layout == GN_COIL_LAST)) && mfma_tiles_ok(a, dim)) {
         s.kind = kSpreadTile;
         s.width = a.nc == 1 ? 2 : a.nc == 2 ? 4 : 8;
         s.coils = s.width / 2;
