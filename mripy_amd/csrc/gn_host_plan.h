@@ -151,8 +151,9 @@ inline int largest_prime(int64_t L)
 //     many coils: 22 x 52 x 220 x 28 coils 1.23 (type 1 1.30), 22 x 96 x 80 x 23 1.09 (1.22), 12 x
 //     220 x 312 x 10 1.02 (1.13), 14 x 196 x 264 x 27 0.98 (1.08); 22 x 44 x 48 x 22 0.78, 24 x 128 x
 //     306 x 3 0.89, 26 x 110 x 32 x 24 0.85 (0.90)
-//   columns of 891 to 1024 points with two line buffers, large 2-D grids: 984 x 502 x 20 (41) 1.29, 950 x 796 x 20
-//     (19) 1.16, 920 x 660 x 24 (23) 1.10; 948 x 728 x 7 (79) 0.98, 1010 x 1010 x 8 (101) 0.94
+//   columns of 891 to 1024 points with two line buffers, large 2-D grids: 984 x 502 x 20 (41)
+//     1.29, 950 x 796 x 20 (19) 1.16, 920 x 660 x 24 (23) 1.10; 948 x 728 x 7 (79) 0.98, 1010 x
+//     1010 x 8 (101) 0.94
 inline bool pruned_passes_pay(int dim, const int64_t *nf, int64_t ncoils)
 {
     const int64_t cells = nf[0] * nf[1] * (dim == 3 ? nf[2] : 1) * ncoils;
@@ -173,8 +174,8 @@ inline bool pruned_passes_pay(int dim, const int64_t *nf, int64_t ncoils)
 
 // Whether a strided axis of this length (several columns) is left to the Cartesian axis
 // passes: not where a block's LDS holds one column, so that a row segment is 8 bytes.
-// Microseconds, rocFFT with its shift passes / axis passes, n x n x 2: 1834 (prime 131) 352 / 295, 1820 206 / 150, 1875 218 / 233,
-// 2000 228 / 272, 2048 230 / 286, 1912 (prime 239) 361 / 522; rocFFT has radix 17:
+// Microseconds, rocFFT with its shift passes / axis passes, n x n x 2: 1834 (prime 131) 352 /
+// 295, 1820 206 / 150, 1875 218 / 233, 2000 228 / 272, 2048 230 / 286, 1912 (prime 239) 361 / 522; rocFFT has radix 17:
 // 1088 105 / 79, 1156 121 / 132, 1360 135 / 159, 1530 162 / 210, 1700 184 / 235.
 inline bool axis_strided_ok(int L)
 {

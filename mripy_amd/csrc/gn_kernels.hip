@@ -2957,7 +2957,7 @@ inline bool grid_ok(dim3 g) { return (uint64_t)g.x * g.y * g.z < (1ull << 31); }
 } // namespace
 
 // Kernel and launch shape of a spread.  Default tiles: k_spread_tile for up to 2 coils in
-// 2-D and 4 in 3-D, k_spread_sub for more in 2-D.  3-D with 5 and more coils, and other
+// 2-D and 4 in 3-D (3 coil-major), k_spread_sub for more in 2-D.  3-D with more, and other
 // block-aligned tiles, take k_spread_mfma (128^3, 1,048,576 samples, nspread 3: 4 coils
 // 499 -> 459 us with k_spread_tile, but 8 coils 571 -> 763 us: its products fill the
 // matrix cores without skipping half tiles).  Any other tile takes k_spread.
